@@ -6,11 +6,13 @@
 // fp16) -- the reference's numerics -- and fed to v_mfma_f32_32x32x16_{bf16,f16}
 // with fp32 accumulation. The output is rounded once to the activation dtype.
 //
-// As in the W8A8 GEMM, the MFMA "A" operand is a 32-row weight slab and "B" a
+// The general kernel (scale blocks that are no multiple of 64 K, past the decode batches;
+// w8a16_tile.hip takes the others): as in the W8A8 GEMM, the MFMA "A" operand is a 32-row weight slab and "B" a
 // 32-row activation slab, so each lane owns one weight row n per slab and the
 // per-row scale lookup happens once per 8-element K chunk. Tiles are staged through
 // LDS with double buffering, 64 K elements per step.
 #include "ayk_common.h"
+#include "w8a16_tile.h"
 
 #include <utility>
 
@@ -1408,11 +1410,13 @@ extern "C" {
 
 size_t ayk_fp8_weight_only_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t block_size_x) {
   if (M < 2) return 0;
-  // An upper bound over the decode kernels (alignment decides which one runs).
+  // An upper bound over the kernels (alignment decides which one runs).
   const size_t st = stream_workspace(stream_plan(M, N, K, block_size_x), M, N);
   const size_t rs = rows_workspace(rows_plan(M, N, K, block_size_x), M, N);
   const size_t sk = skinny_workspace(skinny_plan(M, N, K, block_size_x), M, N);
-  return st > rs ? (st > sk ? st : sk) : (rs > sk ? rs : sk);
+  const size_t decode = st > rs ? (st > sk ? st : sk) : (rs > sk ? rs : sk);
+  const size_t tile = w16_tile_workspace(M, N, K);
+  return decode > tile ? decode : tile;
 }
 
 int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M, const void* w,
@@ -1485,6 +1489,10 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
                                  : launch_skinny<false>(p, a, workspace_bytes, st);
     }
   }
+  // Everything else: the tiled kernel, but for scale blocks that split its 64-K stages.
+  const W16TileArgs t{g.x, ldx, g.w, ldw, M, N, K, scale, scale_dtype, scale_row_stride, block_size_y, block_size_x,
+                      out, ldo, static_cast<float*>(workspace), workspace_bytes};
+  if (w16_tile_supported(t)) return w16_tile_launch(t, x_dtype == AYK_BF16, st, op);
   return x_dtype == AYK_BF16 ? dispatch_w16<true>(g, st) : dispatch_w16<false>(g, st);
 }
 
