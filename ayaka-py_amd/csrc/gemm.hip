@@ -1,6 +1,6 @@
 // FP8 GEMM on gfx950 matrix cores: out[M, N] = epilogue(a[M, K] . w[N, K]^T).
 //
-// One kernel template serves the three W8A8 recipes of the reference
+// The W8A8 recipes of the reference
 // (python/ayaka/kernel/triton/gemm/fp8_gemm.py, fp8_mxfp8_gemm.py):
 //   MODE_SCALED  fp8_scaled_mm     out = acc * sa[m] * sb[n] + bias[n]
 //   MODE_BLOCK   fp8_blockwise_mm  acc += (partial over 128 K) * sa[m, kb] * sb[n/128, kb]
@@ -17,17 +17,20 @@
 // and applies the scale byte of lane half b to K block [32b, 32b+32). Fragments are
 // read from LDS in that order, so scale block b is exactly MX group 2*step + b.
 //
-// Tiling. A 256-thread workgroup (4 wavefronts) owns a BN x BM output tile and
-// walks K in 128-byte steps (BK = 128: one block-scale step, four MX groups). Tiles
-// are staged global -> VGPR -> LDS with double buffering: the next step's 16-byte
-// global loads are issued before the current step's MFMAs. LDS rows are padded to
-// 144 bytes so the 32 rows a wavefront reads at one K offset fall on distinct banks.
+// The kernels here are the 256 x 256 ones (and the block-scaled 128 x 128 one);
+// gemm_mid.hip has the medium tiles, gemm_skinny.hip the decode batches, and launch_gemm
+// chooses. The general kernel below remains for row strides past 32-bit tile offsets: a
+// 256-thread workgroup owns a BN x BM tile and walks K in 128-byte steps, staged global ->
+// VGPR -> LDS with double buffering; LDS rows are padded to 144 bytes so the 32 rows a
+// wavefront reads at one K offset fall on distinct banks.
 #include "ayk_common.h"
 #include "gemm_block.h"
+#include "gemm_mid.h"
 #include "gemm_skinny.h"
 #include "gemm_tiles.h"
 #include "gemm_util.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace ayk {
@@ -71,9 +74,9 @@ struct GemmArgs {
   int out_dtype;
   int64_t ldo;
   int tiles_m;     // number of BM tiles along M
-  float* ws;       // split-K partials (block-scaled GEMM), ws_bytes long
+  float* ws;       // split-K partials, ws_bytes long
   size_t ws_bytes;
-  int64_t kps;     // general kernel, block mode: K per split (0: no split; blockIdx.y = split)
+  int64_t kps;     // 256 x 256 pair kernel: K per piece of a K split (0: no split)
   // 256 x 256 pair kernel, tail split (tail_split > 1): workgroups past dp_tiles take
   // K piece (b - dp_tiles) % tail_split of tile dp_tiles + (b - dp_tiles) / tail_split.
   int dp_tiles;
@@ -160,34 +163,8 @@ __device__ inline void store4(const GemmArgs& g, int64_t m, int64_t n, const flo
 
 // BN: weight rows per tile, BM: activation rows per tile, WN x WM wavefront grid.
 template <int MODE, int BN, int BM, int WN, int WM>
-__global__ __launch_bounds__(kThreads) void fp8_gemm_kernel(GemmArgs gin) {
+__global__ __launch_bounds__(kThreads) void fp8_gemm_kernel(GemmArgs g) {
   static_assert(WN * WM == kThreads / kWave, "4 wavefronts per workgroup");
-  // Block or rowwise mode with a K split: blockIdx.y takes K range [y kps, (y + 1) kps)
-  // (kps % 128 == 0) and writes its fp32 partials (rowwise: already scaled) to ws[y]
-  // ([M, N]); block_split_reduce sums them, adds the bias and rounds once.
-  GemmArgs g = gin;
-  if constexpr (MODE == MODE_BLOCK || MODE == MODE_SCALED || MODE == MODE_MX || MODE == MODE_INT8) {
-    if (gin.kps > 0) {
-      const int64_t k0 = (int64_t)blockIdx.y * gin.kps, kb0 = k0 / 128, kb_total = gin.K / 128;
-      g.K = gin.K - k0 < gin.kps ? gin.K - k0 : gin.kps;
-      g.a = gin.a + k0;
-      g.w = gin.w + k0;
-      if constexpr (MODE == MODE_BLOCK) {  // K-blocked scale tables follow the K range
-        g.sa = static_cast<const float*>(gin.sa) + (gin.sa_vec ? kb0 * gin.M : kb0);
-        g.ld_sa = gin.sa_vec ? 0 : kb_total;
-        g.sb = static_cast<const uint8_t*>(gin.sb) + kb0 * (gin.sb_dtype == AYK_F32 ? 4 : (gin.sb_dtype == AYK_U8 ? 1 : 2));
-        g.ld_sb = kb_total;
-      }
-      if constexpr (MODE == MODE_MX) {  // UE8M0 code rows: the range's codes start k0 / 32 in
-        g.sa = static_cast<const uint8_t*>(gin.sa) + k0 / 32;
-        g.sb = static_cast<const uint8_t*>(gin.sb) + k0 / 32;
-      }
-      g.bias = nullptr;
-      g.out = gin.ws + (int64_t)blockIdx.y * gin.M * gin.N;
-      g.out_dtype = AYK_F32;
-      g.ldo = gin.N;
-    }
-  }
   constexpr int TN = BN / WN, TM = BM / WM;  // wavefront tile
   constexpr int FN = TN / 32, FM = TM / 32;  // 32x32 MFMA tiles per wavefront
   static_assert(FN >= 1 && FM >= 1, "wavefront tile must be a multiple of 32x32");
@@ -1662,26 +1639,16 @@ int64_t block_split(int64_t M, int64_t N, int64_t K) {
   while (tiles * split < kBlkSplitTarget && K / (split * 2) >= 1024 && (K / 128) % (split * 2) == 0) split *= 2;
   return split;
 }
-// The same rule for the general kernel's 32- or 64-row tiles (M <= 64, K % 128 == 0).
-int64_t general_split(int64_t M, int64_t N, int64_t K) {
-  if (M > 64 || K % 128) return 1;
-  const int64_t tiles = cdiv(M, M <= 32 ? 32 : 64) * cdiv(N, 128);
-  int64_t split = 1;
-  while (tiles * split < kBlkSplitTarget && K / (split * 2) >= 1024 && (K / 128) % (split * 2) == 0) split *= 2;
-  return split;
-}
-// Rowwise / per-tensor K split for launches short of one round of bm x bn tiles (one
-// round: 256 workgroups of the 256 x 256 kernel, one per CU; 512 of the general
-// kernel's): as many splits as still fit in that one round, at least 1024 K each (the
-// last may be shorter). Spilling into a second round doubles the time of the splits
-// and multiplies the partial-sum traffic (Qwen2 down at M = 2048: 5 splits 231 us,
-// 2 splits fill the round).
-int64_t scaled_split(int64_t M, int64_t N, int64_t K, int bm, int bn) {
+// Rowwise / per-tensor / MXFP8 K split for launches short of one round of 256 x 256 tiles
+// (256 workgroups, one per CU): as many splits as still fit in that one round, at least
+// 1024 K each (the last may be shorter). Spilling into a second round doubles the time of
+// the splits and multiplies the partial-sum traffic (Qwen2 down at M = 2048: 5 splits
+// 231 us, 2 splits fill the round).
+int64_t scaled_split(int64_t M, int64_t N, int64_t K) {
   if (K % 128) return 1;
-  const int64_t round = bm == kBigTile ? 256 : kBlkSplitTarget;
-  const int64_t tiles = cdiv(M, bm) * cdiv(N, bn);
-  if (tiles * 2 > round) return 1;
-  const int64_t want = round / tiles, most = K / 1024;
+  const int64_t tiles = cdiv(M, kBigTile) * cdiv(N, kBigTile);
+  if (tiles * 2 > 256) return 1;
+  const int64_t want = 256 / tiles, most = K / 1024;
   const int64_t split = want < most ? want : most;
   if (split <= 1) return 1;
   const int64_t kps = cdiv(K / 128, split) * 128;
@@ -1728,182 +1695,20 @@ size_t tail_workspace(const TailPlan& p) {
 }
 
 size_t scaled_split_workspace(int64_t M, int64_t N, int64_t K) {
-  const int bm = M <= 32 ? 32 : (M <= 64 ? 64 : 128);
-  int64_t split = scaled_split(M, N, K, bm, 128);
-  if (M >= 256 && N >= 256) {
-    const int64_t big = scaled_split(M, N, K, kBigTile, kBigTile);
-    split = big > split ? big : split;
-  }
+  if (M < kBigTile || N < kBigTile) return 0;
+  const int64_t split = scaled_split(M, N, K);
   return split > 1 ? (size_t)split * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
-// Mirrors launch_gemm<MODE_BLOCK>: up to 64 rows the general kernel's split (any N);
-// above, the 128 x 128 kernel's split when N allows that kernel (else no split).
+// Upper bounds over the block kernels that may take the launch (alignment and the models
+// decide which one does).
 bool block256_wanted(int64_t M, int64_t N, int64_t K);
 size_t block_split_workspace(int64_t M, int64_t N, int64_t K) {
-  int64_t split = M <= 64 ? general_split(M, N, K) : (N >= kBlkTile ? block_split(M, N, K) : 1);
-  // The 256 x 256 kernel when it takes the launch (an upper bound: alignment may still
-  // send the launch to the 128 x 128 kernel).
+  int64_t split = M > 64 && N >= kBlkTile ? block_split(M, N, K) : 1;
   if (block256_wanted(M, N, K)) {
     const int64_t s256 = block256_split(M, N, K);
     split = s256 > split ? s256 : split;
   }
   return split > 1 ? (size_t)split * (size_t)M * (size_t)N * sizeof(float) : 0;
-}
-
-// MXFP8 large-tile kernel with 128-K stages: two 64 KB LDS stages, one code dword (four
-// UE8M0 codes) per fragment row and stage. The 64-K-stage kernel above would need one
-// code load per row and stage, which doubles its L2 request count; until its codes
-// travel in wider blocks, MXFP8 keeps this pipeline (K % 128 == 0).
-constexpr int kMx128Stage = 2 * kBigTile * BK;  // 64 KB
-
-template <int MODE>
-__global__ __launch_bounds__(kThreads, 1) void fp8_gemm_mx128_kernel(GemmArgs g) {
-  static_assert(MODE == MODE_MX, "MX codes only");
-  constexpr int FN = 4, FM = 4;                  // 32x32 MFMA tiles per wavefront (n, m)
-  constexpr int kLoads = kMx128Stage / 1024 / 4;   // direct loads per wavefront per stage
-  // Two distinct LDS objects (not one array indexed by stage), so the compiler can
-  // tell that reads of one stage never alias the in-flight direct loads of the other
-  // and does not wait for those loads before reading.
-  __shared__ __attribute__((aligned(1024))) uint8_t lds0[kMx128Stage];
-  __shared__ __attribute__((aligned(1024))) uint8_t lds1[kMx128Stage];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wn = wave >> 1, wm = wave & 1;
-  const int h = lane >> 5, frow = lane & 31;
-  int tm, tn;
-  big_tile_coords(blockIdx.x, g.tiles_m, (int)cdiv(g.N, kBigTile), tm, tn);
-  const int64_t n_base = (int64_t)tn * kBigTile, m_base = (int64_t)tm * kBigTile;
-  const int nk = (int)(g.K / BK);
-
-  // Direct loads: wavefronts 0-1 fetch the 256 weight rows, 2-3 the 256 activation
-  // rows (128 each), as buffer loads into LDS. Load instruction jj of a wavefront
-  // fills LDS tile rows r = 8 * (16 * wave + jj) + lane/8; lane fetches logical chunk
-  // (lane & 7) ^ ((r >> 1) & 7), which depends only on the lane and jj's parity. The
-  // buffer resource starts at the wavefront's first row and ends at the operand's last
-  // row: rows past M / N read as zero (their results are never stored), no clamping.
-  // Per load: a per-lane vector offset (row, chunk) and a wave-uniform scalar offset
-  // (jj's 8 rows + K step), so no 64-bit address is kept per load.
-  const int q = lane >> 3, pc = lane & 7;
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);  // keep the descriptor in SGPRs
-  const bool w_wave = wave_u < 2;
-  const int64_t ld = w_wave ? g.ldw : g.lda;
-  const int64_t row0 = (w_wave ? n_base : m_base) + (wave_u & 1) * 128;
-  const OperandWindow win = operand_window(row0, w_wave ? g.N : g.M, ld);
-  const __amdgpu_buffer_rsrc_t op_rsrc = uniform_rsrc((w_wave ? g.w : g.a) + win.base_offset, win.records);
-  const int voff[2] = {(int)(q * ld) + ((pc ^ ((q >> 1) & 7)) << 4), (int)(q * ld) + ((pc ^ ((4 + (q >> 1)) & 7)) << 4)};
-  auto issue_stage = [&](int kt, uint8_t* dst) {
-#pragma unroll
-    for (int jj = 0; jj < kLoads; ++jj) {
-      const int soff = __builtin_amdgcn_readfirstlane((int)(jj * 8 * ld) + kt * BK);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(op_rsrc, (__attribute__((address_space(3))) void*)(dst + (wave_u * kLoads + jj) * 1024),
-                                               16, voff[jj & 1], soff, 0, 0);
-    }
-  };
-  // Fragment reads. A fragment row is frow + (a multiple of 32), so its swizzle term
-  // (row >> 1) & 7 == (frow >> 1) & 7 is the same for every fragment of this lane: the
-  // four chunk offsets below plus compile-time row offsets address all of them.
-  const int fsw = (frow >> 1) & 7;
-  const int choff[4] = {(h ^ fsw) << 4, ((2 + h) ^ fsw) << 4, ((4 + h) ^ fsw) << 4, ((6 + h) ^ fsw) << 4};
-  auto frag = [&](const uint8_t* buf, int tile_row0, int ks) -> v8i {
-    const uint8_t* base = buf + (tile_row0 + frow) * BK;
-    const uint4 lo = *reinterpret_cast<const uint4*>(base + choff[2 * ks]);
-    const uint4 hi = *reinterpret_cast<const uint4*>(base + choff[2 * ks + 1]);
-    v8i r;
-    r[0] = (int)lo.x; r[1] = (int)lo.y; r[2] = (int)lo.z; r[3] = (int)lo.w;
-    r[4] = (int)hi.x; r[5] = (int)hi.y; r[6] = (int)hi.z; r[7] = (int)hi.w;
-    return r;
-  };
-  // MX: the four UE8M0 codes of one row for K step kt (one dword; K/32 % 4 == 0).
-  uint32_t wsc[FN], asc[FM];
-  // MX codes via buffer loads as well: rows past M / N read zero codes (never stored).
-  const OperandWindow wcw = MODE == MODE_MX ? operand_window(n_base + (wave_u >> 1) * 128, g.N, g.ld_sb) : OperandWindow{0, 0};
-  const OperandWindow acw = MODE == MODE_MX ? operand_window(m_base + (wave_u & 1) * 128, g.M, g.ld_sa) : OperandWindow{0, 0};
-  const __amdgpu_buffer_rsrc_t wcode_rsrc = uniform_rsrc(reinterpret_cast<const uint8_t*>(g.sb) + wcw.base_offset, wcw.records);
-  const __amdgpu_buffer_rsrc_t acode_rsrc = uniform_rsrc(reinterpret_cast<const uint8_t*>(g.sa) + acw.base_offset, acw.records);
-  auto load_mx_codes = [&](int kt) {
-    if constexpr (MODE == MODE_MX) {
-#pragma unroll
-      for (int i = 0; i < FN; ++i)
-        wsc[i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(wcode_rsrc, (int)((i * 32 + frow) * g.ld_sb), kt * 4, 0);
-#pragma unroll
-      for (int j = 0; j < FM; ++j)
-        asc[j] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(acode_rsrc, (int)((j * 32 + frow) * g.ld_sa), kt * 4, 0);
-    }
-  };
-
-  // Declaring an AGPR clobber makes the compiler select the AGPR form of the MFMAs,
-  // so the 256 accumulators live in the accumulation registers and the 256
-  // architectural VGPRs stay free for fragments and addresses.
-  asm volatile("" ::: "a255");
-  v16f acc[FN][FM];
-#pragma unroll
-  for (int i = 0; i < FN; ++i)
-#pragma unroll
-    for (int j = 0; j < FM; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-  // One K step from `cur` while the next step's loads stream into `nxt`. Fragments
-  // are double-buffered: the 64-K half ks+1 is read from LDS while the 16 MFMAs of
-  // half ks execute.
-  //
-  // The body has no branches: the next step's loads are issued unconditionally (the
-  // last step re-loads itself into the buffer nobody reads again), so the whole loop
-  // body is one basic block and the MFMAs cannot be moved below the barrier.
-  auto stage = [&](int kt, const uint8_t* cur, uint8_t* nxt) {
-    const int kn = kt + 1 < nk ? kt + 1 : kt;
-    uint32_t wcur[FN], acur[FM];
-#pragma unroll
-    for (int i = 0; i < FN; ++i) wcur[i] = wsc[i];
-#pragma unroll
-    for (int j = 0; j < FM; ++j) acur[j] = asc[j];
-    issue_stage(kn, nxt);
-    load_mx_codes(kn);
-    // Keep the next step's loads at the top of the step (the scheduler would otherwise
-    // sink them next to the barrier that waits for them).
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int ks = 0; ks < BK / 64; ++ks) {
-      v8i af[FM], wf[FN];
-#pragma unroll
-      for (int j = 0; j < FM; ++j) af[j] = frag(cur, kBigTile + wm * 128 + j * 32, ks);
-#pragma unroll
-      for (int i = 0; i < FN; ++i) wf[i] = frag(cur, wn * 128 + i * 32, ks);
-      const int shift = 8 * (ks * 2 + h);
-#pragma unroll
-      for (int i = 0; i < FN; ++i) {
-        const int sw = MODE == MODE_MX ? (int)((wcur[i] >> shift) & 0xFF) : kScaleOne;
-#pragma unroll
-        for (int j = 0; j < FM; ++j) {
-          const int sa = MODE == MODE_MX ? (int)((acur[j] >> shift) & 0xFF) : kScaleOne;
-          acc[i][j] = mfma(wf[i], af[j], acc[i][j], sw, sa);
-        }
-      }
-    }
-    // MFMAs touch no memory, so the compiler may sink them below the barrier, whose
-    // wait for all loads would then stall on the loads just issued for the next step
-    // before any MFMA of this step. Pin them above it.
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-  };
-
-  // The loop body is the unconditional pair of steps (lds0, lds1): a conditional
-  // second step would make the accumulators a phi across a branch, and the compiler
-  // then copies all 256 of them between AGPRs and VGPRs every iteration. An odd step
-  // count peels the first step, staged in lds1.
-  const int k0 = nk & 1;
-  issue_stage(0, k0 ? lds1 : lds0);
-  load_mx_codes(0);
-  __syncthreads();
-  if (k0) stage(0, lds1, lds0);
-  for (int kt = k0; kt < nk; kt += 2) {
-    stage(kt, lds0, lds1);
-    stage(kt + 1, lds1, lds0);
-  }
-
-  // The last step's barrier guarantees no wavefront still reads lds0 / lds1 and every
-  // direct load has landed (the last issue re-loaded a step into the idle buffer).
-  big_epilogue<MODE>(g, acc, BigScales{}, m_base, n_base, lds0);
 }
 
 // Compute units of the current device (cached per device): the persistent pair
@@ -1961,32 +1766,27 @@ int launch_big(GemmArgs g, hipStream_t st, const char* op) {
   const int64_t tiles = (int64_t)g.tiles_m * cdiv(g.N, kBigTile);
   if (tiles > 0x7FFFFFFF) return fail(AYK_EINVAL, "%s: problem too large", op);
   if constexpr (MODE == MODE_MX) {
-    if (g.K % 512 == 0 && g.ld_sa % 16 == 0 && g.ld_sb % 16 == 0 && aligned16(g.sa) && aligned16(g.sb)) {
-      // K per split in whole chunks of four 128-K pairs (keeps the code rows 16-byte aligned)
-      const int64_t planned = xcd_pieces(scaled_split(g.M, g.N, g.K, kBigTile, kBigTile));
-      const int64_t kps = planned > 1 ? cdiv(g.K / 512, planned) * 512 : g.K;
-      const int64_t split = cdiv(g.K, kps);
-      g.kps = split > 1 ? kps : 0;
-      if (split > 1) {
-        const size_t need = (size_t)split * (size_t)g.M * (size_t)g.N * sizeof(float);
-        if (g.ws == nullptr || g.ws_bytes < need)
-          return fail(AYK_EWORKSPACE, "%s: workspace of %zu bytes required, %zu given", op, need, g.ws_bytes);
-      }
-      if (split == 1) return launch_pair_tail<MODE>(g, tiles, st, op);
-      note_plan("pair split=%d", (int)split);
-      g.items = (int)tiles;  // one item per workgroup, piece-major
-      g.kpieces = (int)split;
-      hipLaunchKernelGGL((fp8_gemm_pair_kernel<MODE>), dim3((unsigned)(tiles * split)), dim3(kThreads), 0, st, g);
-      if (int rc = check_launch(op)) return rc;
-      launch_split_reduce(block_split_reduce, g.ws, g.M, g.N, (int)split, g.bias, g.bias_dtype, g.out, g.out_dtype,
-                          g.ldo, st);
-    } else {
-      note_plan("mx128");
-      hipLaunchKernelGGL((fp8_gemm_mx128_kernel<MODE>), dim3((unsigned)tiles), dim3(kThreads), 0, st, g);
+    // K per split in whole chunks of four 128-K pairs (keeps the code rows 16-byte aligned)
+    const int64_t planned = xcd_pieces(scaled_split(g.M, g.N, g.K));
+    const int64_t kps = planned > 1 ? cdiv(g.K / 512, planned) * 512 : g.K;
+    const int64_t split = cdiv(g.K, kps);
+    g.kps = split > 1 ? kps : 0;
+    if (split > 1) {
+      const size_t need = (size_t)split * (size_t)g.M * (size_t)g.N * sizeof(float);
+      if (g.ws == nullptr || g.ws_bytes < need)
+        return fail(AYK_EWORKSPACE, "%s: workspace of %zu bytes required, %zu given", op, need, g.ws_bytes);
     }
+    if (split == 1) return launch_pair_tail<MODE>(g, tiles, st, op);
+    note_plan("pair split=%d", (int)split);
+    g.items = (int)tiles;  // one item per workgroup, piece-major
+    g.kpieces = (int)split;
+    hipLaunchKernelGGL((fp8_gemm_pair_kernel<MODE>), dim3((unsigned)(tiles * split)), dim3(kThreads), 0, st, g);
+    if (int rc = check_launch(op)) return rc;
+    launch_split_reduce(block_split_reduce, g.ws, g.M, g.N, (int)split, g.bias, g.bias_dtype, g.out, g.out_dtype,
+                        g.ldo, st);
   } else if (g.K % (2 * kBigK) == 0) {
     // INT8 never splits: a split's partial would leave the exact int32 accumulator.
-    const int64_t planned = MODE == MODE_SCALED ? xcd_pieces(scaled_split(g.M, g.N, g.K, kBigTile, kBigTile)) : 1;
+    const int64_t planned = MODE == MODE_SCALED ? xcd_pieces(scaled_split(g.M, g.N, g.K)) : 1;
     g.kps = planned > 1 ? scaled_kps(g.K, planned) : 0;
     const int64_t split = planned > 1 ? cdiv(g.K, g.kps) : 1;
     if (split > 1) {
@@ -2033,29 +1833,16 @@ int launch_block_big(GemmArgs g, hipStream_t st, const char* op) {
   return check_launch(op);
 }
 
-template <int MODE, int BN, int BM, int WN, int WM>
-int launch_cfg(GemmArgs g, hipStream_t st, const char* op) {
-  g.tiles_m = (int)cdiv(g.M, BM);
-  const int64_t tiles = (int64_t)g.tiles_m * cdiv(g.N, BN);
+// The general kernel: operands whose row strides leave the medium tiles' 32-bit offsets.
+template <int MODE>
+int launch_general(GemmArgs g, hipStream_t st, const char* op) {
+  constexpr int kTile = 128;
+  g.tiles_m = (int)cdiv(g.M, kTile);
+  const int64_t tiles = (int64_t)g.tiles_m * cdiv(g.N, kTile);
   if (tiles > 0x7FFFFFFF) return fail(AYK_EINVAL, "%s: problem too large", op);
-  const int64_t split = MODE == MODE_BLOCK ? (BM <= 64 ? general_split(g.M, g.N, g.K) : 1)
-                        : (MODE == MODE_INT8 ? 1 : scaled_split(g.M, g.N, g.K, BM, BN));
-  g.kps = 0;
-  if (split > 1) {
-    const size_t need = (size_t)split * (size_t)g.M * (size_t)g.N * sizeof(float);
-    if (g.ws == nullptr || g.ws_bytes < need)
-      return fail(AYK_EWORKSPACE, "%s: workspace of %zu bytes required, %zu given", op, need, g.ws_bytes);
-    g.kps = MODE == MODE_BLOCK ? g.K / split : scaled_kps(g.K, split);
-  }
-  note_plan("general %dx%d split=%d", BM, BN, (int)split);
-  hipLaunchKernelGGL((fp8_gemm_kernel<MODE, BN, BM, WN, WM>), dim3((unsigned)tiles, (unsigned)split), dim3(kThreads), 0, st, g);
-  if (int rc = check_launch(op)) return rc;
-  if (split > 1) {
-    launch_split_reduce(block_split_reduce, g.ws, g.M, g.N, (int)split, g.bias, g.bias_dtype, g.out, g.out_dtype,
-                          g.ldo, st);
-    return check_launch(op);
-  }
-  return AYK_OK;
+  note_plan("general");
+  hipLaunchKernelGGL((fp8_gemm_kernel<MODE, kTile, kTile, 2, 2>), dim3((unsigned)tiles), dim3(kThreads), 0, st, g);
+  return check_launch(op);
 }
 
 // The 256 x 256 block-scaled kernel serves launches of at least half a round (128) of
@@ -2096,37 +1883,88 @@ SkinnyFp8Args skinny_args(const GemmArgs& g, int mode) {
   return k;
 }
 
+constexpr MidMode mid_mode(int mode) {
+  return mode == MODE_BLOCK ? kMidBlock : (mode == MODE_MX ? kMidMx : (mode == MODE_INT8 ? kMidInt8 : kMidScaled));
+}
+MidArgs mid_args(const GemmArgs& g) {
+  return {g.a, g.lda, g.w, g.ldw, g.M, g.N, g.K, g.sa, g.sa_dtype, g.sa_vec, g.ld_sa, g.sb, g.sb_dtype, g.sb_vec, g.ld_sb,
+          g.bias, g.bias_dtype, g.out, g.out_dtype, g.ldo, g.ws, g.ws_bytes};
+}
+
+// Modelled times (microseconds) of the large-tile kernels on the plans above, fitted on
+// the shapes of the medium-tile kernel's model (3-4% mean error): a launch, `rounds` of
+// one workgroup a CU over `steps` 128-K blocks each, a split's reduce and partials.
+// A launch goes to the medium tiles where their model is below 0.95 (block-128 128 x 128
+// kernel: 0.9) of these: over the fitted shapes no such launch got slower, and batches of
+// 256 to 2048 rows gained 19% (per-row), 17% (MXFP8) and 10% (block) in the mean.
+struct LargeModel {
+  float base, step, tile, reduce, partial;
+  float time(int64_t rounds, int64_t steps, int64_t split, int64_t part_elems) const {
+    return base + (float)rounds * ((float)steps * step + tile) + (split > 1 ? reduce + partial * (float)part_elems : 0.0f);
+  }
+};
+constexpr LargeModel kPairScaled{2.7f, 1.57f, 2.65f, 8.6f, 1.0e-6f}, kPairMx{3.5f, 1.79f, 1.6f, 7.8f, 0.9e-6f};
+constexpr LargeModel kBlock256{0.1f, 1.85f, 4.5f, 3.4f, 1.3e-6f}, kBlock128{6.0f, 0.97f, 1.8f, 0.0f, 2.1e-6f};
+
+float pair_time(int mode, int64_t M, int64_t N, int64_t K) {
+  const bool mx = mode == MODE_MX;
+  const LargeModel& m = mx ? kPairMx : kPairScaled;
+  const int64_t unit = mx ? 512 : 128, tiles = cdiv(M, kBigTile) * cdiv(N, kBigTile);
+  if (mode == MODE_INT8) return m.time(cdiv(tiles, 256), cdiv(K, 128), 1, 0);  // never split
+  const int64_t planned = xcd_pieces(scaled_split(M, N, K));
+  if (planned > 1) {
+    const int64_t kps = cdiv(K / unit, planned) * unit, split = cdiv(K, kps);
+    return m.time(1, cdiv(kps, 128), split, split * M * N);
+  }
+  const TailPlan tp = tail_plan(M, N, K, mx);
+  if (tp.split == 1) return m.time(cdiv(tiles, 256), cdiv(K, 128), 1, 0);
+  return m.time(tp.dp_tiles / 256, K / 128, 1, 0) - m.base +
+         m.time(1, K / 128 / tp.split, tp.split, (int64_t)tp.split * tp.tail_tiles * kBigTile * kBigTile);
+}
+float block256_time(int64_t M, int64_t N, int64_t K) {
+  const int64_t split = block256_split(M, N, K);
+  return kBlock256.time(cdiv(cdiv(M, 256) * cdiv(N, 256) * split, 256), cdiv(K / 128, split), split, split * M * N);
+}
+float block128_time(int64_t M, int64_t N, int64_t K) {
+  const int64_t split = block_split(M, N, K);
+  return kBlock128.time(cdiv(cdiv(M, kBlkTile) * cdiv(N, kBlkTile) * split, 256), K / 128 / split, split, split * M * N);
+}
+
 template <int MODE>
 int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
-  // The large-tile kernels need K % 64 == 0 (128 for MXFP8), fp32 scales, N % 4 == 0 and 16-byte
-  // aligned output rows (its epilogue stores 16-byte chunks); anything else runs the
-  // general kernel.
+  const MidArgs mid = mid_args(g);
+  const bool mid_ok = mid_supported(mid);
+  // Whether the medium tiles beat a kernel that is modelled at `us`.
+  auto mid_beats = [&](float us) { return mid_ok && mid_time(mid_mode(MODE), g.M, g.N, g.K) < us; };
+  // The large-tile kernels need K % 64 == 0, fp32 scales (MXFP8: K % 512 == 0 and 16-byte
+  // aligned code rows), N % 4 == 0 and 16-byte aligned output rows (its epilogue stores
+  // 16-byte chunks).
   if constexpr (MODE != MODE_BLOCK) {
   const int64_t out_bytes = g.out_dtype == AYK_F32 ? 4 : 2;
   // (256 rows of the output, and of an fp32 partial [M, N], within 2 GB: the pair
   // kernel's epilogue addresses a tile with 32-bit offsets.)
-  const bool big_ok = g.K % (MODE == MODE_MX ? BK : kBigK) == 0 && g.M >= 256 && g.N >= 256 && g.N % 4 == 0 &&
+  const bool codes_ok = MODE != MODE_MX || (g.K % 512 == 0 && g.ld_sa % 16 == 0 && g.ld_sb % 16 == 0 && aligned16(g.sa) && aligned16(g.sb));
+  const bool big_ok = codes_ok && g.K % kBigK == 0 && g.M >= 256 && g.N >= 256 && g.N % 4 == 0 &&
                       (g.ldo * out_bytes) % 16 == 0 && aligned16(g.out) && g.ldo < (1 << 21) && g.N < (1 << 21) &&
                       (MODE == MODE_MX || (g.sa_dtype == AYK_F32 && g.sb_dtype == AYK_F32 &&
                                            (!g.sb_vec || aligned16(g.sb)))) &&
                       (g.bias == nullptr || (reinterpret_cast<uintptr_t>(g.bias) & 15) == 0);
-  if (big_ok) return launch_big<MODE>(g, st, op);
+  if (big_ok && !mid_beats(0.95f * pair_time(MODE, g.M, g.N, g.K))) return launch_big<MODE>(g, st, op);
   } else {
     // The 256 x 256 block-scaled kernel from half a round of its tiles on.
     if (g.sa_dtype == AYK_F32 && block256_wanted(g.M, g.N, g.K)) {
       const Block256Args b = block256_args(g);
-      if (block256_supported(b)) return block256_launch(b, st, op);
+      if (block256_supported(b) && !mid_beats(0.95f * block256_time(g.M, g.N, g.K))) return block256_launch(b, st, op);
     }
     // The block-scaled 128 x 128 kernel: K % 128 == 0, fp32 activation scales, any float
     // weight-scale dtype, and the same output / bias alignment as above.
     const int64_t out_bytes = g.out_dtype == AYK_F32 ? 4 : 2;
-    // 65-127 rows also take it when the K split applies (rows past M read zeros); up to
-    // 64 rows the general kernel's 32- / 64-row tiles split K instead.
+    // 65-127 rows also take it when the K split applies (rows past M read zeros).
     const bool big_ok = g.K % 128 == 0 && (g.M >= kBlkTile || (g.M > 64 && block_split(g.M, g.N, g.K) > 1)) && g.N >= kBlkTile &&
                         g.N % 4 == 0 && g.sa_dtype == AYK_F32 &&
                         (g.ldo * out_bytes) % 16 == 0 && aligned16(g.out) &&
                         (g.bias == nullptr || (reinterpret_cast<uintptr_t>(g.bias) & 15) == 0);
-    if (big_ok) return launch_block_big(g, st, op);
+    if (big_ok && !mid_beats(0.9f * block128_time(g.M, g.N, g.K))) return launch_block_big(g, st, op);
   }
   // Decode batches (M <= 64) with fp32 or UE8M0 scales: the weight-streaming kernel
   // (gemm_skinny.hip) where its shape and alignment rules hold.
@@ -2136,9 +1974,8 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
       if (skinny_fp8_supported(sk)) return skinny_fp8_launch(sk, st, op);
     }
   }
-  if (g.M <= 32) return launch_cfg<MODE, 128, 32, 4, 1>(g, st, op);
-  if (g.M <= 64) return launch_cfg<MODE, 128, 64, 2, 2>(g, st, op);
-  return launch_cfg<MODE, 128, 128, 2, 2>(g, st, op);
+  if (mid_ok) return mid_launch(mid_mode(MODE), mid, st, op);
+  return launch_general<MODE>(g, st, op);
 }
 
 bool is_float_dtype(int dt) { return dt == AYK_F32 || dt == AYK_F16 || dt == AYK_BF16; }
@@ -2165,10 +2002,8 @@ extern "C" {
 
 size_t ayk_fp8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 1 || K < 1) return 0;
-  const size_t split = scaled_split_workspace(M, N, K);
   const size_t tail = M >= kBigTile && N >= kBigTile ? tail_workspace(tail_plan(M, N, K, false)) : 0;
-  const size_t skinny = skinny_fp8_workspace(M, N, K, 0);
-  return split > tail ? (split > skinny ? split : skinny) : (tail > skinny ? tail : skinny);
+  return std::max({scaled_split_workspace(M, N, K), tail, skinny_fp8_workspace(M, N, K, 0), mid_workspace(kMidScaled, M, N, K)});
 }
 
 int ayk_fp8_scaled_mm(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N,
@@ -2249,9 +2084,7 @@ int ayk_int8_scaled_mm(const void* a, int64_t lda, const void* b, int64_t ldb, i
 
 size_t ayk_fp8_blockwise_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 1 || K < 1 || K % 128) return 0;
-  const size_t split = block_split_workspace(M, N, K);
-  const size_t skinny = skinny_fp8_workspace(M, N, K, 2);
-  return split > skinny ? split : skinny;
+  return std::max({block_split_workspace(M, N, K), skinny_fp8_workspace(M, N, K, 2), mid_workspace(kMidBlock, M, N, K)});
 }
 
 int ayk_fp8_blockwise_mm(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t M,
@@ -2323,10 +2156,8 @@ int ayk_fp8_grouped_blockwise_mm(const void* a, const void* b, const float* scal
 
 size_t ayk_mxfp8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 1 || K < 1) return 0;
-  const size_t split = scaled_split_workspace(M, N, K);
   const size_t tail = M >= kBigTile && N >= kBigTile ? tail_workspace(tail_plan(M, N, K, true)) : 0;
-  const size_t skinny = skinny_fp8_workspace(M, N, K, 1);
-  return split > tail ? (split > skinny ? split : skinny) : (tail > skinny ? tail : skinny);
+  return std::max({scaled_split_workspace(M, N, K), tail, skinny_fp8_workspace(M, N, K, 1), mid_workspace(kMidMx, M, N, K)});
 }
 
 int ayk_mxfp8_scaled_mm(const void* a, int64_t lda, const uint8_t* a_scale, int64_t ld_as,

@@ -555,7 +555,10 @@ SkPlan skinny_plan(int64_t M, int64_t N, int64_t K, int sm) {
   while (wgs * split * 2 <= 256 && K % (gran * split * 2) == 0 && K / (split * 2) >= 2048) split *= 2;
   p.split = (int)split;
   p.kps = K / split;
-  p.ok = wgs <= 0x7FFFFFFF;
+  // A K whose factors allow neither parts nor a split leaves each wavefront one long walk
+  // on a few CUs: the medium tiles (gemm_mid.hip) split such a K and take it (MXFP8, M = 40:
+  // 4096 x 11008 68 -> 26 us; per-row, M = 64: 3584 x 18944 49 -> 26 us).
+  p.ok = wgs <= 0x7FFFFFFF && p.kps / p.ks <= 8192;
   return p;
 }
 

@@ -21,6 +21,7 @@
 #include "ayk_common.h"
 #include "gemm_tiles.h"
 #include "gemm_util.h"
+#include "tile_store.h"
 
 namespace ayk {
 namespace {
@@ -221,24 +222,15 @@ __global__ __launch_bounds__(WN * WM * 64, WGS) void w8a16_tile_kernel(W16TileAr
         for (int grp = 0; grp < 4; ++grp) {
           const int64_t n = n_w + 32 * i + 8 * grp + 4 * h;
           const float v[4] = {acc[i][j][4 * grp], acc[i][j][4 * grp + 1], acc[i][j][4 * grp + 2], acc[i][j][4 * grp + 3]};
-          if (n + 3 < g.N && g.N % 4 == 0) {
-            *reinterpret_cast<float4*>(prow + n) = make_float4(v[0], v[1], v[2], v[3]);
-          } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              if (n + q < g.N) prow[n + q] = v[q];
-          }
+          store4_f32(prow + n, g.N - n, v);
         }
     }
     return;
   }
-  // Every wavefront stages 32 (m) x TN (n) slabs in a private region of the stage buffers
-  // (16-byte chunks XOR-swizzled by row) and stores them row by row in 16-byte pieces.
-  constexpr int kRowB = TN * 2, kChunks = kRowB / 16, kRowsPerStore = 64 / kChunks;
-  constexpr int kRegion = 32 * kRowB, kPerBuf = kStage / kRegion;
+  // Every wavefront stages 32 (m) x TN (n) slabs in a private region of the stage buffers.
+  constexpr int kRegion = 32 * TN * 2, kPerBuf = kStage / kRegion;
   static_assert(2 * kPerBuf >= kWaves, "the staging regions fit the stage buffers");
   uint8_t* region = wave < kPerBuf ? B0 + wave * kRegion : B1 + (wave - kPerBuf) * kRegion;
-  uint16_t* out = static_cast<uint16_t*>(g.out);
 #pragma unroll
   for (int j = 0; j < FM; ++j) {
 #pragma unroll
@@ -246,35 +238,9 @@ __global__ __launch_bounds__(WN * WM * 64, WGS) void w8a16_tile_kernel(W16TileAr
 #pragma unroll
       for (int grp = 0; grp < 4; ++grp) {
         const float v[4] = {acc[i][j][4 * grp], acc[i][j][4 * grp + 1], acc[i][j][4 * grp + 2], acc[i][j][4 * grp + 3]};
-        const int byte = 2 * (32 * i + 8 * grp + 4 * h);
-        uint8_t* dst = region + frow * kRowB + (((byte >> 4) ^ (frow & (kChunks - 1))) << 4) + (byte & 15);
-        uint2 pk;
-        if constexpr (BF16) {
-          pk = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-        } else {
-          pk = make_uint2((uint32_t)f32_to_f16_bits(v[0]) | ((uint32_t)f32_to_f16_bits(v[1]) << 16),
-                          (uint32_t)f32_to_f16_bits(v[2]) | ((uint32_t)f32_to_f16_bits(v[3]) << 16));
-        }
-        *reinterpret_cast<uint2*>(dst) = pk;
+        stage_slab16<BF16, TN>(region, frow, 2 * (32 * i + 8 * grp + 4 * h), v);
       }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wavefront's own staging writes
-#pragma unroll
-    for (int r0 = 0; r0 < 32; r0 += kRowsPerStore) {
-      const int rr = r0 + lane / kChunks, cc = lane % kChunks;
-      const int64_t gm = m_w + 32 * j + rr, gn = n_w + 8 * cc;
-      const v4i val = *reinterpret_cast<const v4i*>(region + rr * kRowB + ((cc ^ (rr & (kChunks - 1))) << 4));
-      if (gm < g.M && gn < g.N) {
-        uint16_t* p = out + gm * g.ldo + gn;
-        if (gn + 8 <= g.N && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
-          __builtin_nontemporal_store(val, reinterpret_cast<v4i*>(p));
-        } else {
-#pragma unroll
-          for (int c = 0; c < 8; ++c)
-            if (gn + c < g.N) p[c] = (uint16_t)((uint32_t)val[c / 2] >> (16 * (c % 2)));
-        }
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read back before the next slab overwrites it
+    store_slab16<TN>(region, static_cast<uint16_t*>(g.out), g.ldo, g.M, g.N, m_w + 32 * j, n_w, lane);
   }
 }
 

@@ -1,0 +1,119 @@
+"""GPU: the medium-tile W8A8 GEMM at the edges of its tiles, K stages, scale chunks and K
+splits, for every recipe, against the fp64 product of the same operands under the
+package's stated tolerance (``tests/_tol.py``); INT8 against the exact integer sum."""
+
+import pytest
+import torch
+
+from tests._tol import assert_linear_close
+
+pytestmark = pytest.mark.gpu
+FP8 = torch.float8_e4m3fn
+
+
+def _fp8(shape, g):
+    return (torch.randn(shape, generator=g) * 50).clamp(-448, 448).to(FP8)
+
+
+def _expand(scale, rows, cols, by, bx):
+    return scale.double().repeat_interleave(by, 0)[:rows].repeat_interleave(bx, 1)[:, :cols]
+
+
+def _run(recipe, m, n, k, bias, odt, col_major, gpu):
+    """(output, fp64 reference, plan) of one call with seeded operands."""
+    from ayaka.kernel.hip import _lib, fp8_blockwise_mm, fp8_scaled_mm, mxfp8_scaled_mm
+
+    g = torch.Generator().manual_seed(m * 131 + n * 7 + k)
+    a, w = _fp8((m, k), g), _fp8((n, k), g)
+    b = torch.randn(n, generator=g).to(odt) if bias else None
+    out = torch.empty(m, n, dtype=odt, device=gpu)
+    bg = None if b is None else b.to(gpu)
+    if recipe == "scaled":
+        sa, sb = torch.rand(m, generator=g) * 1e-2, torch.rand(n, generator=g) * 1e-2
+        fp8_scaled_mm(a.to(gpu), w.to(gpu).t(), sa.to(gpu), sb.to(gpu), bias=bg, out=out)
+        sa, sb = sa[:, None].double(), sb[:, None].double()
+    elif recipe == "scalar":
+        sa, sb = torch.tensor(0.003), torch.tensor(0.02)
+        fp8_scaled_mm(a.to(gpu), w.to(gpu).t(), sa.to(gpu), sb.to(gpu), bias=bg, out=out)
+    elif recipe == "block":
+        kb = -(-k // 128)
+        ta, tb = torch.rand(m, kb, generator=g) * 1e-2, torch.rand(-(-n // 128), kb, generator=g) * 1e-2
+        if not col_major:
+            tb = tb.to(torch.bfloat16)
+        table = ta.t().contiguous() if col_major else ta
+        fp8_blockwise_mm(a.to(gpu), w.to(gpu), table.to(gpu), tb.to(gpu), bias=bg, out=out, a_scale_col_major=col_major)
+        sa, sb = _expand(ta, m, k, 1, 128), _expand(tb, n, k, 128, 128)
+    else:
+        ca = torch.randint(112, 122, (m, k // 32), generator=g, dtype=torch.uint8)
+        cb = torch.randint(112, 122, (n, k // 32), generator=g, dtype=torch.uint8)
+        mxfp8_scaled_mm(a.to(gpu), ca.to(gpu), w.to(gpu), cb.to(gpu), bg, out=out)
+        sa, sb = (_expand(torch.exp2(c.double() - 127), c.shape[0], k, 1, 32) for c in (ca, cb))
+    plan = _lib.last_plan()
+    ref = (a.double() * sa).to(gpu) @ (w.double() * sb).to(gpu).t()
+    return out, ref if b is None else ref + bg.double(), plan
+
+
+@pytest.mark.parametrize("recipe,m,n,k,bias,odt,col_major", [
+    ("scaled", 65, 129, 16, True, torch.float32, False),       # one short stage
+    ("scaled", 100, 128, 128, False, torch.bfloat16, False),   # exact stage
+    ("scaled", 33, 1001, 4112, True, torch.float16, False),    # K tail, odd N, split
+    ("scaled", 300, 2052, 3696, True, torch.float16, False),   # K % 64 != 0
+    ("scalar", 255, 300, 2064, False, torch.float32, False),   # odd stage count
+    ("scaled", 1025, 3072, 1024, True, torch.bfloat16, False),
+    ("scaled", 700, 9000, 2096, False, torch.bfloat16, False),
+    ("block", 70, 130, 128, True, torch.bfloat16, True),
+    ("block", 65, 1000, 4096, False, torch.float16, True),     # split
+    ("block", 129, 2052, 1152, True, torch.float32, False),    # row-major, bf16 weight scales
+    ("block", 40, 100, 384, False, torch.bfloat16, False),     # N < 128
+    ("block", 1000, 4096, 4096, False, torch.bfloat16, True),
+    ("mx", 66, 136, 512, True, torch.float32, False),          # one code chunk
+    ("mx", 100, 1000, 4096, False, torch.bfloat16, False),     # split in whole chunks
+    ("mx", 70, 260, 1184, True, torch.float16, False),         # K % 128 != 0: unaligned codes
+    ("mx", 40, 300, 2688, False, torch.bfloat16, False),       # K % 512 != 0
+    ("mx", 200, 2050, 2944, True, torch.float32, False),       # K % 512 != 0, split
+    ("mx", 40, 4096, 11008, False, torch.bfloat16, False),     # a K the decode kernel cannot split
+    ("mx", 300, 3072, 1536, True, torch.bfloat16, False),
+])
+def test_medium_tiles(gpu, recipe, m, n, k, bias, odt, col_major):
+    print(f"medium tiles recipe={recipe} m={m} n={n} k={k} bias={bias} out={odt} col_major={col_major}", flush=True)
+    out, ref, plan = _run(recipe, m, n, k, bias, odt, col_major, gpu)
+    assert plan.startswith("mid "), plan
+    assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("recipe,k", [("scaled", 4096), ("block", 4096), ("mx", 4096), ("mx", 1184)])
+def test_medium_tiles_half_outputs(gpu, recipe, k):
+    """16-bit outputs are the fp32 output rounded once (N % 4 != 0: no aligned rows)."""
+    m, n = 97, 642
+    full, _, plan = _run(recipe, m, n, k, False, torch.float32, False, gpu)
+    for odt in (torch.bfloat16, torch.float16):
+        half, _, plan2 = _run(recipe, m, n, k, False, odt, False, gpu)
+        assert plan == plan2 and torch.equal(half, full.to(odt))
+
+
+@pytest.mark.parametrize("m,n,k", [(8, 130, 16), (100, 1000, 1040), (65, 257, 4096), (300, 2052, 2064)])
+def test_medium_tiles_int8_exact(gpu, m, n, k):
+    """The int32 sums are exact (4096 x 127^2 < 2^31): scales of one return them rounded to fp32."""
+    from ayaka.kernel.hip import _lib, int8_scaled_mm
+
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.randint(-127, 128, (m, k), generator=g, dtype=torch.int8)
+    w = torch.randint(-127, 128, (n, k), generator=g, dtype=torch.int8)
+    out = int8_scaled_mm(a.to(gpu), w.to(gpu).t(), torch.ones(m, device=gpu), torch.ones(n, device=gpu), out_dtype=torch.float32)
+    assert _lib.last_plan().startswith("mid ")
+    assert torch.equal(out.cpu(), (a.double() @ w.double().t()).float())
+
+
+def test_medium_tiles_nan_codes_stay_in_their_row(gpu):
+    """A NaN code (weight rows of 37 groups, so that the next row's codes follow a row's last
+    stage at once) makes its own output column NaN and no other."""
+    from ayaka.kernel.hip import mxfp8_scaled_mm
+
+    m, n, k = 70, 140, 1184
+    g = torch.Generator().manual_seed(5)
+    a, w = _fp8((m, k), g).to(gpu), _fp8((n, k), g).to(gpu)
+    ca = torch.full((m, k // 32), 120, dtype=torch.uint8, device=gpu)
+    cb = torch.full((n, k // 32), 120, dtype=torch.uint8, device=gpu)
+    cb[3, 0] = 0xFF
+    y = mxfp8_scaled_mm(a, ca, w, cb, out=torch.empty(m, n, device=gpu))
+    assert y[:, 3].isnan().all() and torch.isfinite(y[:, [c for c in range(n) if c != 3]]).all()
