@@ -1,4 +1,4 @@
-"""MoE FP8 block-128 grouped GEMM on the gfx950 kernel ``fp8_grouped_block_kernel``.
+"""MoE FP8 block-128 grouped GEMM on the gfx950 kernel ``fp8_grouped_block256_kernel``.
 
 Same function, argument order, checks and messages as the reference's
 ``kernel/triton/moe/moe_grouped_gemm.py:599`` ``fp8_blockwise_scaled_grouped_mm``
@@ -12,12 +12,12 @@ output dtype once; rows of no expert are left untouched.
 
 The pointer tables (``a_ptrs`` .. ``b_scales_ptrs``) and scale-layout descriptors
 (``layout_sfa`` / ``layout_sfb``) are workspaces the reference fills as a side effect
-(``get_group_gemm_starts``, :61-135, in its normal and swap-AB flavours); they are
-filled here with the same values by device tensor arithmetic, without a host sync.
-The kernel itself reads ``problem_sizes`` and ``expert_offsets`` on the device and
-derives every operand address from them, so one kernel serves both flavours: swap-AB
-is a tiling choice of the CUTLASS kernels that changes the summation order only, and
-``swap_ab`` picks the flavour of the tables. ``stride_a/b/c`` must hold the dense
+(``get_group_gemm_starts``, :61-135, in its normal and swap-AB flavours); the kernel
+fills them with the same values (the function of that name here does it by tensor
+arithmetic), without a host sync. For the product it reads ``problem_sizes`` and
+``expert_offsets`` on the device and derives every operand address from them, so one
+kernel serves both flavours: swap-AB is a tiling choice of the CUTLASS kernels that
+changes the summation order only, and ``swap_ab`` picks the flavour of the tables. ``stride_a/b/c`` must hold the dense
 leading dimensions (K, K, N) that the layout checks below already imply; ``workspace``
 is accepted for signature compatibility only.
 """
@@ -173,17 +173,21 @@ def fp8_blockwise_scaled_grouped_mm(
 
     swap = (m_total <= 2048) if swap_ab is None else bool(swap_ab)
     with torch.cuda.device(a.device):
-        if swap:
-            transposed = torch.empty((num_experts, 3), dtype=torch.int32, device=a.device)
-            get_group_gemm_starts(expert_offsets, a_ptrs, b_ptrs, out_ptrs, a_scales_ptrs, b_scales_ptrs, b, a,
-                                  output, scales_b, scales_a, layout_sfa, layout_sfb, problem_sizes, transposed, True)
+        tables = (a_ptrs, b_ptrs, out_ptrs, a_scales_ptrs, b_scales_ptrs)
+        # The kernel fills the tables where it can write them as they are laid out here.
+        in_kernel = n > 0 and k > 0 and all(t.device == a.device for t in (*tables, layout_sfa, layout_sfb)) and all(
+            t.size(0) >= num_experts and t.size(1) >= 5 for t in (layout_sfa, layout_sfb))
+        if in_kernel:
+            targets = (*(t.data_ptr() for t in tables), layout_sfa.data_ptr(), layout_sfa.size(1),
+                       layout_sfb.data_ptr(), layout_sfb.size(1), int(swap))
         else:
-            get_group_gemm_starts(expert_offsets, a_ptrs, b_ptrs, out_ptrs, a_scales_ptrs, b_scales_ptrs, a, b,
-                                  output, scales_a, scales_b, layout_sfa, layout_sfb, problem_sizes, problem_sizes,
-                                  False)
+            targets = (None, None, None, None, None, None, 0, None, 0, 0)
+            operands = (b, a, output, scales_b, scales_a) if swap else (a, b, output, scales_a, scales_b)
+            transposed = torch.empty((num_experts, 3), dtype=torch.int32, device=a.device) if swap else problem_sizes
+            get_group_gemm_starts(expert_offsets, *tables, *operands, layout_sfa, layout_sfb, problem_sizes, transposed, swap)
         # Large batches: experts over the whole K read the activation scales transposed
         # ([K/128, M_total], 32 rows per cache line), copied once here; the same values.
         sa_t = scales_a.t().contiguous() if m_total >= COLUMN_MAJOR_SCALES_MIN_ROWS else None
-        _lib.call("ayk_fp8_grouped_blockwise_mm", a.data_ptr(), b.data_ptr(), scales_a.data_ptr(), _lib.ptr(sa_t),
+        _lib.call("ayk_fp8_grouped_blockwise_mm_tables", a.data_ptr(), b.data_ptr(), scales_a.data_ptr(), _lib.ptr(sa_t),
                   scales_b.data_ptr(), problem_sizes.data_ptr(), expert_offsets.data_ptr(), num_experts, m_total, n,
-                  k, output.data_ptr(), _lib.dtype_code(output.dtype), _lib.stream_of(output))
+                  k, output.data_ptr(), _lib.dtype_code(output.dtype), *targets, _lib.stream_of(output))

@@ -2122,6 +2122,17 @@ int ayk_fp8_grouped_blockwise_mm(const void* a, const void* b, const float* scal
                                  const int32_t* problem_sizes, const int32_t* expert_offsets, int64_t num_experts,
                                  int64_t m_total, int64_t n, int64_t k, void* out, int out_dtype,
                                  ayk_stream_t stream) {
+  return ayk_fp8_grouped_blockwise_mm_tables(a, b, scales_a, scales_a_t, scales_b, problem_sizes, expert_offsets, num_experts,
+                                             m_total, n, k, out, out_dtype, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                             nullptr, 0, nullptr, 0, 0, stream);
+}
+
+int ayk_fp8_grouped_blockwise_mm_tables(const void* a, const void* b, const float* scales_a, const float* scales_a_t,
+                                        const float* scales_b, const int32_t* problem_sizes, const int32_t* expert_offsets,
+                                        int64_t num_experts, int64_t m_total, int64_t n, int64_t k, void* out, int out_dtype,
+                                        int64_t* a_ptrs, int64_t* b_ptrs, int64_t* out_ptrs, int64_t* a_scales_ptrs,
+                                        int64_t* b_scales_ptrs, int32_t* layout_sfa, int64_t ld_sfa, int32_t* layout_sfb,
+                                        int64_t ld_sfb, int transpose, ayk_stream_t stream) {
   const char* op = "fp8_blockwise_scaled_grouped_mm";
   if (num_experts < 0 || m_total < 0 || n < 0 || k < 0)
     return fail(AYK_EINVAL, "%s: bad shape experts=%lld M=%lld N=%lld K=%lld", op, (long long)num_experts,
@@ -2136,8 +2147,11 @@ int ayk_fp8_grouped_blockwise_mm(const void* a, const void* b, const float* scal
       (reinterpret_cast<uintptr_t>(scales_b) & 3) || (reinterpret_cast<uintptr_t>(scales_a_t) & 3))
     return fail(AYK_EINVAL, "%s: operands must be 16-byte aligned (scales 4-byte)", op);
   if (k > 0x7FFFFFFF || n * k > ((int64_t)1 << 31)) return fail(AYK_EINVAL, "%s: expert weight too large", op);
+  if (a_ptrs && (!b_ptrs || !out_ptrs || !a_scales_ptrs || !b_scales_ptrs || !layout_sfa || !layout_sfb || ld_sfa < 5 || ld_sfb < 5))
+    return fail(AYK_EINVAL, "%s: tables come together, with layout rows of at least 5", op);
   if (int rc = check_device()) return rc;
   Grouped256Args gb{};
+  gb.tables = {a_ptrs, b_ptrs, out_ptrs, a_scales_ptrs, b_scales_ptrs, layout_sfa, layout_sfb, ld_sfa, ld_sfb, transpose};
   gb.a = static_cast<const uint8_t*>(a);
   gb.b = static_cast<const uint8_t*>(b);
   gb.sa = scales_a;

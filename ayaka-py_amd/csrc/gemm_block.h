@@ -31,6 +31,17 @@ struct Block256Args {
   int nt_stores;     // store final outputs nontemporally (set by the kernels, not callers)
 };
 
+// The per-expert address tables and scale descriptors that a grouped call fills beside its
+// output (a_ptrs null: none): normal flavour a = tokens at off_e K_e and b = weights at
+// e N_e K_e; `transpose` swaps the two roles. Descriptors are [rows, k blocks, 1, k blocks,
+// rows * k blocks], rows = tokens or 128-row weight blocks, at row stride ld_sfa / ld_sfb.
+struct GroupTables {
+  int64_t *a_ptrs, *b_ptrs, *out_ptrs, *a_scales_ptrs, *b_scales_ptrs;
+  int32_t *layout_sfa, *layout_sfb;
+  int64_t ld_sfa, ld_sfb;
+  int transpose;
+};
+
 // Grouped (MoE) problem: expert e owns activation rows [expert_offsets[e], + M_e) of
 // a [m_total, k] and weights b[e] = [n, k]; scales sa [m_total, k / 128], sb[e]
 // [n / 128, k / 128] fp32; out [m_total, n]. problem_sizes [E, 3] = (M_e, N_e, K_e) and
@@ -47,6 +58,7 @@ struct Grouped256Args {
   const int32_t* expert_offsets;
   int num_experts;
   int64_t m_total, n, k;
+  GroupTables tables;
 };
 
 // Whether the 256 x 256 kernel takes this problem (shape, alignment and dtype rules).

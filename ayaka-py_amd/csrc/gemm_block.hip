@@ -447,6 +447,36 @@ __device__ inline Expert256 expert256(const Grouped256Args& ga, int e) {
 }
 __device__ inline int64_t expert256_tiles(const Expert256& p) { return cdiv(p.m, kTile) * cdiv(p.n, kTile); }
 
+// The address tables of every expert, from problem_sizes and expert_offsets as they are
+// (not clamped: they describe the call, nothing here reads through them).
+__device__ inline void fill_tables(const Grouped256Args& ga) {
+  const GroupTables& t = ga.tables;
+  const int64_t out_bytes = ga.out_dtype == AYK_F32 ? 4 : 2;
+  const auto addr = [](const void* p) { return (int64_t)reinterpret_cast<uintptr_t>(p); };
+  const int64_t tok = addr(ga.a), wgt = addr(ga.b), tok_s = addr(ga.sa), wgt_s = addr(ga.sb), out = addr(ga.out);
+  for (int e = threadIdx.x; e < ga.num_experts; e += kThreads) {
+    const int64_t m = ga.problem_sizes[3 * e], n = ga.problem_sizes[3 * e + 1], k = ga.problem_sizes[3 * e + 2];
+    const int64_t off = ga.expert_offsets[e];
+    const int64_t tok_at = tok + off * k, wgt_at = wgt + e * k * n;
+    const int64_t tok_s_at = tok_s + 4 * ((off * k) >> 7), wgt_s_at = wgt_s + 4 * ((e * k * n) >> 14);
+    t.a_ptrs[e] = t.transpose ? wgt_at : tok_at;
+    t.b_ptrs[e] = t.transpose ? tok_at : wgt_at;
+    t.a_scales_ptrs[e] = t.transpose ? wgt_s_at : tok_s_at;
+    t.b_scales_ptrs[e] = t.transpose ? tok_s_at : wgt_s_at;
+    t.out_ptrs[e] = out + off * n * out_bytes;
+    const int64_t kb = (k + 127) >> 7, nb = (n + 127) >> 7;  // floor divisions, negative values included
+    const int64_t rows[2] = {t.transpose ? nb : m, t.transpose ? m : nb};
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      int32_t* d = side ? t.layout_sfb + e * t.ld_sfb : t.layout_sfa + e * t.ld_sfa;
+      d[0] = (int32_t)rows[side];
+      d[1] = d[3] = (int32_t)kb;
+      d[2] = 1;
+      d[4] = (int32_t)(rows[side] * kb);
+    }
+  }
+}
+
 // Grouped (MoE) form: workgroup b takes logical tile pid of the concatenation of every
 // expert's tiles (row tiles first within a column tile). Workgroup b runs on XCD b % 8;
 // pid maps the 16 logical tiles 16 x .. 16 x + 15 to workgroups 8 apart (one XCD,
@@ -456,6 +486,10 @@ __device__ inline int64_t expert256_tiles(const Expert256& p) { return cdiv(p.m,
 __global__ __launch_bounds__(kThreads, 1) void fp8_grouped_block256_kernel(Grouped256Args ga) {
   __shared__ __attribute__((aligned(1024))) uint8_t P0[kPairBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t P1[kPairBytes];
+  // The tables cost no launch of their own: the last workgroup of the upper-bound grid,
+  // which seldom has a tile, fills them (about 30 tensor operations took 100 us of a 64-token
+  // call's 1315 us, and most of a small call's 266 us).
+  if (ga.tables.a_ptrs != nullptr && blockIdx.x == gridDim.x - 1) fill_tables(ga);
   const int lane = threadIdx.x & 63;
   const int E = ga.num_experts, per = (E + 63) / 64;
   const int64_t b = blockIdx.x;

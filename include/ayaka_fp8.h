@@ -186,6 +186,16 @@ int ayk_fp8_grouped_blockwise_mm(const void* a, const void* b, const float* scal
                                  const int32_t* problem_sizes, const int32_t* expert_offsets, int64_t num_experts,
                                  int64_t m_total, int64_t n, int64_t k, void* out, int out_dtype,
                                  ayk_stream_t stream);
+/* The same launch, which also fills the reference's per-expert pointer tables and scale
+ * descriptors (get_group_gemm_starts, moe_grouped_gemm.py:61-135): int64 addresses
+ * [num_experts] each, int32 descriptors [num_experts][>= 5] at row strides ld_sfa / ld_sfb;
+ * `transpose` for the swapped operand roles. a_ptrs NULL: no tables. */
+int ayk_fp8_grouped_blockwise_mm_tables(const void* a, const void* b, const float* scales_a, const float* scales_a_t,
+                                        const float* scales_b, const int32_t* problem_sizes, const int32_t* expert_offsets,
+                                        int64_t num_experts, int64_t m_total, int64_t n, int64_t k, void* out, int out_dtype,
+                                        int64_t* a_ptrs, int64_t* b_ptrs, int64_t* out_ptrs, int64_t* a_scales_ptrs,
+                                        int64_t* b_scales_ptrs, int32_t* layout_sfa, int64_t ld_sfa, int32_t* layout_sfb,
+                                        int64_t ld_sfb, int transpose, ayk_stream_t stream);
 
 /* Replaces ayaka::mxfp8_scaled_mm (gemm/fp8_mxfp8_gemm.py:163; oracle reference/gemm.py:73-92).
  * out = sum_g (a[:, g] @ w[:, g]^T) * 2^(a_scale[m,g]-127) * 2^(w_scale[n,g]-127) + bias

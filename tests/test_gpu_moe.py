@@ -229,3 +229,36 @@ def test_grouped_mm_random_experts(gpu, case):
     assert torch.equal(got[~owned], sentinel[~owned]), "rows of no expert were written"
     if owned.any():
         assert_linear_close(got[owned], ref[owned], f"random case {case}")
+
+
+@pytest.mark.parametrize("swap_ab", [False, True])
+@pytest.mark.parametrize("experts,columns", [(1, 5), (513, 7), (1200, 5)])
+def test_pointer_tables_match_tensor_arithmetic(gpu, swap_ab, experts, columns):
+    """The tables that the kernel fills (more experts than a workgroup has threads, wide
+    descriptor rows, experts past the end and short ones) equal ``get_group_gemm_starts``."""
+    from ayaka.kernel.hip import fp8_blockwise_scaled_grouped_mm
+    from ayaka.kernel.hip.moe import get_group_gemm_starts
+
+    n, k, rows = 128, 256, 300
+    _say(f"grouped mm tables experts={experts} columns={columns} swap_ab={swap_ab}")
+    g = torch.Generator().manual_seed(experts)
+    a = torch.zeros(rows, k, dtype=torch.float8_e4m3fn, device=gpu)
+    b = torch.zeros(experts, n, k, dtype=torch.float8_e4m3fn, device=gpu)
+    sa, sb = torch.ones(rows, k // 128, device=gpu), torch.ones(experts, 1, k // 128, device=gpu)
+    ps = torch.stack([torch.randint(0, 3, (experts,), generator=g), torch.randint(0, n + 1, (experts,), generator=g),
+                      torch.randint(0, k + 1, (experts,), generator=g)], 1).to(torch.int32).to(gpu)
+    off = torch.randint(0, rows, (experts,), generator=g).to(torch.int32).to(gpu)
+    out = torch.zeros(rows, n, dtype=torch.bfloat16, device=gpu)
+
+    def tables():
+        return ([torch.full((experts,), -1, dtype=torch.int64, device=gpu) for _ in range(5)],
+                [torch.full((experts, columns), -7, dtype=torch.int32, device=gpu) for _ in range(2)])
+
+    got, want = tables(), tables()
+    stride = [torch.full((experts,), v, dtype=torch.int64, device=gpu) for v in (k, k, n)]
+    fp8_blockwise_scaled_grouped_mm(out, *got[0], a, b, sa, sb, *stride, *got[1], ps, off,
+                                    torch.empty(1, dtype=torch.uint8, device=gpu), swap_ab=swap_ab)
+    operands = (b, a, out, sb, sa) if swap_ab else (a, b, out, sa, sb)
+    get_group_gemm_starts(off, *want[0], *operands, *want[1], ps, torch.empty_like(ps), swap_ab)
+    for x, y in zip(got[0] + got[1], want[0] + want[1]):
+        assert torch.equal(x, y)
