@@ -29,6 +29,10 @@ def require_fp8_dtype() -> torch.dtype:
 
 def validate_operand(tensor: torch.Tensor, name: str, *, dtype: torch.dtype, allow_transposed: bool) -> None:
     """2-D operand of ``dtype``, row-major (or column-major when ``allow_transposed``)."""
+    if isinstance(tensor, torch.Tensor) and tensor.dtype is dtype and tensor.is_cuda and tensor.ndim == 2:
+        strides = tensor.stride()
+        if strides[1] == 1 or (allow_transposed and strides[0] == 1):
+            return
     require_tensor(tensor, name)
     require_dtype(tensor, name, (dtype,))
     require_cuda(tensor, name)

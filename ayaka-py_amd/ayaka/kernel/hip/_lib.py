@@ -136,9 +136,27 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# The raw handle without the Stream object that torch.cuda.current_stream builds around it:
+# 0.2 us against 2.0 us, of the 8-14 us an operator's Python side takes.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
     """Handle of the current torch stream on ``t``'s device."""
+    if _raw_stream is not None:
+        return _raw_stream(t.device.index)
     return torch.cuda.current_stream(t.device).cuda_stream
+
+
+# Entry points by name, bound on first use (load_library takes a lock on every call).
+_entries: dict[str, Any] = {}
+
+
+def _entry(name: str) -> Any:
+    fn = _entries.get(name)
+    if fn is None:
+        fn = _entries[name] = getattr(load_library(), name)
+    return fn
 
 
 def call(name: str, *args: Any) -> None:
@@ -147,10 +165,10 @@ def call(name: str, *args: Any) -> None:
     ``AYK_EARCH`` becomes :class:`CapabilityError`; ``AYK_EINVAL`` becomes
     ``ValueError``; every other failure ``RuntimeError``.
     """
-    lib = load_library()
-    status = getattr(lib, name)(*args)
+    status = _entry(name)(*args)
     if status == AYK_OK:
         return
+    lib = load_library()
     message = (lib.ayk_last_error() or b"").decode("utf-8", "replace")
     if status == AYK_EARCH:
         raise CapabilityError(
@@ -170,4 +188,4 @@ def last_plan() -> str:
 
 def query(name: str, *args: Any) -> int:
     """Call a size-returning entry point."""
-    return int(getattr(load_library(), name)(*args))
+    return int(_entry(name)(*args))

@@ -60,6 +60,8 @@ def _source_rows(source: torch.Tensor, width: int) -> tuple[torch.Tensor, int]:
     """``source`` as rows of ``width`` contiguous elements and the row stride. Any
     alignment is accepted: the library takes 8-element vector kernels when rows are
     16-byte aligned, per-element kernels otherwise."""
+    if source.is_contiguous():
+        return source, width
     rows = source.reshape(source.shape[0], width)
     if rows.stride(-1) != 1 or (rows.shape[0] > 1 and rows.stride(0) < width):
         rows = rows.contiguous()
@@ -74,7 +76,7 @@ def _launch_write(key, value, key_cache, value_cache, slots, k_inverse, v_invers
         v_rows, v_stride = _source_rows(value, width)
         if v_stride != stride:
             k_rows, v_rows, stride = k_rows.contiguous(), v_rows.contiguous(), width
-    slots_c = slots.contiguous()
+    slots_c = slots if slots.is_contiguous() else slots.contiguous()
     _lib.call(
         "ayk_kv_cache_write", k_rows.data_ptr(), None if v_rows is None else v_rows.data_ptr(),
         _lib.dtype_code(key.dtype), int(slots_c.numel()), width, stride, key_cache.data_ptr(),
@@ -146,7 +148,7 @@ def gather_cache(source: torch.Tensor, slots: torch.Tensor, destination: torch.T
         raise ValueError("gather needs a contiguous cache and destination")
     if slots.numel() == 0:
         return
-    slots_c = slots.contiguous()
+    slots_c = slots if slots.is_contiguous() else slots.contiguous()
     _lib.call(
         "ayk_kv_cache_gather", source.data_ptr(), _lib.dtype_code(source.dtype), int(source.shape[0] * source.shape[1]),
         width, slots_c.data_ptr(), int(slots_c.numel()), destination.data_ptr(), _lib.dtype_code(destination.dtype),

@@ -48,7 +48,7 @@ _SCALE_TILE = 128
 _DECODE_BATCH_ROWS = 64
 
 
-@dataclass(frozen=True)
+@dataclass(slots=True)
 class _Activation:
     """A validated ``[..., K]`` activation viewed as a contiguous ``[M, K]`` matrix, and
     the ``[N, K]`` weight it is multiplied with."""
@@ -74,8 +74,9 @@ class _Activation:
         if x.ndim < 1:
             raise ValueError("x must have at least one dimension")
         k = int(x.shape[-1])
-        lead = tuple(int(d) for d in x.shape[:-1])
-        matrix = x.reshape(math.prod(lead), k)  # prod(()) == 1: a [K] input is one row
+        lead = tuple(x.shape[:-1])
+        # prod(()) == 1: a [K] input is one row
+        matrix = x if x.ndim == 2 else x.reshape(math.prod(lead), k)
         if not matrix.is_contiguous():
             matrix = matrix.contiguous()
         validate_operand(weight, "weight", dtype=require_fp8_dtype(), allow_transposed=False)
@@ -92,7 +93,7 @@ class _Activation:
         """``result`` ([M, N] or [N]) back to ``[..., N]``, adding a not-yet-applied bias."""
         if bias_after is not None:
             result = result + bias_after
-        return result.reshape(*self.lead, self.columns)
+        return result if len(self.lead) == 1 and result.ndim == 2 else result.reshape(*self.lead, self.columns)
 
     def weight_only(self, weight: torch.Tensor, scale: torch.Tensor, scale_rows: int, scale_cols: int,
                     scale_dtype: str) -> torch.Tensor:

@@ -47,7 +47,7 @@ def _validate_input(x: torch.Tensor, name: str) -> None:
 
 def _rows_2d(x: torch.Tensor) -> torch.Tensor:
     k = int(x.shape[-1])
-    x2d = x.reshape(-1, k)
+    x2d = x if x.ndim == 2 and k > 0 else x.reshape(-1, k)
     if x2d.stride(-1) != 1 or (x2d.shape[0] > 1 and x2d.stride(0) < k):
         x2d = x2d.contiguous()
     return x2d
