@@ -1967,11 +1967,15 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
     if (big_ok && !mid_beats(0.9f * block128_time(g.M, g.N, g.K))) return launch_block_big(g, st, op);
   }
   // Decode batches (M <= 64) with fp32 or UE8M0 scales: the weight-streaming kernel
-  // (gemm_skinny.hip) where its shape and alignment rules hold.
+  // (gemm_skinny.hip) where its shape and alignment rules hold. Its plans leave some shapes
+  // on a few workgroups with a long K, or two rounds of them; the medium tiles split those
+  // (1664 x 17408, M = 32: per-row 25.1 -> 15.6 us, MXFP8 35.7 -> 17.1, block 30.1 -> 17.1;
+  // 5248 x 13824: 30.8 -> 21.0, 47.1 -> 24.0, 37.6 -> 21.8). Below these shares of its model
+  // none of the fitted launches got slower; the recipes gained 11%, 10% and 7% in the mean.
   if constexpr (MODE == MODE_SCALED || MODE == MODE_MX || MODE == MODE_BLOCK) {
     if (g.M <= 64 && (MODE == MODE_MX || (g.sa_dtype == AYK_F32 && g.sb_dtype == AYK_F32))) {
       const SkinnyFp8Args sk = skinny_args(g, MODE == MODE_MX ? 1 : (MODE == MODE_BLOCK ? 2 : 0));
-      if (skinny_fp8_supported(sk)) return skinny_fp8_launch(sk, st, op);
+      if (skinny_fp8_supported(sk) && !mid_beats((MODE == MODE_SCALED ? 0.75f : (MODE == MODE_MX ? 0.63f : 0.7f)) * skinny_fp8_time(sk))) return skinny_fp8_launch(sk, st, op);
     }
   }
   if (mid_ok) return mid_launch(mid_mode(MODE), mid, st, op);

@@ -35,6 +35,8 @@ struct SkinnyFp8Args {
 
 // Whether the kernel takes this problem (shape, alignment and scale-layout rules).
 bool skinny_fp8_supported(const SkinnyFp8Args& g);
+// Its modelled time in microseconds, for a problem it takes (0: do not compare).
+float skinny_fp8_time(const SkinnyFp8Args& g);
 // Bytes of K-split partials a launch of this shape needs (0: none); shape only.
 size_t skinny_fp8_workspace(int64_t M, int64_t N, int64_t K, int mode);
 // Launch (the kernel and, with a K split, the fixed-order reduce). Returns an ayk_status.

@@ -809,6 +809,28 @@ bool skinny_fp8_supported(const SkinnyFp8Args& g) {
   return out_ok;
 }
 
+// Modelled time (microseconds) of this kernel on its plan: a launch, rounds of resident
+// workgroups that each walk their K at `step` per 128 (one or two 32-row activation tiles),
+// no faster than the weights stream, and a split's reduce. Fitted on 36 weight shapes from
+// 1280 x 8320 to 38400 x 3584 and batches of 2 to 64 (mean error 7-10%). 0: the GEMV-shaped
+// kernel takes the launch.
+float skinny_fp8_time(const SkinnyFp8Args& g) {
+  if (rows_gemv_wanted(g)) return 0.0f;
+  const SkPlan p = skinny_plan(g.M, g.N, g.K, g.mode);
+  struct Model {
+    float base, step[2], bytes_us, reduce, partial;
+  };
+  constexpr Model kModel[3] = {{6.9f, {0.40f, 0.61f}, 5.2e6f, 1.9f, 2.7e-6f},
+                               {5.0f, {0.56f, 0.81f}, 4.5e6f, 5.5f, 4.0e-6f},
+                               {5.5f, {0.41f, 0.79f}, 4.9e6f, 4.0f, 0.0f}};  // by mode: rows, MX, block
+  const Model& m = kModel[g.mode];
+  const int64_t wgs = cdiv(g.N, 32 * p.fn * (kWaves / p.ks)) * p.split;
+  const int resident = skinny_lds(p.fn, p.fm, p.ks, p.g, g.mode) <= 80 * 1024 ? 2 : 1;
+  const float walk = (float)cdiv(wgs, 256 * resident) * (float)(p.kps / p.ks) / 128.0f * m.step[p.fm - 1] * (p.fn == 2 ? 1.35f : 1.0f);
+  const float stream = (float)g.N * (float)g.K / m.bytes_us;
+  return m.base + (walk > stream ? walk : stream) + (p.split > 1 ? m.reduce + m.partial * (float)p.split * (float)g.M * (float)g.N : 0.0f);
+}
+
 size_t skinny_fp8_workspace(int64_t M, int64_t N, int64_t K, int mode) {
   const SkPlan p = skinny_plan(M, N, K, mode);
   return p.ok && p.split > 1 ? (size_t)p.split * (size_t)M * (size_t)N * sizeof(float) : 0;

@@ -493,6 +493,7 @@ void launch_skinny_kernel(const SkinnyPlan& p, const SkinnyArgs& a, hipStream_t 
 
 template <bool BF16>
 int launch_skinny(const SkinnyPlan& p, SkinnyArgs a, size_t ws_bytes, hipStream_t st) {
+  note_plan("w8a16 skinny split=%d", p.split);
   a.k_per_split = p.kps;
   a.x_pitch = p.x_pitch;
   a.s_cols = p.s_cols;
@@ -896,6 +897,22 @@ RsPlan rows_plan(int64_t M, int64_t N, int64_t K, int64_t bx) {
   p.split = (int)split;
   p.ok = cdiv(N, 16 * p.rt) <= 0x7FFFFFFF;
   return p;
+}
+// Modelled times (microseconds) of the row-stream and the stream kernel on their plans: a
+// launch, rounds of resident workgroups that each walk their 256-K stages, no faster than
+// the weights stream, and a split's reduce. Fitted on 36 weight shapes from 1280 x 8320 to
+// 38400 x 3584 and batches of 2 to 32 (mean error 4% and 11%). A launch goes to the tiled
+// kernel (w8a16_tile.hip) where its model is below 0.75 of these: plans that leave a long K
+// to few workgroups, or a second round nearly empty (1280 x 17664, M = 32: 35.0 -> 17.6 us;
+// 5248 x 13824, M = 16: 32.8 -> 22.7; 8320 x 7680, M = 32: 33.7 -> 23.4). None of the fitted
+// launches got slower.
+float rows_time(const RsPlan& p, int64_t N, int64_t K) {
+  const int64_t lds = 4 * (16 * p.rt * kRsStageK + 8 * p.xj * 2 * kRsStageK) + 1024;
+  const int64_t fit = 160 * 1024 / lds, resident = fit < 1 ? 1 : (fit > 4 ? 4 : fit);
+  const float stage = (0.177f + 0.029f * (float)p.xj) * (p.rt == 1 ? 1.0f : (p.rt == 2 ? 1.69f : 2.86f));
+  const float walk = (float)cdiv(cdiv(N, 16 * p.rt) * p.split, 256 * resident) * (float)(p.kps / kRsStageK) * stage;
+  const float stream = (float)N * (float)K / 5.4e6f;
+  return 4.0f + (walk > stream ? walk : stream) + (p.split > 1 ? 3.7f : 0.0f);
 }
 size_t rows_workspace(const RsPlan& p, int64_t M, int64_t N) {
   return p.ok && p.split > 1 ? (size_t)p.split * (size_t)M * (size_t)N * sizeof(float) : 0;
@@ -1323,6 +1340,13 @@ StPlan stream_plan(int64_t M, int64_t N, int64_t K, int64_t bx) {
   p.ok = cdiv(N, 16 * p.tw * (kStWaves / p.ks)) <= 0x7FFFFFFF;
   return p;
 }
+float stream_time(const StPlan& p, int64_t N, int64_t K) {  // see rows_time
+  const int64_t wgs = cdiv(N, 16 * p.tw * (kStWaves / p.ks)) * p.split, resident = p.tw == 1 ? 2 : 1;
+  const float stage = (0.24f + 0.0095f * (float)p.mp) * (p.tw == 1 ? 1.36f : 1.17f);
+  const float walk = (float)cdiv(wgs, 256 * resident) * (float)(p.kps / p.ks / kStK) * stage;
+  const float stream = (float)N * (float)K / 4.24e6f;
+  return 4.2f + (walk > stream ? walk : stream) + (p.split > 1 ? 2.9f : 0.0f);
+}
 size_t stream_workspace(const StPlan& p, int64_t M, int64_t N) {
   return p.ok && p.split > 1 ? (size_t)p.split * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
@@ -1456,9 +1480,13 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
   // projections take the stream kernel (K a multiple of 512, scale blocks of whole
   // 16 K), the others the row-stream kernel (whole 256-K stages, scale blocks of whole
   // 16 K), else the skinny streaming kernel (whole 128-K steps, scale blocks of >= 32 K).
+  const W16TileArgs t{g.x, ldx, g.w, ldw, M, N, K, scale, scale_dtype, scale_row_stride, block_size_y, block_size_x,
+                      out, ldo, static_cast<float*>(workspace), workspace_bytes};
+  const bool tile_ok = w16_tile_supported(t);
+  auto tile_beats = [&](float us) { return tile_ok && w16_tile_time(M, N, K) < 0.75f * us; };
   if (M >= 2 && ldx % 8 == 0) {
     const StPlan sp = stream_plan(M, N, K, block_size_x);
-    if (sp.ok) {
+    if (sp.ok && !tile_beats(stream_time(sp, N, K))) {
       RsArgs a{};
       a.x = g.x; a.ldx = ldx; a.M = M; a.w = g.w; a.ldw = ldw; a.N = N; a.K = K;
       a.scale = scale; a.scale_dtype = scale_dtype; a.srs = scale_row_stride; a.by = block_size_y; a.bx = block_size_x;
@@ -1469,7 +1497,7 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
   }
   if (M >= 2 && ldx % 8 == 0) {
     const RsPlan rp = rows_plan(M, N, K, block_size_x);
-    if (rp.ok) {
+    if (rp.ok && !tile_beats(rows_time(rp, N, K))) {
       RsArgs a{};
       a.x = g.x; a.ldx = ldx; a.M = M; a.w = g.w; a.ldw = ldw; a.N = N; a.K = K;
       a.scale = scale; a.scale_dtype = scale_dtype; a.srs = scale_row_stride; a.by = block_size_y; a.bx = block_size_x;
@@ -1480,7 +1508,10 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
   }
   if (M >= 2 && ldx % 8 == 0) {
     const SkinnyPlan p = skinny_plan(M, N, K, block_size_x);
-    if (p.ok) {
+    // From 17 rows the tiled kernel is faster on weights past 9 MB (M = 32: 2432 x 3968 14.0
+    // -> 13.0 us, 3840 x 3200 15.8 -> 12.8, 6656 x 18560 48.2 -> 34.3; 1920 x 3200 11.8 against
+    // 12.0); up to 16 rows this one is (M = 16: 6656 x 18560 28.7 against 30.7).
+    if (p.ok && !(tile_ok && M > 16 && N * K > 9000000)) {
       SkinnyArgs a{};
       a.x = g.x; a.ldx = ldx; a.M = M; a.w = g.w; a.ldw = ldw; a.N = N; a.K = K;
       a.scale = scale; a.scale_dtype = scale_dtype; a.srs = scale_row_stride; a.by = block_size_y; a.bx = block_size_x;
@@ -1490,9 +1521,7 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
     }
   }
   // Everything else: the tiled kernel, but for scale blocks that split its 64-K stages.
-  const W16TileArgs t{g.x, ldx, g.w, ldw, M, N, K, scale, scale_dtype, scale_row_stride, block_size_y, block_size_x,
-                      out, ldo, static_cast<float*>(workspace), workspace_bytes};
-  if (w16_tile_supported(t)) return w16_tile_launch(t, x_dtype == AYK_BF16, st, op);
+  if (tile_ok) return w16_tile_launch(t, x_dtype == AYK_BF16, st, op);
   return x_dtype == AYK_BF16 ? dispatch_w16<true>(g, st) : dispatch_w16<false>(g, st);
 }
 

@@ -27,6 +27,8 @@ struct W16TileArgs {
 
 // Workspace bytes of the launch below (0: no K split); a function of the shape only.
 size_t w16_tile_workspace(int64_t M, int64_t N, int64_t K);
+// Its modelled time in microseconds.
+float w16_tile_time(int64_t M, int64_t N, int64_t K);
 // Whether the tiled kernel takes this problem.
 bool w16_tile_supported(const W16TileArgs& a);
 int w16_tile_launch(const W16TileArgs& a, bool bf16, hipStream_t st, const char* op);

@@ -265,6 +265,7 @@ __global__ __launch_bounds__(256) void w8a16_tile_reduce(const float* __restrict
 // fastest tile and split on average, 15% at worst.
 struct TilePlan {
   int config, split;
+  float us;
 };
 struct TileConfig {
   int bn, bm, resident;
@@ -280,8 +281,7 @@ int64_t stages(int64_t K) { return cdiv(K, kStepK); }
 int64_t split_kps(int64_t K, int split) { return cdiv(stages(K), split) * kStepK; }
 
 TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
-  TilePlan best{0, 1};
-  float best_us = 0.0f;
+  TilePlan best{0, 1, 0.0f};
   bool first = true;
   for (int c = 0; c < 4; ++c) {
     const TileConfig& t = kConfigs[c];
@@ -292,10 +292,9 @@ TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
       const float stage = rounds * t.lambda > u * t.tau ? rounds * t.lambda : u * t.tau;
       float us = (float)cdiv(stages(K), s) * stage + 1.5f * u * (float)(t.bn * t.bm) / 65536.0f;
       if (s > 1) us += 5.0f + 1.6e-6f * (float)s * (float)M * (float)N;
-      if (first || us < best_us) {
+      if (first || us < best.us) {
         first = false;
-        best_us = us;
-        best = {c, s};
+        best = {c, s, us};
       }
     }
   }
@@ -323,6 +322,12 @@ void launch_config(const W16TileArgs& a, const TilePlan& p, hipStream_t st) {
 }  // namespace
 
 size_t w16_tile_workspace(int64_t M, int64_t N, int64_t K) { return split_bytes(tile_plan(M, N, K, true), M, N); }
+
+// The weights stream at no more than 4.4 TB/s beside a launch and its prologue.
+float w16_tile_time(int64_t M, int64_t N, int64_t K) {
+  const float us = tile_plan(M, N, K, true).us, stream = 6.0f + (float)N * (float)K / 4.4e6f;
+  return us > stream ? us : stream;
+}
 
 bool w16_tile_supported(const W16TileArgs& a) {
   // 32-bit offsets within a tile's rows; whole stages of one scale block.
