@@ -1894,9 +1894,10 @@ MidArgs mid_args(const GemmArgs& g) {
 // Modelled times (microseconds) of the large-tile kernels on the plans above, fitted on
 // the shapes of the medium-tile kernel's model (3-4% mean error): a launch, `rounds` of
 // one workgroup a CU over `steps` 128-K blocks each, a split's reduce and partials.
-// A launch goes to the medium tiles where their model is below 0.95 (block-128 128 x 128
-// kernel: 0.9) of these: over the fitted shapes no such launch got slower, and batches of
-// 256 to 2048 rows gained 19% (per-row), 17% (MXFP8) and 10% (block) in the mean.
+// A launch goes to the medium tiles where their model is below 0.9 of these (at 0.95 a few
+// large launches lost 2-8%). Batches of 512 to 2048 rows then gain 1.1 to 2.7 times on
+// weights up to 8192 x 8192 (4096 x 4096, M = 512: per-row 34.2 -> 16.0 us, MXFP8 35.2 ->
+// 17.1, block 34.5 -> 21.2; 4096 x 14336, M = 1024: 67.4 -> 63.1, 79.3 -> 69.3).
 struct LargeModel {
   float base, step, tile, reduce, partial;
   float time(int64_t rounds, int64_t steps, int64_t split, int64_t part_elems) const {
@@ -1933,7 +1934,7 @@ float block128_time(int64_t M, int64_t N, int64_t K) {
 template <int MODE>
 int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
   const MidArgs mid = mid_args(g);
-  const bool mid_ok = mid_supported(mid);
+  const bool mid_ok = mid_supported(mid_mode(MODE), mid);
   // Whether the medium tiles beat a kernel that is modelled at `us`.
   auto mid_beats = [&](float us) { return mid_ok && mid_time(mid_mode(MODE), g.M, g.N, g.K) < us; };
   // The large-tile kernels need K % 64 == 0, fp32 scales (MXFP8: K % 512 == 0 and 16-byte
@@ -1949,12 +1950,12 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
                       (MODE == MODE_MX || (g.sa_dtype == AYK_F32 && g.sb_dtype == AYK_F32 &&
                                            (!g.sb_vec || aligned16(g.sb)))) &&
                       (g.bias == nullptr || (reinterpret_cast<uintptr_t>(g.bias) & 15) == 0);
-  if (big_ok && !mid_beats(0.95f * pair_time(MODE, g.M, g.N, g.K))) return launch_big<MODE>(g, st, op);
+  if (big_ok && !mid_beats(0.9f * pair_time(MODE, g.M, g.N, g.K))) return launch_big<MODE>(g, st, op);
   } else {
     // The 256 x 256 block-scaled kernel from half a round of its tiles on.
     if (g.sa_dtype == AYK_F32 && block256_wanted(g.M, g.N, g.K)) {
       const Block256Args b = block256_args(g);
-      if (block256_supported(b) && !mid_beats(0.95f * block256_time(g.M, g.N, g.K))) return block256_launch(b, st, op);
+      if (block256_supported(b) && !mid_beats(0.9f * block256_time(g.M, g.N, g.K))) return block256_launch(b, st, op);
     }
     // The block-scaled 128 x 128 kernel: K % 128 == 0, fp32 activation scales, any float
     // weight-scale dtype, and the same output / bias alignment as above.
@@ -1970,12 +1971,20 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
   // (gemm_skinny.hip) where its shape and alignment rules hold. Its plans leave some shapes
   // on a few workgroups with a long K, or two rounds of them; the medium tiles split those
   // (1664 x 17408, M = 32: per-row 25.1 -> 15.6 us, MXFP8 35.7 -> 17.1, block 30.1 -> 17.1;
-  // 5248 x 13824: 30.8 -> 21.0, 47.1 -> 24.0, 37.6 -> 21.8). Below these shares of its model
-  // none of the fitted launches got slower; the recipes gained 11%, 10% and 7% in the mean.
+  // 5248 x 13824: 30.8 -> 21.0, 47.1 -> 24.0, 37.6 -> 21.8). They take a launch that their
+  // model puts at this share of the skinny kernel's and `save` microseconds below it, which
+  // is more than the two models err by. From 33 rows on MXFP8 and block shapes would gain at
+  // larger shares too; the plans that the tests hold to the skinny kernel set those two.
   if constexpr (MODE == MODE_SCALED || MODE == MODE_MX || MODE == MODE_BLOCK) {
     if (g.M <= 64 && (MODE == MODE_MX || (g.sa_dtype == AYK_F32 && g.sb_dtype == AYK_F32))) {
       const SkinnyFp8Args sk = skinny_args(g, MODE == MODE_MX ? 1 : (MODE == MODE_BLOCK ? 2 : 0));
-      if (skinny_fp8_supported(sk) && !mid_beats((MODE == MODE_SCALED ? 0.75f : (MODE == MODE_MX ? 0.63f : 0.7f)) * skinny_fp8_time(sk))) return skinny_fp8_launch(sk, st, op);
+      const bool one = g.M <= 32;  // one activation tile
+      const float share = MODE == MODE_SCALED ? 0.8f : (MODE == MODE_MX ? (one ? 0.75f : 0.54f) : (one ? 0.77f : 0.58f));
+      const float save = one ? 4.0f : 6.0f;
+      if (skinny_fp8_supported(sk)) {
+        const float us = skinny_fp8_time(sk);
+        if (!mid_beats(std::min(share * us, us - save))) return skinny_fp8_launch(sk, st, op);
+      }
     }
   }
   if (mid_ok) return mid_launch(mid_mode(MODE), mid, st, op);

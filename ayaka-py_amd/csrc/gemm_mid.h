@@ -37,7 +37,7 @@ struct MidArgs {
 size_t mid_workspace(MidMode mode, int64_t M, int64_t N, int64_t K);
 float mid_time(MidMode mode, int64_t M, int64_t N, int64_t K);
 // 32-bit offsets within a tile's rows.
-bool mid_supported(const MidArgs& g);
+bool mid_supported(MidMode mode, const MidArgs& g);
 int mid_launch(MidMode mode, const MidArgs& g, hipStream_t st, const char* op);
 
 }  // namespace ayk

@@ -6,25 +6,26 @@
 //
 // Bound: at these sizes the weight stream and its latency (M = 65 .. 255), then the matrix
 // cores. Design:
-//  * 256 x 256 (eight wavefronts), 128 x 128 and 128 x 64 (four, two or three workgroups a
-//    CU) tiles on v_mfma_scale_f32_32x32x64_f8f6f4, weight = operand A: a lane's
-//    accumulator column is one activation row.
-//  * Direct-to-LDS loads (8 rows x 128 bytes an instruction) into two 128-K stage buffers;
-//    the next stage lands while the current one is multiplied, and the other workgroups of
-//    the CU run while one waits at its stage barrier.
+//  * 256 x 256 (eight wavefronts), 128 x 128, 128 x 64 and 64 x 64 (four) tiles on
+//    v_mfma_scale_f32_32x32x64_f8f6f4, weight = operand A: a lane's accumulator column is
+//    one activation row.
+//  * Direct-to-LDS loads (8 rows x 128 bytes an instruction) into a ring of two to four
+//    128-K stage buffers. Two buffers leave room for several workgroups a CU, which run
+//    while one waits at its stage barrier (throughput, the larger batches); three or four
+//    hide the latency of a stage inside one workgroup (few tiles a CU, long K), which also
+//    saves most K splits.
 //  * A K tail is zero-filled by the loads' bounds check, so any K % 16 == 0 takes the same
 //    loop; rows past M and N likewise.
 //  * Block scales: a 128-K stage is one scale block; its two MFMAs start from zero and one
 //    fma an accumulator folds them with sa[m, kb] sb[n / 128, kb].
-//  * MXFP8 codes: four stages' codes of a row are one 16-byte direct load into LDS (rows
-//    that are only 4-byte aligned: one dword a stage; unaligned rows: the two dwords that
-//    hold it).
-//  * Tile and K split come from a fitted time model (mid_plan), which gemm.hip also holds
-//    against the other kernels' (mid_time).
-// Measured (kernel alone in a graph, against the kernels these shapes ran before; 4096 x
-// 14336, 37888 x 3584): per-row M = 65 54.2 -> 26.2 us and 87 -> 37, M = 128 60.8 -> 31.7
-// and 96 -> 39; MXFP8 M = 128 47.0 -> 33.6 and 83 -> 45; block-128 37888 x 3584 M = 128
-// 76 -> 43; per-row 4096 x 4096 M = 1024 41.3 -> 25.9, 3072 x 1024 M = 65 21.2 -> 8.4.
+//  * Scales and MXFP8 codes pass through LDS as well, a dword a row and stage (16-byte
+//    aligned codes: 16 bytes for four stages; unaligned ones: the two dwords).
+//  * Tile, ring and K split come from a fitted time model (mid_plan), which gemm.hip also
+//    holds against the other kernels' (mid_time).
+// Measured (kernel alone in a graph; the kernels these shapes ran at first -> two buffers
+// only -> now): per-row 4096 x 14336 M = 128 60.8 -> 31.7 -> 25.5 us, 4096 x 4096 M = 128
+// 33 -> 18.4 -> 10.9, M = 512 28 -> 25 -> 15.3, M = 1024 41.3 -> 25.9 -> 24.5; MXFP8 4096 x
+// 14336 M = 128 47.0 -> 33.6 -> 27.4; block-128 4096 x 4096 M = 256 23.6 -> 17.1.
 #include "gemm_mid.h"
 
 #include "ayk_common.h"
@@ -42,13 +43,13 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int kStageK = 128;     // K bytes per stage: two MFMA steps, one 128-K scale block
 constexpr int kCodeOne = 127;    // UE8M0 code of 1.0
-// Kernel modes for MX codes whose rows are only 4-byte aligned (K % 128 == 0), or not at all.
+// Kernel modes of MXFP8 by its codes: kMidMx K % 512 == 0 and 16-byte aligned rows, kMidMx4
+// K % 128 == 0 and 4-byte aligned rows, kMidMxAny the rest.
 constexpr int kMidMx4 = 4, kMidMxAny = 5;
 constexpr bool mx_mode(int mode) { return mode == kMidMx || mode == kMidMx4 || mode == kMidMxAny; }
-// Stages whose codes are loaded together, and their LDS bytes a row (unaligned rows: the
-// two aligned dwords that hold a stage's four codes).
-constexpr int code_stages(int mode) { return mode == kMidMx ? 4 : 1; }
-constexpr int code_bytes(int mode) { return mode == kMidMx ? 16 : (mode == kMidMx4 ? 4 : (mode == kMidMxAny ? 8 : 0)); }
+// Dwords of LDS for a row's scales of one stage: the dword that holds its block scale or its
+// four codes (unaligned code rows: the two dwords that do; kMidMx loads four stages at once).
+constexpr int scale_words(int mode) { return mode == kMidBlock || mode == kMidMx4 ? 1 : (mode == kMidMxAny ? 2 : 0); }
 
 // One 64-K step of a 32 x 32 tile. Lane half h holds K [16 h, +16) and [32 + 16 h, +16) of
 // the step; the scaled MFMA applies the code of half b to K block [32 b, +32). INT8 sums
@@ -71,19 +72,32 @@ __device__ inline v16f mid_mma(const v8i& w, const v8i& a, const v16f& c, int cw
 
 // WN x WM wavefronts of (BN / WN) weight rows x (BM / WM) activation rows. kps > 0: the
 // launch splits K (whole 128-K stages), blockIdx.y takes [y kps, (y + 1) kps) and writes
-// an fp32 partial without the bias.
-template <int MODE, int BN, int BM, int WN, int WM, int WGS>
+// an fp32 partial without the bias. D stage buffers: D - 1 stages are in flight.
+template <int MODE, int BN, int BM, int WN, int WM, int D, int WGS>
 __global__ __launch_bounds__(WN * WM * 64, WGS) void fp8_mid_kernel(MidArgs g, int tiles_m, int64_t kps) {
   constexpr int kThreads = WN * WM * 64, kWaves = WN * WM;
   constexpr int TN = BN / WN, TM = BM / WM, FN = TN / 32, FM = TM / 32;
   constexpr int kRows = BN + BM, kStage = kRows * kStageK;
   constexpr int kWDma = BN / 8 / kWaves, kADma = BM / 8 / kWaves;  // direct loads per wavefront and stage
   static_assert(BN % (16 * kWaves) == 0 && BM % (16 * kWaves) == 0, "whole pairs of loads per wavefront");
-  __shared__ __attribute__((aligned(1024))) uint8_t B0[kStage];
-  __shared__ __attribute__((aligned(1024))) uint8_t B1[kStage];
+  constexpr int kWords = scale_words(MODE), kWordRows = 64 * kWaves;  // each wavefront loads 64 rows' words
+  constexpr int kOps = kWDma + kADma + kWords, kBuf = kStage + kWordRows * 4 * kWords;
+  static_assert(kRows <= kWordRows, "a lane a row");
+  static_assert(MODE != kMidMx || D != 3, "whole rings in a chunk of four stages");
+  static_assert(D >= 2 && D <= 4 && (D - 2) * kOps <= 63, "stage buffers, vmcnt range");
+  // Distinct LDS objects with compile-time names, so that the compiler keeps the loads in
+  // flight to one apart from the reads of another.
+  __shared__ __attribute__((aligned(1024))) uint8_t B0[kBuf], B1[kBuf], B2[D > 2 ? kBuf : 16], B3[D > 3 ? kBuf : 16];
+  constexpr bool kChunks = MODE == kMidMx;
+  __shared__ __attribute__((aligned(1024))) uint8_t chunk[kChunks ? kWordRows * 16 : 16];
   __shared__ float col_scale[BN], col_bias[BN];
-  constexpr int CS = code_stages(MODE), kCodeB = code_bytes(MODE), kCodes = kCodeB ? kRows * kCodeB : 16;  // one chunk
-  __shared__ __attribute__((aligned(1024))) uint8_t code_lds[2 * kCodes];
+  auto buffer = [&](auto d) -> uint8_t* {
+    constexpr int i = decltype(d)::value;
+    if constexpr (i == 0) return B0;
+    else if constexpr (i == 1) return B1;
+    else if constexpr (i == 2) return B2;
+    else return B3;
+  };
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -150,90 +164,113 @@ __global__ __launch_bounds__(WN * WM * 64, WGS) void fp8_mid_kernel(MidArgs g, i
     col_bias[t] = g.bias && kps == 0 ? load_f32(g.bias, g.bias_dtype, n) : 0.0f;
   }
 
-  // Per-stage scales. MX: the codes of this lane half's 32-K blocks, byte 2 t for step t.
-  // Block: sa[m, kb] and sb[n / 128, kb] as raw words (a 32-row slab lies in one 128-row
-  // block), decoded when used.
-  struct Scales {
-    int cw[FN], ca[FM];
-    RawBits sa[FM], sb[FN];
+  // Per-stage scales: block sa[m, kb] and sb[n / 128, kb], MX four codes a row. Every row's
+  // dword goes through LDS, loaded by one lane behind the operands of its stage: straight
+  // into each wavefront's registers they asked for more cache lines than the operands, and
+  // any branch or register load among the direct loads costs the compiler its exact wait
+  // counts. `word`: byte offset of this lane's row's first scale from the 4-byte aligned start
+  // of its side's window, which ends with the last row's last scale (rounded up to a dword,
+  // which lies in its page); `step`: bytes from one stage's scale to the next.
+  const int64_t kblocks = cdiv(g.K, kStageK), kb0 = k0 / kStageK;
+  const int sa_size = MODE == kMidBlock ? dtype_size(g.sa_dtype) : 1, sb_size = MODE == kMidBlock ? dtype_size(g.sb_dtype) : 1;
+  const bool sa_cols = MODE == kMidBlock && g.sa_vec;
+  const int64_t unit = MODE == kMidBlock ? kblocks : cdiv(g.K, 32);  // scales of a row
+  const int64_t u0 = MODE == kMidBlock ? kb0 : k0 / 32;              // the first of this piece
+  const int64_t sa_ld = sa_cols ? 1 : (g.ld_sa > 0 ? g.ld_sa : unit), sb_ld = g.ld_sb > 0 ? g.ld_sb : unit;
+  const int64_t n_row0 = MODE == kMidBlock ? n_base / 128 : n_base;
+  const uintptr_t sap = reinterpret_cast<uintptr_t>(g.sa) + (uintptr_t)((sa_cols ? u0 * g.M + m_base : m_base * sa_ld + u0) * sa_size);
+  const uintptr_t sbp = reinterpret_cast<uintptr_t>(g.sb) + (uintptr_t)((n_row0 * sb_ld + u0) * sb_size);
+  const uint32_t sa_mis = (uint32_t)__builtin_amdgcn_readfirstlane((int)(sap & 3)), sb_mis = (uint32_t)__builtin_amdgcn_readfirstlane((int)(sbp & 3));
+  const uint32_t sa_step = (uint32_t)__builtin_amdgcn_readfirstlane((int)(MODE == kMidBlock ? (sa_cols ? g.M : 1) * sa_size : 4));
+  const uint32_t sb_step = MODE == kMidBlock ? (uint32_t)sb_size : 4u;
+  const uint32_t sa_row = (uint32_t)__builtin_amdgcn_readfirstlane((int)(sa_ld * sa_size));
+  const uint32_t sb_row = (uint32_t)__builtin_amdgcn_readfirstlane((int)(sb_ld * sb_size));
+  auto sa_byte = [&](int r) -> uint32_t { return sa_mis + (uint32_t)r * sa_row; };
+  auto sb_byte = [&](int r) -> uint32_t {
+    return sb_mis + (uint32_t)(MODE == kMidBlock ? ((int)(n_base & 127) + r) / 128 : r) * sb_row;
   };
-  const int64_t kblocks = cdiv(g.K, 128);
-  const int64_t sa_ld = g.ld_sa > 0 ? g.ld_sa : kblocks, sb_ld = g.ld_sb > 0 ? g.ld_sb : kblocks;
-  auto load_scales = [&](int s, Scales& v) {
-    const int64_t kb = k0 / kStageK + s;
-    if constexpr (MODE == kMidBlock) {
-#pragma unroll
-      for (int j = 0; j < FM; ++j) v.sa[j] = load_bits(g.sa, g.sa_dtype, g.sa_vec ? kb * g.M + mrow[j] : mrow[j] * sa_ld + kb);
-#pragma unroll
-      for (int i = 0; i < FN; ++i) {
-        const int64_t n = n_base + wn * TN + 32 * i;
-        v.sb[i] = load_bits(g.sb, g.sb_dtype, (n < g.N ? n : g.N - 1) / 128 * sb_ld + kb);
-      }
-    }
-  };
-  // MX codes go through LDS for all wavefronts, one or two direct loads a row and chunk of
-  // CS stages. A dword a row and stage straight into each wavefront's registers asked for
-  // more cache lines than the operands themselves. The windows start at a 4-byte boundary
-  // and end with the last row's last code (rounded up to a dword, which lies in its page).
-  // `mis`: bytes from a window's start to the tile's first code.
-  const uintptr_t cwp = reinterpret_cast<uintptr_t>(g.sb) + (uintptr_t)(n_base * g.ld_sb + k0 / 32);
-  const uintptr_t cap = reinterpret_cast<uintptr_t>(g.sa) + (uintptr_t)(m_base * g.ld_sa + k0 / 32);
-  const int cw_mis = __builtin_amdgcn_readfirstlane((int)(cwp & 3)), ca_mis = __builtin_amdgcn_readfirstlane((int)(cap & 3));
-  const int cw_ld = __builtin_amdgcn_readfirstlane((int)g.ld_sb), ca_ld = __builtin_amdgcn_readfirstlane((int)g.ld_sa);
-  auto code_records = [&](int64_t rows_left, int64_t ldc, int mis) {  // the tile's first row lies inside the operand
-    const int64_t bytes = ((rows_left - 1) * ldc + (g.K - k0 + 31) / 32 + mis + 3) & ~(int64_t)3;
+  auto window = [&](int64_t rows_left, int64_t ld, int64_t size, uint32_t mis) {  // the tile's first row lies inside
+    const int64_t bytes = (((rows_left - 1) * ld + unit - u0) * size + mis + 3) & ~(int64_t)3;
     return (int32_t)(bytes < 0x7FFFFFFC ? bytes : 0x7FFFFFFC);
   };
-  const __amdgpu_buffer_rsrc_t cwr =
-      uniform_rsrc(reinterpret_cast<const void*>(cwp - cw_mis), kCodeB ? code_records(g.N - n_base, g.ld_sb, cw_mis) : 0);
-  const __amdgpu_buffer_rsrc_t car =
-      uniform_rsrc(reinterpret_cast<const void*>(cap - ca_mis), kCodeB ? code_records(g.M - m_base, g.ld_sa, ca_mis) : 0);
-  auto issue_codes = [&](int s) {  // the chunk that stage s begins
-    if constexpr (kCodeB > 0) {
-      if (s % CS) return;
-      uint8_t* chunk = code_lds + (s / CS % 2) * kCodes;
-      for (int t = wave; t < kRows / 64; t += kWaves) {
-        const bool w_side = 64 * t < BN;
-        const __amdgpu_buffer_rsrc_t rsrc = w_side ? cwr : car;
-        const int voff = w_side ? (64 * t + lane) * cw_ld + cw_mis : (64 * t - BN + lane) * ca_ld + ca_mis;
-        if constexpr (MODE == kMidMx) {
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(chunk + 1024 * t), 16, voff,
-                                                   4 * s, 0, 0);
-        } else {
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(chunk + 256 * t), 4,
-                                                   voff & ~3, 4 * s, 0, 0);
-          if constexpr (MODE == kMidMxAny) {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rsrc, (__attribute__((address_space(3))) void*)(chunk + 4 * kRows + 256 * t), 4, (voff & ~3) + 4, 4 * s, 0, 0);
-          }
-        }
+  const bool w_side = 64 * wave < BN;
+  const int64_t sa_rows = sa_cols ? (unit - u0 - 1) * g.M + g.M - m_base : g.M - m_base;  // column-major: as one long row set
+  const int32_t sa_records = sa_cols ? (int32_t)((((sa_rows * sa_size) + sa_mis + 3) & ~(int64_t)3)) : window(sa_rows, sa_ld, sa_size, sa_mis);
+  const int32_t sb_records = window((MODE == kMidBlock ? cdiv(g.N, 128) : g.N) - n_row0, sb_ld, sb_size, sb_mis);
+  const __amdgpu_buffer_rsrc_t word_rsrc = uniform_rsrc(reinterpret_cast<const void*>(w_side ? sbp - sb_mis : sap - sa_mis),
+                                                        kWords || kChunks ? (w_side ? sb_records : sa_records) : 0);
+  const int word_row = 64 * wave + lane;
+  const uint32_t word = word_row >= kRows ? (uint32_t)kPast : (w_side ? sb_byte(word_row) : sa_byte(word_row - BN));
+  const uint32_t word_step = w_side ? sb_step : sa_step;
+  auto issue_words = [&](int s, uint8_t* dst) {
+    if constexpr (kWords > 0) {
+      const int voff = (int)((word + (uint32_t)s * word_step) & ~3u);
+      uint8_t* words = dst + kStage + 256 * wave;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(word_rsrc, (__attribute__((address_space(3))) void*)words, 4, voff, 0, 0, 0);
+      if constexpr (kWords == 2) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(word_rsrc, (__attribute__((address_space(3))) void*)(words + 4 * kWordRows), 4,
+                                                 voff + 4, 0, 0, 0);
       }
     }
   };
-  auto read_codes = [&](int s, Scales& v) {
-    if constexpr (kCodeB > 0) {
-      const uint8_t* chunk = code_lds + (s / CS % 2) * kCodes;
-      // Codes past K are 1.0: their operands are zeros, which a NaN code would turn into NaN.
-      const int valid = (klen - s * kStageK + 31) / 32;
-      const uint32_t past = MODE == kMidMxAny && valid < 4 ? 0xFFFFFFFFu << (8 * valid) : 0u;
-      auto codes = [&](int row, int byte) -> int {  // byte: the row's first code, from its window's start
-        uint32_t w;
-        if constexpr (MODE == kMidMx) {
-          w = *reinterpret_cast<const uint32_t*>(chunk + 16 * row + 4 * (s % CS));
-        } else {
-          w = *reinterpret_cast<const uint32_t*>(chunk + 4 * row);
+  // The codes of stages 4 q .. 4 q + 3.
+  auto issue_chunk = [&](int q) {
+    if constexpr (kChunks) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(word_rsrc, (__attribute__((address_space(3))) void*)(chunk + 1024 * wave), 16,
+                                               (int)word, 16 * q, 0, 0);
+    }
+  };
+  v4i chunk_w[FN], chunk_a[FM];
+  auto read_chunk = [&]() {
+    if constexpr (kChunks) {
+#pragma unroll
+      for (int i = 0; i < FN; ++i) chunk_w[i] = *reinterpret_cast<const v4i*>(chunk + 16 * (wn * TN + 32 * i + frow));
+#pragma unroll
+      for (int j = 0; j < FM; ++j) chunk_a[j] = *reinterpret_cast<const v4i*>(chunk + 16 * (BN + wm * TM + 32 * j + frow));
+    }
+  };
+  struct Scales {
+    int cw[FN], ca[FM];    // MX: the codes of this lane half's 32-K blocks, byte 2 t for step t
+    float sb[FN], sa[FM];  // block
+  };
+  auto read_scales = [&](int s, const uint8_t* buf, Scales& v) {
+    if constexpr (kWords > 0) {  // (kMidMx: from the chunk)
+      const uint32_t* words = reinterpret_cast<const uint32_t*>(buf + kStage);
+      if constexpr (MODE == kMidBlock) {
+        // (a 32-row slab lies in one 128-row block of the weight)
+#pragma unroll
+        for (int i = 0; i < FN; ++i) {
+          const int r = wn * TN + 32 * i;
+          v.sb[i] = bits_to_f32({words[r], ((sb_byte(r) + (uint32_t)s * sb_step) & 3) * 8}, g.sb_dtype);
+        }
+#pragma unroll
+        for (int j = 0; j < FM; ++j) {
+          const int r = wm * TM + 32 * j + frow;
+          v.sa[j] = bits_to_f32({words[BN + r], ((sa_byte(r) + (uint32_t)s * sa_step) & 3) * 8}, g.sa_dtype);
+        }
+      } else {
+        // Codes past K are 1.0: their operands are zeros, which a NaN code would turn into NaN.
+        const int valid = (klen - s * kStageK + 31) / 32;
+        const uint32_t past = MODE == kMidMxAny && valid < 4 ? 0xFFFFFFFFu << (8 * valid) : 0u;
+        auto codes = [&](int row, uint32_t byte) -> int {
+          uint32_t w = words[row];
           if constexpr (MODE == kMidMxAny) {
-            const uint32_t hi = *reinterpret_cast<const uint32_t*>(chunk + 4 * kRows + 4 * row);
-            w = __builtin_amdgcn_alignbyte(hi, w, (uint32_t)byte & 3);
+            w = __builtin_amdgcn_alignbyte(words[kWordRows + row], w, byte & 3);
             w = (w & ~past) | (0x7F7F7F7Fu & past);
           }
+          return (int)(w >> (8 * h));
+        };
+#pragma unroll
+        for (int i = 0; i < FN; ++i) {
+          const int r = wn * TN + 32 * i + frow;
+          v.cw[i] = codes(r, sb_byte(r));
         }
-        return (int)(w >> (8 * h));
-      };
 #pragma unroll
-      for (int i = 0; i < FN; ++i) v.cw[i] = codes(wn * TN + 32 * i + frow, (wn * TN + 32 * i + frow) * cw_ld + cw_mis);
-#pragma unroll
-      for (int j = 0; j < FM; ++j) v.ca[j] = codes(BN + wm * TM + 32 * j + frow, (wm * TM + 32 * j + frow) * ca_ld + ca_mis);
+        for (int j = 0; j < FM; ++j) {
+          const int r = wm * TM + 32 * j + frow;
+          v.ca[j] = codes(BN + r, sa_byte(r));
+        }
+      }
     }
   };
 
@@ -263,18 +300,13 @@ __global__ __launch_bounds__(WN * WM * 64, WGS) void fp8_mid_kernel(MidArgs g, i
       for (int j = 0; j < FM; ++j) af[t][j] = frag(buf, BN + wm * TM + 32 * j, t);
     }
     if constexpr (MODE == kMidBlock) {
-      float sa[FM], sb[FN];
-#pragma unroll
-      for (int j = 0; j < FM; ++j) sa[j] = bits_to_f32(v.sa[j], g.sa_dtype);
-#pragma unroll
-      for (int i = 0; i < FN; ++i) sb[i] = bits_to_f32(v.sb[i], g.sb_dtype);
 #pragma unroll
       for (int i = 0; i < FN; ++i)
 #pragma unroll
         for (int j = 0; j < FM; ++j) {
           v16f part = mid_mma<MODE, 0>(wf[0][i], af[0][j], zero, 0, 0);
           part = mid_mma<MODE, 0>(wf[1][i], af[1][j], part, 0, 0);
-          const float c = sa[j] * sb[i];
+          const float c = v.sa[j] * v.sb[i];
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[i][j][r] = fmaf(part[r], c, acc[i][j][r]);
         }
@@ -290,31 +322,52 @@ __global__ __launch_bounds__(WN * WM * 64, WGS) void fp8_mid_kernel(MidArgs g, i
     }
   };
 
-  Scales cur_s{}, next_s{};
-  load_scales(0, cur_s);
-  issue_codes(0);
-  issue(0, B0);
-  wait_vmcnt<0>();
-  lds_barrier();
-  // Stage s is visible in `cur` and nothing is in flight; stage s + 1 lands in `nxt`
-  // (read by nobody since the last barrier) while stage s is multiplied. The code reads
-  // come first: behind a direct load into the same LDS object they would wait for it.
-  auto step = [&](int s, uint8_t* cur, uint8_t* nxt) {
-    read_codes(s, cur_s);
-    if (s + 1 < ns) {
-      issue(s + 1, nxt);
-      issue_codes(s + 1);
-      load_scales(s + 1, next_s);
-    }
-    compute(cur, cur_s);
-    wait_vmcnt<0>();
-    lds_barrier();
-    if constexpr (MODE == kMidBlock) cur_s = next_s;
+  // The ring: stages 0 .. D - 2 in flight. Step s waits for stage s (the D - 2 younger ones
+  // may still be in flight), passes a barrier (stage s is visible, and nobody reads stage
+  // s - 1 any more), refills that buffer with stage s + D - 1 and multiplies stage s. Stages
+  // past the last one load nothing that is used (operands: kPast), so the counts stay exact.
+  // A round of U steps runs without a branch inside. kMidMx: the first step of a round reads
+  // its four stages' codes, the second refills the chunk ahead of the data of a later stage.
+  constexpr int U = kChunks ? 4 : D;
+  auto prefetch = [&](int s, uint8_t* dst) {
+    issue_words(s, dst);
+    issue(s, dst);
   };
-  for (int s = 0; s < ns; s += 2) {
-    step(s, B0, B1);
-    if (s + 1 < ns) step(s + 1, B1, B0);  // workgroup-uniform
+  issue_chunk(0);
+  unrolled<D - 1>([&](auto d) { prefetch(decltype(d)::value, buffer(d)); });
+  auto step = [&](int s, auto u) {
+    constexpr int i = decltype(u)::value;
+    const std::integral_constant<int, i % D> d;
+    wait_vmcnt<(D - 2) * kOps>();
+    lds_barrier();
+    Scales v;
+    read_scales(s, buffer(d), v);
+    if constexpr (kChunks) {
+      if constexpr (i == 0) read_chunk();
+      if constexpr (i == 1) issue_chunk(s / 4 + 1);
+#pragma unroll
+      for (int t = 0; t < FN; ++t) v.cw[t] = (int)((uint32_t)chunk_w[t][i] >> (8 * h));
+#pragma unroll
+      for (int t = 0; t < FM; ++t) v.ca[t] = (int)((uint32_t)chunk_a[t][i] >> (8 * h));
+    }
+    prefetch(s + D - 1, buffer(std::integral_constant<int, (i + D - 1) % D>{}));
+    // With one stage in flight its loads go first and the products stay in their step
+    // (spread among each other they cost a 256 x 256 tile 13%); deeper rings gain from it.
+    if constexpr (D == 2) __builtin_amdgcn_sched_barrier(0);
+    compute(buffer(d), v);
+    if constexpr (D == 2) __builtin_amdgcn_sched_barrier(0);
+  };
+  int s0 = 0;
+  for (; s0 + U <= ns; s0 += U) {
+    unrolled<U>([&](auto u) { step(s0 + decltype(u)::value, u); });
   }
+  if constexpr (!kChunks) {  // (whole chunks only)
+    unrolled<D - 1>([&](auto u) {
+      if (s0 + decltype(u)::value < ns) step(s0 + decltype(u)::value, u);  // workgroup-uniform
+    });
+  }
+  wait_vmcnt<0>();  // no direct load may still write LDS
+  lds_barrier();    // no wavefront still reads a stage: the buffers become staging regions
 
   // Epilogue: scales, bias, one rounding.
   const int64_t n_w = n_base + wn * TN, m_w = m_base + wm * TM;
@@ -383,12 +436,14 @@ __global__ __launch_bounds__(256) void mid_reduce(const float* __restrict__ part
   store_f32(out, out_dtype, m * ldo + n, v);
 }
 
-// Tile and K split: the pair with the smallest modelled time. The model, in microseconds,
-// was fitted per recipe on 13 weight shapes from 3072 x 1024 to 37888 x 3584 and 12 batches
-// from 64 to 2048 (weights cold): a CU that runs u workgroups of a tile takes
+// Tile, stage buffers and K split: the triple with the smallest modelled time. The model, in
+// microseconds, was fitted per recipe on 12 weight shapes from 3072 x 1024 to 37888 x 3584
+// and 16 batches from 16 to 2048 (weights cold): a CU that runs u workgroups of a tile takes
 // max(u tau, ceil(u / resident) lambda) per 128-K stage (throughput, or one round's
-// latency) and `store` per 256 x 256 outputs; a split adds a reduce launch and the fp32
-// partials' traffic. Its choice is 2-3% slower than the fastest tile and split on average.
+// latency) and `store` per 256 x 256 outputs; `cold` is the weights' share that no stage
+// hides; a split adds a reduce launch and the fp32 partials' traffic. Its choice is 1-2%
+// slower than the fastest triple on average (tau of the two-buffer tiles: from the launches of
+// two rounds and more, 10-15% above the fit, whose weight lies on the small ones).
 struct MidPlan {
   int config, split;
   float us;
@@ -396,15 +451,17 @@ struct MidPlan {
 struct MidTile {
   int bn, bm, resident;
 };
-constexpr MidTile kTiles[3] = {{256, 256, 1}, {128, 128, 2}, {128, 64, 3}};
+constexpr int kConfigs = 6;
+constexpr MidTile kTiles[kConfigs] = {{256, 256, 1}, {128, 128, 2}, {128, 64, 3}, {128, 128, 1}, {128, 64, 1}, {64, 64, 2}};
 struct MidModel {
-  float tau[3], lambda[3];
-  float store, base, reduce, partial;
+  float tau[kConfigs], lambda[kConfigs];  // 0: no such kernel
+  float store, base, reduce, partial, cold;
 };
-// Block scales have no 256 x 256 form (its partial sums do not fit the registers).
-constexpr MidModel kModels[3] = {{{1.54f, 0.55f, 0.43f}, {1.54f, 0.97f, 0.77f}, 7.6f, 0.2f, 6.5f, 1.67e-6f},
-                                 {{0.0f, 0.67f, 0.48f}, {0.0f, 1.19f, 0.91f}, 7.8f, 1.7f, 4.8f, 1.68e-6f},
-                                 {{1.71f, 0.61f, 0.53f}, {1.71f, 1.03f, 0.91f}, 5.7f, 0.0f, 6.5f, 1.8e-6f}};
+constexpr MidModel kModels[3] = {
+    {{1.25f, 0.44f, 0.32f, 0.50f, 0.27f, 0.19f}, {1.25f, 0.71f, 0.52f, 0.32f, 0.34f, 0.20f}, 9.0f, 2.9f, 3.4f, 1.68e-6f, 8.0e-8f},
+    // (128 x 64 ring: three buffers, two workgroups a CU)
+    {{0.0f, 0.57f, 0.36f, 0.0f, 0.37f, 0.25f}, {0.0f, 0.99f, 0.74f, 0.0f, 0.545f, 0.33f}, 4.6f, 4.2f, 2.8f, 1.95e-6f, 7.0e-8f},
+    {{1.40f, 0.55f, 0.37f, 0.33f, 0.37f, 0.22f}, {1.40f, 0.70f, 0.54f, 0.56f, 0.39f, 0.24f}, 3.8f, 2.8f, 3.5f, 1.92e-6f, 9.0e-8f}};
 constexpr int kSplits[8] = {1, 2, 3, 4, 6, 8, 12, 16};
 constexpr int kMinSplitK = 512;
 constexpr int kCus = 256;
@@ -417,17 +474,19 @@ int64_t mid_kps(MidMode mode, int64_t K, int split) {
 
 MidPlan mid_plan(MidMode mode, int64_t M, int64_t N, int64_t K, bool may_split) {
   const MidModel& m = kModels[mode == kMidInt8 ? kMidScaled : mode];
-  MidPlan best{2, 1, 0.0f};
+  MidPlan best{5, 1, 0.0f};
   bool first = true;
-  for (int c = mode == kMidBlock ? 1 : 0; c < 3; ++c) {
+  for (int c = 0; c < kConfigs; ++c) {
+    if (m.tau[c] == 0.0f) continue;
     const MidTile& t = kTiles[c];
+    const int resident = mode == kMidBlock && c == 4 ? 2 : t.resident;
     const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
     for (const int s : kSplits) {
       // INT8 never splits: a partial would leave the exact int32 sum.
       if (s > 1 && (!may_split || mode == kMidInt8 || K < (int64_t)kMinSplitK * s)) break;
-      const float u = (float)cdiv(tiles * s, kCus), rounds = (float)cdiv(cdiv(tiles * s, kCus), t.resident);
+      const float u = (float)cdiv(tiles * s, kCus), rounds = (float)cdiv(cdiv(tiles * s, kCus), resident);
       const float stage = rounds * m.lambda[c] > u * m.tau[c] ? rounds * m.lambda[c] : u * m.tau[c];
-      float us = m.base + (float)cdiv(cdiv(K, kStageK), s) * stage + m.store * u * (float)(t.bn * t.bm) / 65536.0f;
+      float us = m.base + m.cold * (float)N * (float)K + (float)cdiv(cdiv(K, kStageK), s) * stage + m.store * u * (float)(t.bn * t.bm) / 65536.0f;
       if (s > 1) us += m.reduce + m.partial * (float)s * (float)M * (float)N;
       if (first || us < best.us) {
         first = false;
@@ -447,14 +506,26 @@ void launch_tile(const MidArgs& g, const MidPlan& p, int64_t kps, hipStream_t st
   const MidTile& t = kTiles[p.config];
   const int tiles_m = (int)cdiv(g.M, t.bm);
   const dim3 grid((unsigned)(tiles_m * cdiv(g.N, t.bn)), (unsigned)p.split);
-  if constexpr (MODE != kMidBlock) {
-    if (p.config == 0) {
-      hipLaunchKernelGGL((fp8_mid_kernel<MODE, 256, 256, 2, 4, 1>), grid, dim3(512), 0, st, g, tiles_m, kps);
-      return;
+#define AYK_MID(...) hipLaunchKernelGGL((fp8_mid_kernel<MODE, __VA_ARGS__>), grid, dim3(threads), 0, st, g, tiles_m, kps)
+  const unsigned threads = p.config == 0 ? 512 : 256;
+  if constexpr (MODE == kMidBlock) {
+    switch (p.config) {
+      case 1: AYK_MID(128, 128, 2, 2, 2, 2); break;
+      case 2: AYK_MID(128, 64, 2, 2, 2, 2); break;
+      case 4: AYK_MID(128, 64, 2, 2, 3, 2); break;
+      default: AYK_MID(64, 64, 2, 2, 4, 2); break;
+    }
+  } else {
+    switch (p.config) {
+      case 0: AYK_MID(256, 256, 2, 4, 2, 1); break;
+      case 1: AYK_MID(128, 128, 2, 2, 2, 2); break;
+      case 2: AYK_MID(128, 64, 2, 2, 2, 2); break;
+      case 3: AYK_MID(128, 128, 2, 2, 4, 1); break;
+      case 4: AYK_MID(128, 64, 2, 2, 4, 1); break;
+      default: AYK_MID(64, 64, 2, 2, 4, 2); break;
     }
   }
-  if (p.config == 1) hipLaunchKernelGGL((fp8_mid_kernel<MODE, 128, 128, 2, 2, 2>), grid, dim3(256), 0, st, g, tiles_m, kps);
-  else hipLaunchKernelGGL((fp8_mid_kernel<MODE, 128, 64, 2, 2, 2>), grid, dim3(256), 0, st, g, tiles_m, kps);
+#undef AYK_MID
 }
 
 }  // namespace
@@ -469,10 +540,12 @@ float mid_time(MidMode mode, int64_t M, int64_t N, int64_t K) {
   return us > stream ? us : stream;
 }
 
-bool mid_supported(const MidArgs& g) {
-  return g.K < ((int64_t)1 << 30) && 256 * g.lda < ((int64_t)1 << 31) && 256 * g.ldw < ((int64_t)1 << 31) &&
-         256 * g.ld_sa < ((int64_t)1 << 31) && 256 * g.ld_sb < ((int64_t)1 << 31) &&
-         cdiv(g.M, 64) * cdiv(g.N, 128) < ((int64_t)1 << 31);
+bool mid_supported(MidMode mode, const MidArgs& g) {
+  const int64_t lim = (int64_t)1 << 31;
+  // 256 rows of the operands and of their scales (four bytes at most), and a column-major
+  // scale table, within 32-bit offsets.
+  return g.K < ((int64_t)1 << 30) && 256 * g.lda < lim && 256 * g.ldw < lim && 1024 * g.ld_sa < lim && 1024 * g.ld_sb < lim &&
+         !(mode == kMidBlock && g.sa_vec && 4 * g.M * cdiv(g.K, 128) >= lim) && cdiv(g.M, 64) * cdiv(g.N, 64) < lim;
 }
 
 int mid_launch(MidMode mode, const MidArgs& g, hipStream_t st, const char* op) {
@@ -480,18 +553,16 @@ int mid_launch(MidMode mode, const MidArgs& g, hipStream_t st, const char* op) {
   // A caller that brings no workspace gets the best plan without a split.
   if (p.split > 1 && (g.ws == nullptr || g.ws_bytes < split_bytes(p, g.M, g.N))) p = mid_plan(mode, g.M, g.N, g.K, false);
   const int64_t kps = p.split > 1 ? mid_kps(mode, g.K, p.split) : 0;
-  note_plan("mid %dx%d split=%d", kTiles[p.config].bn, kTiles[p.config].bm, p.split);
+  note_plan("mid %dx%d%s split=%d", kTiles[p.config].bn, kTiles[p.config].bm, p.config >= 3 ? " ring" : "", p.split);
+  const uintptr_t code_align = reinterpret_cast<uintptr_t>(g.sa) | reinterpret_cast<uintptr_t>(g.sb) | (uintptr_t)(g.ld_sa | g.ld_sb);
   switch (mode) {
     case kMidScaled: launch_tile<kMidScaled>(g, p, kps, st); break;
     case kMidBlock: launch_tile<kMidBlock>(g, p, kps, st); break;
     case kMidInt8: launch_tile<kMidInt8>(g, p, kps, st); break;
     default:
-      // 16-byte code loads need whole 512-K chunks and 16-byte aligned code rows, 4-byte ones
-      // whole stages and 4-byte aligned rows.
-      if (g.K % (4 * kStageK) == 0 && g.ld_sa % 16 == 0 && g.ld_sb % 16 == 0 && aligned16(g.sa) && aligned16(g.sb)) {
+      if (g.K % (4 * kStageK) == 0 && (code_align & 15) == 0) {
         launch_tile<kMidMx>(g, p, kps, st);
-      } else if (g.K % kStageK == 0 && g.ld_sa % 4 == 0 && g.ld_sb % 4 == 0 &&
-                 ((reinterpret_cast<uintptr_t>(g.sa) | reinterpret_cast<uintptr_t>(g.sb)) & 3) == 0) {
+      } else if (g.K % kStageK == 0 && (code_align & 3) == 0) {
         launch_tile<kMidMx4>(g, p, kps, st);
       } else {
         launch_tile<kMidMxAny>(g, p, kps, st);

@@ -1,6 +1,8 @@
 // Device helpers shared by the GEMM translation units (gemm.hip, gemm_block.hip).
 #pragma once
 
+#include <utility>
+
 #include "ayk_common.h"
 
 namespace ayk {
@@ -15,6 +17,16 @@ template <int N>
 __device__ inline void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+// Calls f(std::integral_constant<int, i>{}) for i = 0 .. N - 1 (an unrolled loop whose
+// index is a compile-time constant in the body).
+template <typename F, int... I>
+__device__ inline void unrolled_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ inline void unrolled(F&& f) {
+  unrolled_impl(f, std::make_integer_sequence<int, N>{});
 }
 // Workgroup barrier after this wavefront's LDS accesses completed (lgkmcnt(0)); unlike
 // __syncthreads it does not wait for outstanding global loads.

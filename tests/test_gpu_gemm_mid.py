@@ -117,3 +117,33 @@ def test_medium_tiles_nan_codes_stay_in_their_row(gpu):
     cb[3, 0] = 0xFF
     y = mxfp8_scaled_mm(a, ca, w, cb, out=torch.empty(m, n, device=gpu))
     assert y[:, 3].isnan().all() and torch.isfinite(y[:, [c for c in range(n) if c != 3]]).all()
+
+
+@pytest.mark.parametrize("stages", [1, 2, 3, 4, 5, 7, 8, 9])
+@pytest.mark.parametrize("recipe", ["scaled", "block", "block16", "mx", "int8"])
+def test_ring_stage_counts(gpu, recipe, stages):
+    """Every remainder of a K loop that runs in rounds of two, three or four 128-K stages, on
+    shapes of one and of several tiles a side; 16-bit block scales start off a dword."""
+    from ayaka.kernel.hip import _lib, fp8_blockwise_mm, int8_scaled_mm
+
+    k = 128 * stages
+    for m, n in ((70, 136), (200, 1028)):
+        print(f"ring recipe={recipe} m={m} n={n} k={k}", flush=True)
+        if recipe == "int8":
+            g = torch.Generator().manual_seed(k + m)
+            a, w = (torch.randint(-127, 128, (r, k), generator=g, dtype=torch.int8) for r in (m, n))
+            out = int8_scaled_mm(a.to(gpu), w.to(gpu).t(), torch.ones(m, device=gpu), torch.ones(n, device=gpu), out_dtype=torch.float32)
+            assert torch.equal(out.cpu(), (a.double() @ w.double().t()).float())
+        elif recipe == "block16":
+            g = torch.Generator().manual_seed(k + m)
+            a, w = _fp8((m, k), g), _fp8((n, k), g)
+            pool = (torch.rand(1 + m * stages, generator=g) * 1e-2 + 1e-3).to(torch.float16).to(gpu)
+            poolb = (torch.rand(1 + -(-n // 128) * stages, generator=g) * 1e-2 + 1e-3).to(torch.bfloat16).to(gpu)
+            sa, sb = pool[1:].view(m, stages), poolb[1:].view(-1, stages)
+            out = fp8_blockwise_mm(a.to(gpu), w.to(gpu), sa, sb, out=torch.empty(m, n, dtype=torch.float32, device=gpu))
+            ref = (a.to(gpu).double() * _expand(sa, m, k, 1, 128)) @ (w.to(gpu).double() * _expand(sb, n, k, 128, 128)).t()
+            assert_linear_close(out, ref, f"block16 {m}x{n}x{k}")
+        else:
+            out, ref, _ = _run(recipe, m, n, k, True, torch.bfloat16, stages % 2 == 0, gpu)
+            assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
+        assert _lib.last_plan().startswith("mid "), _lib.last_plan()
