@@ -1897,7 +1897,7 @@ MidArgs mid_args(const GemmArgs& g) {
 // A launch goes to the medium tiles where their model is below 0.9 of these (at 0.95 a few
 // large launches lost 2-8%). Batches of 512 to 2048 rows then gain 1.1 to 2.7 times on
 // weights up to 8192 x 8192 (4096 x 4096, M = 512: per-row 34.2 -> 16.0 us, MXFP8 35.2 ->
-// 17.1, block 34.5 -> 21.2; 4096 x 14336, M = 1024: 67.4 -> 63.1, 79.3 -> 69.3).
+// 17.1, block 34.5 -> 21.2).
 struct LargeModel {
   float base, step, tile, reduce, partial;
   float time(int64_t rounds, int64_t steps, int64_t split, int64_t part_elems) const {

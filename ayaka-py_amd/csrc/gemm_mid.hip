@@ -443,7 +443,7 @@ __global__ __launch_bounds__(256) void mid_reduce(const float* __restrict__ part
 // latency) and `store` per 256 x 256 outputs; `cold` is the weights' share that no stage
 // hides; a split adds a reduce launch and the fp32 partials' traffic. Its choice is 1-2%
 // slower than the fastest triple on average (tau of the two-buffer tiles: from the launches of
-// two rounds and more, 10-15% above the fit, whose weight lies on the small ones).
+// two rounds and more, above the fit, whose weight lies on the small ones).
 struct MidPlan {
   int config, split;
   float us;
@@ -461,7 +461,7 @@ constexpr MidModel kModels[3] = {
     {{1.25f, 0.44f, 0.32f, 0.50f, 0.27f, 0.19f}, {1.25f, 0.71f, 0.52f, 0.32f, 0.34f, 0.20f}, 9.0f, 2.9f, 3.4f, 1.68e-6f, 8.0e-8f},
     // (128 x 64 ring: three buffers, two workgroups a CU)
     {{0.0f, 0.57f, 0.36f, 0.0f, 0.37f, 0.25f}, {0.0f, 0.99f, 0.74f, 0.0f, 0.545f, 0.33f}, 4.6f, 4.2f, 2.8f, 1.95e-6f, 7.0e-8f},
-    {{1.40f, 0.55f, 0.37f, 0.33f, 0.37f, 0.22f}, {1.40f, 0.70f, 0.54f, 0.56f, 0.39f, 0.24f}, 3.8f, 2.8f, 3.5f, 1.92e-6f, 9.0e-8f}};
+    {{1.71f, 0.55f, 0.37f, 0.33f, 0.37f, 0.22f}, {1.40f, 0.70f, 0.54f, 0.56f, 0.39f, 0.24f}, 3.8f, 2.8f, 3.5f, 1.92e-6f, 9.0e-8f}};
 constexpr int kSplits[8] = {1, 2, 3, 4, 6, 8, 12, 16};
 constexpr int kMinSplitK = 512;
 constexpr int kCus = 256;
