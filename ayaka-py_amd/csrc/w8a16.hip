@@ -1433,7 +1433,7 @@ using namespace ayk;
 extern "C" {
 
 size_t ayk_fp8_weight_only_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t block_size_x) {
-  if (M < 2) return 0;
+  if (M < 2 || N < 1 || K < 1 || block_size_x < 1) return 0;
   // An upper bound over the kernels (alignment decides which one runs).
   const size_t st = stream_workspace(stream_plan(M, N, K, block_size_x), M, N);
   const size_t rs = rows_workspace(rows_plan(M, N, K, block_size_x), M, N);

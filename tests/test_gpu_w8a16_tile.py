@@ -109,3 +109,12 @@ def test_weight_only_gemm_tile_views_and_graph(gpu):
         torch.cuda.synchronize()
         assert torch.equal(captured, ref), i
         torch.mm(torch.ones(64, 64, device=gpu), torch.ones(64, 64, device=gpu))
+
+
+def test_weight_only_gemm_empty_k_is_refused(gpu):
+    """An empty K is an argument error, also for callers that give the scale layout."""
+    from ayaka.kernel.hip import fp8_weight_only_gemm
+
+    x, w = torch.empty(2, 0, dtype=torch.bfloat16, device=gpu), torch.empty(128, 0, device=gpu).to(FP8)
+    with pytest.raises(ValueError, match="bad shape"):
+        fp8_weight_only_gemm(x, w, torch.ones(128, device=gpu), 1, 1, 128, "float32")

@@ -9,6 +9,8 @@ Expected values are the reference's documented contracts
 import ctypes
 import pathlib
 import re
+import subprocess
+import sys
 from types import SimpleNamespace
 
 import pytest
@@ -346,3 +348,26 @@ def test_c_abi_rejects_bad_arguments_without_a_gpu():
     assert lib.ayk_fp8_blockwise_mm_workspace_bytes(40, 96, 8192) > 0
     assert lib.ayk_fp8_blockwise_mm_workspace_bytes(32, 7168, 18432) > 0
     assert lib.ayk_fp8_blockwise_mm_workspace_bytes(4096, 18432, 7168) == 0
+
+
+def test_workspace_queries_of_empty_shapes_are_zero():
+    """Every size query is asked before the launch checks its shape, so it answers 0 for a
+    zero or negative dimension. In a process of its own: a fault there must not end the run."""
+    from ayaka.kernel.hip import _lib
+
+    queries = {n: len(sig) for n, sig in _lib.SIGNATURES.items() if n.endswith("_workspace_bytes")}
+    assert len(queries) >= 7
+    code = f"""
+import ctypes
+lib = ctypes.CDLL({str(_lib.load_library()._name)!r})
+for name, args in {queries!r}.items():
+    fn = getattr(lib, name)
+    fn.restype, fn.argtypes = ctypes.c_size_t, [ctypes.c_int64] * args
+    for zero in range(args):
+        for value in (0, -1):
+            shape = [64, 512, 4096, 128][:args] if args > 2 else [512, 4096]
+            shape[zero] = value
+            assert fn(*shape) == 0, (name, shape)
+"""
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert done.returncode == 0, (done.returncode, done.stderr)
