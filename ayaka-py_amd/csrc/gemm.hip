@@ -20,9 +20,10 @@
 // The kernels here are the 256 x 256 ones (and the block-scaled 128 x 128 one);
 // gemm_mid.hip has the medium tiles, gemm_skinny.hip the decode batches, and launch_gemm
 // chooses. The general kernel below remains for row strides past 32-bit tile offsets: a
-// 256-thread workgroup owns a BN x BM tile and walks K in 128-byte steps, staged global ->
-// VGPR -> LDS with double buffering; LDS rows are padded to 144 bytes so the 32 rows a
-// wavefront reads at one K offset fall on distinct banks.
+// 256-thread workgroup owns a 128 x BM tile (BM = 32, 64 or 128 activation rows) and walks
+// K, or its piece of a K split, in 128-byte steps, staged global -> VGPR -> LDS with double
+// buffering; LDS rows are padded to 144 bytes so the 32 rows a wavefront reads at one K
+// offset fall on distinct banks.
 #include "ayk_common.h"
 #include "gemm_block.h"
 #include "gemm_mid.h"
@@ -76,7 +77,7 @@ struct GemmArgs {
   int tiles_m;     // number of BM tiles along M
   float* ws;       // split-K partials, ws_bytes long
   size_t ws_bytes;
-  int64_t kps;     // 256 x 256 pair kernel: K per piece of a K split (0: no split)
+  int64_t kps;     // 256 x 256 pair and general kernels: K per piece of a K split (0: no split)
   // 256 x 256 pair kernel, tail split (tail_split > 1): workgroups past dp_tiles take
   // K piece (b - dp_tiles) % tail_split of tile dp_tiles + (b - dp_tiles) / tail_split.
   int dp_tiles;
@@ -163,8 +164,34 @@ __device__ inline void store4(const GemmArgs& g, int64_t m, int64_t n, const flo
 
 // BN: weight rows per tile, BM: activation rows per tile, WN x WM wavefront grid.
 template <int MODE, int BN, int BM, int WN, int WM>
-__global__ __launch_bounds__(kThreads) void fp8_gemm_kernel(GemmArgs g) {
+__global__ __launch_bounds__(kThreads) void fp8_gemm_kernel(GemmArgs gin) {
   static_assert(WN * WM == kThreads / kWave, "4 wavefronts per workgroup");
+  // With a K split, blockIdx.y takes K range [y kps, (y + 1) kps) (kps % 128 == 0) and
+  // writes its fp32 partials (already scaled) to ws[y] ([M, N]); block_split_reduce sums
+  // them, adds the bias and rounds once.
+  GemmArgs g = gin;
+  if constexpr (MODE != MODE_INT8) {
+    if (gin.kps > 0) {
+      const int64_t k0 = (int64_t)blockIdx.y * gin.kps, kb0 = k0 / 128, kb_total = gin.K / 128;
+      g.K = gin.K - k0 < gin.kps ? gin.K - k0 : gin.kps;
+      g.a = gin.a + k0;
+      g.w = gin.w + k0;
+      if constexpr (MODE == MODE_BLOCK) {  // K-blocked scale tables follow the K range
+        g.sa = static_cast<const uint8_t*>(gin.sa) + (gin.sa_vec ? kb0 * gin.M : kb0) * dtype_size(gin.sa_dtype);
+        g.ld_sa = gin.sa_vec ? 0 : kb_total;
+        g.sb = static_cast<const uint8_t*>(gin.sb) + kb0 * dtype_size(gin.sb_dtype);
+        g.ld_sb = kb_total;
+      }
+      if constexpr (MODE == MODE_MX) {  // UE8M0 code rows: the range's codes start k0 / 32 in
+        g.sa = static_cast<const uint8_t*>(gin.sa) + k0 / 32;
+        g.sb = static_cast<const uint8_t*>(gin.sb) + k0 / 32;
+      }
+      g.bias = nullptr;
+      g.out = gin.ws + (int64_t)blockIdx.y * gin.M * gin.N;
+      g.out_dtype = AYK_F32;
+      g.ldo = gin.N;
+    }
+  }
   constexpr int TN = BN / WN, TM = BM / WM;  // wavefront tile
   constexpr int FN = TN / 32, FM = TM / 32;  // 32x32 MFMA tiles per wavefront
   static_assert(FN >= 1 && FM >= 1, "wavefront tile must be a multiple of 32x32");
@@ -1639,16 +1666,26 @@ int64_t block_split(int64_t M, int64_t N, int64_t K) {
   while (tiles * split < kBlkSplitTarget && K / (split * 2) >= 1024 && (K / 128) % (split * 2) == 0) split *= 2;
   return split;
 }
-// Rowwise / per-tensor / MXFP8 K split for launches short of one round of 256 x 256 tiles
-// (256 workgroups, one per CU): as many splits as still fit in that one round, at least
-// 1024 K each (the last may be shorter). Spilling into a second round doubles the time of
-// the splits and multiplies the partial-sum traffic (Qwen2 down at M = 2048: 5 splits
-// 231 us, 2 splits fill the round).
-int64_t scaled_split(int64_t M, int64_t N, int64_t K) {
+// The same rule for the general kernel's 32- or 64-row tiles in block mode.
+int general_rows(int64_t M) { return M <= 32 ? 32 : (M <= 64 ? 64 : 128); }  // its tile height
+int64_t general_block_split(int64_t M, int64_t N, int64_t K) {
+  if (M > 64 || K % 128) return 1;
+  const int64_t tiles = cdiv(M, general_rows(M)) * cdiv(N, 128);
+  int64_t split = 1;
+  while (tiles * split < kBlkSplitTarget && K / (split * 2) >= 1024 && (K / 128) % (split * 2) == 0) split *= 2;
+  return split;
+}
+// Rowwise / per-tensor / MXFP8 K split for launches short of one round of bm x bn tiles
+// (256 workgroups of the 256 x 256 kernel, one per CU; 512 of the general kernel's): as many
+// splits as still fit in that one round, at least 1024 K each (the last may be shorter).
+// Spilling into a second round doubles the time of the splits and multiplies the
+// partial-sum traffic (Qwen2 down at M = 2048: 5 splits 231 us, 2 splits fill the round).
+int64_t scaled_split(int64_t M, int64_t N, int64_t K, int bm, int bn) {
   if (K % 128) return 1;
-  const int64_t tiles = cdiv(M, kBigTile) * cdiv(N, kBigTile);
-  if (tiles * 2 > 256) return 1;
-  const int64_t want = 256 / tiles, most = K / 1024;
+  const int64_t round = bm == kBigTile ? 256 : kBlkSplitTarget;
+  const int64_t tiles = cdiv(M, bm) * cdiv(N, bn);
+  if (tiles * 2 > round) return 1;
+  const int64_t want = round / tiles, most = K / 1024;
   const int64_t split = want < most ? want : most;
   if (split <= 1) return 1;
   const int64_t kps = cdiv(K / 128, split) * 128;
@@ -1695,15 +1732,15 @@ size_t tail_workspace(const TailPlan& p) {
 }
 
 size_t scaled_split_workspace(int64_t M, int64_t N, int64_t K) {
-  if (M < kBigTile || N < kBigTile) return 0;
-  const int64_t split = scaled_split(M, N, K);
+  int64_t split = scaled_split(M, N, K, general_rows(M), 128);
+  if (M >= kBigTile && N >= kBigTile) split = std::max(split, scaled_split(M, N, K, kBigTile, kBigTile));
   return split > 1 ? (size_t)split * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 // Upper bounds over the block kernels that may take the launch (alignment and the models
 // decide which one does).
 bool block256_wanted(int64_t M, int64_t N, int64_t K);
 size_t block_split_workspace(int64_t M, int64_t N, int64_t K) {
-  int64_t split = M > 64 && N >= kBlkTile ? block_split(M, N, K) : 1;
+  int64_t split = M <= 64 ? general_block_split(M, N, K) : (N >= kBlkTile ? block_split(M, N, K) : 1);
   if (block256_wanted(M, N, K)) {
     const int64_t s256 = block256_split(M, N, K);
     split = s256 > split ? s256 : split;
@@ -1767,7 +1804,7 @@ int launch_big(GemmArgs g, hipStream_t st, const char* op) {
   if (tiles > 0x7FFFFFFF) return fail(AYK_EINVAL, "%s: problem too large", op);
   if constexpr (MODE == MODE_MX) {
     // K per split in whole chunks of four 128-K pairs (keeps the code rows 16-byte aligned)
-    const int64_t planned = xcd_pieces(scaled_split(g.M, g.N, g.K));
+    const int64_t planned = xcd_pieces(scaled_split(g.M, g.N, g.K, kBigTile, kBigTile));
     const int64_t kps = planned > 1 ? cdiv(g.K / 512, planned) * 512 : g.K;
     const int64_t split = cdiv(g.K, kps);
     g.kps = split > 1 ? kps : 0;
@@ -1786,7 +1823,7 @@ int launch_big(GemmArgs g, hipStream_t st, const char* op) {
                         g.ldo, st);
   } else if (g.K % (2 * kBigK) == 0) {
     // INT8 never splits: a split's partial would leave the exact int32 accumulator.
-    const int64_t planned = MODE == MODE_SCALED ? xcd_pieces(scaled_split(g.M, g.N, g.K)) : 1;
+    const int64_t planned = MODE == MODE_SCALED ? xcd_pieces(scaled_split(g.M, g.N, g.K, kBigTile, kBigTile)) : 1;
     g.kps = planned > 1 ? scaled_kps(g.K, planned) : 0;
     const int64_t split = planned > 1 ? cdiv(g.K, g.kps) : 1;
     if (split > 1) {
@@ -1833,16 +1870,38 @@ int launch_block_big(GemmArgs g, hipStream_t st, const char* op) {
   return check_launch(op);
 }
 
-// The general kernel: operands whose row strides leave the medium tiles' 32-bit offsets.
-template <int MODE>
-int launch_general(GemmArgs g, hipStream_t st, const char* op) {
-  constexpr int kTile = 128;
-  g.tiles_m = (int)cdiv(g.M, kTile);
-  const int64_t tiles = (int64_t)g.tiles_m * cdiv(g.N, kTile);
+// The general kernel, for operands whose row strides leave the medium tiles' 32-bit
+// offsets: tiles of 32, 64 or 128 activation rows and a K split. With 128-row tiles and no
+// split alone, a decode batch leaves most CUs idle (activation rows 8 MiB apart: per-row
+// 4096 x 14464, M = 16, 138 us against 21; block 4096 x 4096, M = 16, 57 against 13; MXFP8
+// 4096 x 4224, M = 128, 51 against 26).
+template <int MODE, int BM, int WN, int WM>
+int launch_cfg(GemmArgs g, hipStream_t st, const char* op) {
+  constexpr int kBn = 128;
+  g.tiles_m = (int)cdiv(g.M, BM);
+  const int64_t tiles = (int64_t)g.tiles_m * cdiv(g.N, kBn);
   if (tiles > 0x7FFFFFFF) return fail(AYK_EINVAL, "%s: problem too large", op);
-  note_plan("general");
-  hipLaunchKernelGGL((fp8_gemm_kernel<MODE, kTile, kTile, 2, 2>), dim3((unsigned)tiles), dim3(kThreads), 0, st, g);
+  const int64_t split = MODE == MODE_BLOCK ? general_block_split(g.M, g.N, g.K)
+                        : (MODE == MODE_INT8 ? 1 : scaled_split(g.M, g.N, g.K, BM, kBn));
+  g.kps = 0;
+  if (split > 1) {
+    const size_t need = (size_t)split * (size_t)g.M * (size_t)g.N * sizeof(float);
+    if (g.ws == nullptr || g.ws_bytes < need)
+      return fail(AYK_EWORKSPACE, "%s: workspace of %zu bytes required, %zu given", op, need, g.ws_bytes);
+    g.kps = MODE == MODE_BLOCK ? g.K / split : scaled_kps(g.K, split);
+  }
+  note_plan("general %dx%d split=%d", kBn, BM, (int)split);
+  hipLaunchKernelGGL((fp8_gemm_kernel<MODE, kBn, BM, WN, WM>), dim3((unsigned)tiles, (unsigned)split), dim3(kThreads), 0, st, g);
+  if (int rc = check_launch(op)) return rc;
+  if (split == 1) return AYK_OK;
+  launch_split_reduce(block_split_reduce, g.ws, g.M, g.N, (int)split, g.bias, g.bias_dtype, g.out, g.out_dtype, g.ldo, st);
   return check_launch(op);
+}
+template <int MODE>
+int launch_general(const GemmArgs& g, hipStream_t st, const char* op) {
+  if (g.M <= 32) return launch_cfg<MODE, 32, 4, 1>(g, st, op);
+  if (g.M <= 64) return launch_cfg<MODE, 64, 2, 2>(g, st, op);
+  return launch_cfg<MODE, 128, 2, 2>(g, st, op);
 }
 
 // The 256 x 256 block-scaled kernel serves launches of at least half a round (128) of
@@ -1912,7 +1971,7 @@ float pair_time(int mode, int64_t M, int64_t N, int64_t K) {
   const LargeModel& m = mx ? kPairMx : kPairScaled;
   const int64_t unit = mx ? 512 : 128, tiles = cdiv(M, kBigTile) * cdiv(N, kBigTile);
   if (mode == MODE_INT8) return m.time(cdiv(tiles, 256), cdiv(K, 128), 1, 0);  // never split
-  const int64_t planned = xcd_pieces(scaled_split(M, N, K));
+  const int64_t planned = xcd_pieces(scaled_split(M, N, K, kBigTile, kBigTile));
   if (planned > 1) {
     const int64_t kps = cdiv(K / unit, planned) * unit, split = cdiv(K, kps);
     return m.time(1, cdiv(kps, 128), split, split * M * N);

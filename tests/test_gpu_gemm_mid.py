@@ -19,34 +19,48 @@ def _expand(scale, rows, cols, by, bx):
     return scale.double().repeat_interleave(by, 0)[:rows].repeat_interleave(bx, 1)[:, :cols]
 
 
-def _run(recipe, m, n, k, bias, odt, col_major, gpu):
+def _wide(t, stride, dev):
+    """``t`` on the device, its rows ``stride`` elements apart (None: contiguous)."""
+    t = t.to(dev)
+    if stride is None:
+        return t
+    rows = torch.empty((t.shape[0] - 1) * stride + t.shape[1], dtype=torch.uint8, device=dev).view(t.dtype)
+    view = rows.as_strided(t.shape, (stride, 1))
+    view.copy_(t)
+    return view
+
+
+def _run(recipe, m, n, k, bias, odt, col_major, gpu, lda=None, ldw=None):
     """(output, fp64 reference, plan) of one call with seeded operands."""
     from ayaka.kernel.hip import _lib, fp8_blockwise_mm, fp8_scaled_mm, mxfp8_scaled_mm
 
     g = torch.Generator().manual_seed(m * 131 + n * 7 + k)
     a, w = _fp8((m, k), g), _fp8((n, k), g)
+    ag, wg = _wide(a, lda, gpu), _wide(w, ldw, gpu)
     b = torch.randn(n, generator=g).to(odt) if bias else None
     out = torch.empty(m, n, dtype=odt, device=gpu)
     bg = None if b is None else b.to(gpu)
     if recipe == "scaled":
         sa, sb = torch.rand(m, generator=g) * 1e-2, torch.rand(n, generator=g) * 1e-2
-        fp8_scaled_mm(a.to(gpu), w.to(gpu).t(), sa.to(gpu), sb.to(gpu), bias=bg, out=out)
+        fp8_scaled_mm(ag, wg.t(), sa.to(gpu), sb.to(gpu), bias=bg, out=out)
         sa, sb = sa[:, None].double(), sb[:, None].double()
     elif recipe == "scalar":
         sa, sb = torch.tensor(0.003), torch.tensor(0.02)
-        fp8_scaled_mm(a.to(gpu), w.to(gpu).t(), sa.to(gpu), sb.to(gpu), bias=bg, out=out)
-    elif recipe == "block":
+        fp8_scaled_mm(ag, wg.t(), sa.to(gpu), sb.to(gpu), bias=bg, out=out)
+    elif recipe in ("block", "block16"):
         kb = -(-k // 128)
         ta, tb = torch.rand(m, kb, generator=g) * 1e-2, torch.rand(-(-n // 128), kb, generator=g) * 1e-2
         if not col_major:
             tb = tb.to(torch.bfloat16)
+        if recipe == "block16":
+            ta = ta.to(torch.float16)
         table = ta.t().contiguous() if col_major else ta
-        fp8_blockwise_mm(a.to(gpu), w.to(gpu), table.to(gpu), tb.to(gpu), bias=bg, out=out, a_scale_col_major=col_major)
+        fp8_blockwise_mm(ag, wg, table.to(gpu), tb.to(gpu), bias=bg, out=out, a_scale_col_major=col_major)
         sa, sb = _expand(ta, m, k, 1, 128), _expand(tb, n, k, 128, 128)
     else:
         ca = torch.randint(112, 122, (m, k // 32), generator=g, dtype=torch.uint8)
         cb = torch.randint(112, 122, (n, k // 32), generator=g, dtype=torch.uint8)
-        mxfp8_scaled_mm(a.to(gpu), ca.to(gpu), w.to(gpu), cb.to(gpu), bg, out=out)
+        mxfp8_scaled_mm(ag, ca.to(gpu), wg, cb.to(gpu), bg, out=out)
         sa, sb = (_expand(torch.exp2(c.double() - 127), c.shape[0], k, 1, 32) for c in (ca, cb))
     plan = _lib.last_plan()
     ref = (a.double() * sa).to(gpu) @ (w.double() * sb).to(gpu).t()
@@ -147,3 +161,38 @@ def test_ring_stage_counts(gpu, recipe, stages):
             out, ref, _ = _run(recipe, m, n, k, True, torch.bfloat16, stages % 2 == 0, gpu)
             assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
         assert _lib.last_plan().startswith("mid "), _lib.last_plan()
+
+
+_FAR = 1 << 23  # rows 8 MiB apart: 256 of them leave the medium tiles' 32-bit offsets
+
+
+@pytest.mark.parametrize("recipe,m,n,k,bias,odt,far,expect", [
+    ("scaled", 20, 300, 4224, True, torch.bfloat16, "a", "general 128x32 split=4"),   # last piece shorter
+    ("scalar", 50, 260, 208, False, torch.float32, "a", "general 128x64 split=1"),    # K tail
+    ("scaled", 130, 300, 4224, True, torch.float16, "a", "general 128x128 split=4"),
+    ("scaled", 20, 140, 2176, False, torch.bfloat16, "w", "general 128x32 split=2"),
+    ("block", 17, 300, 4096, True, torch.bfloat16, "a", "general 128x32 split=4"),    # bf16 weight scales
+    ("block16", 40, 200, 4096, True, torch.float32, "a", "general 128x64 split=4"),   # fp16 activation scales too
+    ("block", 129, 140, 1152, False, torch.bfloat16, "a", "general 128x128 split=1"),
+    ("mx", 20, 300, 4224, True, torch.bfloat16, "a", "general 128x32 split=4"),
+    ("mx", 64, 130, 1184, False, torch.float32, "a", "general 128x64 split=1"),       # unaligned codes
+])
+def test_general_kernel_rows_far_apart(gpu, recipe, m, n, k, bias, odt, far, expect):
+    """Operand rows so far apart that the tiled kernels' offsets do not reach them."""
+    print(f"general recipe={recipe} m={m} n={n} k={k} far={far}", flush=True)
+    lda, ldw = (_FAR, None) if far == "a" else (None, _FAR)
+    out, ref, plan = _run(recipe, m, n, k, bias, odt, recipe == "block" and m > 128, gpu, lda, ldw)
+    assert plan == expect, plan
+    assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
+
+
+def test_general_kernel_int8_rows_far_apart(gpu):
+    from ayaka.kernel.hip import _lib, int8_scaled_mm
+
+    g = torch.Generator().manual_seed(3)
+    for m, tile in ((20, 32), (50, 64), (130, 128)):
+        a, w = (torch.randint(-127, 128, (r, 1040), generator=g, dtype=torch.int8) for r in (m, 260))
+        out = int8_scaled_mm(_wide(a, _FAR, gpu), w.to(gpu).t(), torch.ones(m, device=gpu), torch.ones(260, device=gpu),
+                             out_dtype=torch.float32)
+        assert _lib.last_plan() == f"general 128x{tile} split=1", _lib.last_plan()
+        assert torch.equal(out.cpu(), (a.double() @ w.double().t()).float())
