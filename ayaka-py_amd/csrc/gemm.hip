@@ -19,11 +19,11 @@
 //
 // The kernels here are the 256 x 256 ones (and the block-scaled 128 x 128 one);
 // gemm_mid.hip has the medium tiles, gemm_skinny.hip the decode batches, and launch_gemm
-// chooses. The general kernel below remains for row strides past 32-bit tile offsets: a
-// 256-thread workgroup owns a 128 x BM tile (BM = 32, 64 or 128 activation rows) and walks
-// K, or its piece of a K split, in 128-byte steps, staged global -> VGPR -> LDS with double
-// buffering; LDS rows are padded to 144 bytes so the 32 rows a wavefront reads at one K
-// offset fall on distinct banks.
+// chooses. The general kernel below remains for row strides past 32-bit tile offsets and a
+// few decode shapes (general_wanted): a 256-thread workgroup owns a 128 x BM tile (BM = 32,
+// 64 or 128 activation rows) and walks K, or its piece of a K split, in 128-byte steps,
+// staged global -> VGPR -> LDS with double buffering; LDS rows are padded to 144 bytes so
+// the 32 rows a wavefront reads at one K offset fall on distinct banks.
 #include "ayk_common.h"
 #include "gemm_block.h"
 #include "gemm_mid.h"
@@ -1871,7 +1871,7 @@ int launch_block_big(GemmArgs g, hipStream_t st, const char* op) {
 }
 
 // The general kernel, for operands whose row strides leave the medium tiles' 32-bit
-// offsets: tiles of 32, 64 or 128 activation rows and a K split. With 128-row tiles and no
+// offsets and the shapes of general_wanted: tiles of 32, 64 or 128 activation rows and a K split. With 128-row tiles and no
 // split alone, a decode batch leaves most CUs idle (activation rows 8 MiB apart: per-row
 // 4096 x 14464, M = 16, 138 us against 21; block 4096 x 4096, M = 16, 57 against 13; MXFP8
 // 4096 x 4224, M = 128, 51 against 26).
@@ -1990,6 +1990,25 @@ float block128_time(int64_t M, int64_t N, int64_t K) {
   return kBlock128.time(cdiv(cdiv(M, kBlkTile) * cdiv(N, kBlkTile) * split, 256), K / 128 / split, split, split * M * N);
 }
 
+// Decode shapes that the general kernel's small tiles keep from the medium ones, which start
+// a stage ring for them that a short K does not fill, on two rounds of workgroups past 32768
+// columns (general against medium, M = 17 to 25: block 38144 x 128 5.6 us and 8.9, 27648 x 128
+// 5.1 and 5.9, MXFP8 36828 x 128 5.5 and 9.0, 25140 x 320 7.0 and 8.2, per-row 34064 x 96 7.0
+// and 8.1; M = 64, MXFP8 37324 x 128 7.6 and 10.2). Below 16384 columns both take 4 to 5 us,
+// and past these K the medium tiles are faster. MXFP8 batches of up to 8 rows on large weights
+// whose K the decode kernel refuses stream faster in the general kernel's K split (6400 x
+// 21376, M = 5: 38.4 and 44.2, 18584 x 4736, M = 2: 26.9 and 30.9); in two pieces, from 9 rows
+// on and below 66 MB they mostly do not (29184 x 6784, M = 8: 54.5 and 47.2; 13552 x 4736, M = 2:
+// 23.8 and 16.7).
+template <int MODE>
+bool general_wanted(int64_t M, int64_t N, int64_t K) {
+  constexpr bool mx = MODE == MODE_MX, scales = mx || MODE == MODE_BLOCK;  // per-stage scale loads
+  if (N > 32768 && (M <= 32 ? K <= 512 : M <= 64 && scales && K <= (mx ? 128 : 384))) return true;
+  // (MXFP8 rows of codes that no dword bounds cost the medium tiles two loads a row and stage)
+  if (scales && M <= 32 && N > 16384 && K <= (mx && K % 128 ? 448 : 256)) return true;
+  return mx && M <= 8 && N * K > 66000000 && K % 256 == 128 && scaled_split(M, N, K, 32, 128) >= 3;
+}
+
 template <int MODE>
 int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
   const MidArgs mid = mid_args(g);
@@ -2046,7 +2065,7 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
       }
     }
   }
-  if (mid_ok) return mid_launch(mid_mode(MODE), mid, st, op);
+  if (mid_ok && !general_wanted<MODE>(g.M, g.N, g.K)) return mid_launch(mid_mode(MODE), mid, st, op);
   return launch_general<MODE>(g, st, op);
 }
 

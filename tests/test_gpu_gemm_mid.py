@@ -196,3 +196,26 @@ def test_general_kernel_int8_rows_far_apart(gpu):
                              out_dtype=torch.float32)
         assert _lib.last_plan() == f"general 128x{tile} split=1", _lib.last_plan()
         assert torch.equal(out.cpu(), (a.double() @ w.double().t()).float())
+
+
+@pytest.mark.parametrize("recipe,m,n,k,expect", [
+    ("scaled", 32, 32900, 208, "general 128x32 split=1"),
+    ("scaled", 33, 32900, 208, "mid 64x64 ring split=1"),
+    ("block", 17, 32900, 512, "general 128x32 split=1"),     # bf16 weight scales
+    ("block", 64, 32900, 384, "general 128x64 split=1"),
+    ("block", 20, 16500, 128, "general 128x32 split=1"),
+    ("block", 20, 16300, 128, "mid 64x64 ring split=1"),
+    ("mx", 32, 17000, 224, "general 128x32 split=1"),
+    ("mx", 32, 17000, 384, "mid 128x64 ring split=1"),
+    ("mx", 20, 17000, 448, "general 128x32 split=1"),        # K % 128 != 0
+    ("mx", 64, 32900, 128, "general 128x64 split=1"),
+    ("mx", 8, 4100, 16512, "general 128x32 split=15"),
+    ("mx", 9, 4900, 16512, "mid 128x64 ring split=6"),
+    ("mx", 2, 18584, 4736, "general 128x32 split=3"),
+])
+def test_general_kernel_decode_shapes(gpu, recipe, m, n, k, expect):
+    """The decode shapes of the general kernel's small tiles, at the edges of their rule."""
+    print(f"general decode recipe={recipe} m={m} n={n} k={k}", flush=True)
+    out, ref, plan = _run(recipe, m, n, k, True, torch.bfloat16, False, gpu)
+    assert plan == expect, plan
+    assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
