@@ -812,8 +812,10 @@ bool skinny_fp8_supported(const SkinnyFp8Args& g) {
 // Modelled time (microseconds) of this kernel on its plan: a launch, rounds of resident
 // workgroups that each walk their K at `step` per 128 (one or two 32-row activation tiles),
 // no faster than the weights stream, and a split's reduce. Fitted on 36 weight shapes from
-// 1280 x 8320 to 38400 x 3584 and batches of 2 to 64 (mean error 7-10%). 0: the GEMV-shaped
-// kernel takes the launch.
+// 1280 x 8320 to 38400 x 3584 and batches of 2 to 64 (mean error 7-10%); MXFP8's reduce from
+// narrower ones too, whose split launches a reduce of 5.5 us put 3 to 4 us too high, so that
+// they went to the medium tiles at a loss (1807 x 12288, M = 3: 11.9 -> 15.3 us, 2048 x 8192,
+// M = 2: 9.8 -> 11.7). 0: the GEMV-shaped kernel takes the launch.
 float skinny_fp8_time(const SkinnyFp8Args& g) {
   if (rows_gemv_wanted(g)) return 0.0f;
   const SkPlan p = skinny_plan(g.M, g.N, g.K, g.mode);
@@ -821,7 +823,7 @@ float skinny_fp8_time(const SkinnyFp8Args& g) {
     float base, step[2], bytes_us, reduce, partial;
   };
   constexpr Model kModel[3] = {{6.9f, {0.40f, 0.61f}, 5.2e6f, 1.9f, 2.7e-6f},
-                               {5.0f, {0.56f, 0.81f}, 4.5e6f, 5.5f, 4.0e-6f},
+                               {5.0f, {0.56f, 0.81f}, 4.5e6f, 4.0f, 4.0e-6f},
                                {5.5f, {0.41f, 0.79f}, 4.9e6f, 4.0f, 0.0f}};  // by mode: rows, MX, block
   const Model& m = kModel[g.mode];
   const int64_t wgs = cdiv(g.N, 32 * p.fn * (kWaves / p.ks)) * p.split;

@@ -212,10 +212,14 @@ def test_general_kernel_int8_rows_far_apart(gpu):
     ("mx", 8, 4100, 16512, "general 128x32 split=15"),
     ("mx", 9, 4900, 16512, "mid 128x64 ring split=6"),
     ("mx", 2, 18584, 4736, "general 128x32 split=3"),
+    ("mx", 3, 1807, 12288, "skinny fn=1 fm=1 ks=4 g=2 ch=1 split=4"),
+    ("mx", 2, 2048, 8192, "skinny fn=1 fm=1 ks=4 g=2 ch=4 split=4"),
+    ("mx", 20, 4096, 10240, "mid 128x64 ring split=7"),
 ])
-def test_general_kernel_decode_shapes(gpu, recipe, m, n, k, expect):
-    """The decode shapes of the general kernel's small tiles, at the edges of their rule."""
-    print(f"general decode recipe={recipe} m={m} n={n} k={k}", flush=True)
+def test_decode_kernel_choice(gpu, recipe, m, n, k, expect):
+    """Decode shapes at the edges between the general kernel's small tiles, the decode kernel
+    and the medium tiles."""
+    print(f"decode choice recipe={recipe} m={m} n={n} k={k}", flush=True)
     out, ref, plan = _run(recipe, m, n, k, True, torch.bfloat16, False, gpu)
     assert plan == expect, plan
     assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
