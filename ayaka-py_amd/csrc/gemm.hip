@@ -1953,10 +1953,16 @@ MidArgs mid_args(const GemmArgs& g) {
 // Modelled times (microseconds) of the large-tile kernels on the plans above, fitted on
 // the shapes of the medium-tile kernel's model (3-4% mean error): a launch, `rounds` of
 // one workgroup a CU over `steps` 128-K blocks each, a split's reduce and partials.
-// A launch goes to the medium tiles where their model is below 0.9 of these (at 0.95 a few
-// large launches lost 2-8%). Batches of 512 to 2048 rows then gain 1.1 to 2.7 times on
-// weights up to 8192 x 8192 (4096 x 4096, M = 512: per-row 34.2 -> 16.0 us, MXFP8 35.2 ->
-// 17.1, block 34.5 -> 21.2).
+// A launch goes to the medium tiles where their model is below a share of these: 0.9 up to
+// 25 us, 0.78 up to 100, 0.74 above. The medium tiles' model is fitted on small launches and
+// promises too much on large ones: at 0.9 throughout, launches it put at 0.78 to 0.9 lost up
+// to 13% (per-row 1794 x 5888 x 10752 115 -> 127 us, block 2328 x 3456 x 3328 48 -> 55, MXFP8
+// 908 x 8352 x 2048 33 -> 37) and gained little in the median. Batches of 512 to 2048 rows gain
+// 1.1 to 2.7 times on weights up to 8192 x 8192 (4096 x 4096, M = 512: per-row 34.2 -> 16.0 us,
+// MXFP8 35.2 -> 17.1, block 34.5 -> 21.2). Against the block-scaled 128 x 128 kernel 0.9 holds
+// throughout (never more than 0.97 of its time there). INT8 takes the per-row models: its
+// matrix steps are two products of half the K, but over 1950 random shapes from 1 to 4096 rows
+// it takes 0.42 of its time without the medium tiles in the mean.
 struct LargeModel {
   float base, step, tile, reduce, partial;
   float time(int64_t rounds, int64_t steps, int64_t split, int64_t part_elems) const {
@@ -1965,6 +1971,8 @@ struct LargeModel {
 };
 constexpr LargeModel kPairScaled{2.7f, 1.57f, 2.65f, 8.6f, 1.0e-6f}, kPairMx{3.5f, 1.79f, 1.6f, 7.8f, 0.9e-6f};
 constexpr LargeModel kBlock256{0.1f, 1.85f, 4.5f, 3.4f, 1.3e-6f}, kBlock128{6.0f, 0.97f, 1.8f, 0.0f, 2.1e-6f};
+
+float medium_limit(float us) { return (us <= 25.0f ? 0.9f : (us <= 100.0f ? 0.78f : 0.74f)) * us; }
 
 float pair_time(int mode, int64_t M, int64_t N, int64_t K) {
   const bool mx = mode == MODE_MX;
@@ -2028,12 +2036,12 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
                       (MODE == MODE_MX || (g.sa_dtype == AYK_F32 && g.sb_dtype == AYK_F32 &&
                                            (!g.sb_vec || aligned16(g.sb)))) &&
                       (g.bias == nullptr || (reinterpret_cast<uintptr_t>(g.bias) & 15) == 0);
-  if (big_ok && !mid_beats(0.9f * pair_time(MODE, g.M, g.N, g.K))) return launch_big<MODE>(g, st, op);
+  if (big_ok && !mid_beats(medium_limit(pair_time(MODE, g.M, g.N, g.K)))) return launch_big<MODE>(g, st, op);
   } else {
     // The 256 x 256 block-scaled kernel from half a round of its tiles on.
     if (g.sa_dtype == AYK_F32 && block256_wanted(g.M, g.N, g.K)) {
       const Block256Args b = block256_args(g);
-      if (block256_supported(b) && !mid_beats(0.9f * block256_time(g.M, g.N, g.K))) return block256_launch(b, st, op);
+      if (block256_supported(b) && !mid_beats(medium_limit(block256_time(g.M, g.N, g.K)))) return block256_launch(b, st, op);
     }
     // The block-scaled 128 x 128 kernel: K % 128 == 0, fp32 activation scales, any float
     // weight-scale dtype, and the same output / bias alignment as above.

@@ -223,3 +223,18 @@ def test_decode_kernel_choice(gpu, recipe, m, n, k, expect):
     out, ref, plan = _run(recipe, m, n, k, True, torch.bfloat16, False, gpu)
     assert plan == expect, plan
     assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("recipe,m,n,k,expect", [
+    ("scaled", 1794, 5888, 10752, "pair tail=1"),   # 115 us, its model just above the medium tiles'
+    ("scaled", 1025, 3072, 1024, "mid 128x128 ring split=1"),
+    ("block", 2328, 3456, 3328, "block256 split=1"),
+    ("mx", 908, 8352, 2048, "pair tail=1"),
+    ("mx", 700, 4096, 2048, "mid 128x128 ring split=1"),
+])
+def test_large_kernel_choice(gpu, recipe, m, n, k, expect):
+    """Prefill shapes at the edge between the 256 x 256 kernels and the medium tiles."""
+    print(f"large choice recipe={recipe} m={m} n={n} k={k}", flush=True)
+    out, ref, plan = _run(recipe, m, n, k, True, torch.bfloat16, recipe == "block", gpu)
+    assert plan == expect, plan
+    assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
