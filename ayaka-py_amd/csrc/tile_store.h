@@ -27,8 +27,10 @@ __device__ inline void stage_slab16(uint8_t* region, int frow, int byte, const f
 }
 
 // The staged slab to rows [m0, m0 + 32) x columns [n0, n0 + TN) of out (clipped to M, N),
-// row by row in 16-byte pieces where the address allows. The region belongs to the
-// wavefront: no barrier, only its own LDS counter.
+// row by row in 16-byte pieces where the address allows, in 8-byte ones where only that does
+// (N % 8 == 4: every other row, whose elements stored one by one cost MXFP8 2048 x 29692 x 288
+// 104 us against 82, 2048 x 7492 x 128 23 against 16). The region belongs to the wavefront: no
+// barrier, only its own LDS counter.
 template <int TN>
 __device__ inline void store_slab16(const uint8_t* region, uint16_t* out, int64_t ldo, int64_t M, int64_t N, int64_t m0,
                                     int64_t n0, int lane) {
@@ -45,8 +47,15 @@ __device__ inline void store_slab16(const uint8_t* region, uint16_t* out, int64_
         __builtin_nontemporal_store(val, reinterpret_cast<slab_chunk*>(p));
       } else {
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
-          if (gn + c < N) p[c] = (uint16_t)((uint32_t)val[c / 2] >> (16 * (c % 2)));
+        for (int q = 0; q < 8; q += 4) {
+          if (gn + q + 4 <= N && (reinterpret_cast<uintptr_t>(p + q) & 7) == 0) {
+            *reinterpret_cast<uint2*>(p + q) = make_uint2((uint32_t)val[q / 2], (uint32_t)val[q / 2 + 1]);
+          } else {
+#pragma unroll
+            for (int c = q; c < q + 4; ++c)
+              if (gn + c < N) p[c] = (uint16_t)((uint32_t)val[c / 2] >> (16 * (c % 2)));
+          }
+        }
       }
     }
   }

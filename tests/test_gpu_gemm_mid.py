@@ -96,9 +96,11 @@ def test_medium_tiles(gpu, recipe, m, n, k, bias, odt, col_major):
 
 
 @pytest.mark.parametrize("recipe,k", [("scaled", 4096), ("block", 4096), ("mx", 4096), ("mx", 1184)])
-def test_medium_tiles_half_outputs(gpu, recipe, k):
-    """16-bit outputs are the fp32 output rounded once (N % 4 != 0: no aligned rows)."""
-    m, n = 97, 642
+@pytest.mark.parametrize("n", [641, 642, 644, 648])
+def test_medium_tiles_half_outputs(gpu, recipe, k, n):
+    """16-bit outputs are the fp32 output rounded once, whatever part of their rows is aligned
+    (16 bytes for N % 8 == 0, 8 for every other row of N % 8 == 4)."""
+    m = 97
     full, _, plan = _run(recipe, m, n, k, False, torch.float32, False, gpu)
     for odt in (torch.bfloat16, torch.float16):
         half, _, plan2 = _run(recipe, m, n, k, False, odt, False, gpu)
