@@ -1508,10 +1508,13 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
   }
   if (M >= 2 && ldx % 8 == 0) {
     const SkinnyPlan p = skinny_plan(M, N, K, block_size_x);
-    // From 17 rows the tiled kernel is faster on weights past 9 MB (M = 32: 2432 x 3968 14.0
-    // -> 13.0 us, 3840 x 3200 15.8 -> 12.8, 6656 x 18560 48.2 -> 34.3; 1920 x 3200 11.8 against
-    // 12.0); up to 16 rows this one is (M = 16: 6656 x 18560 28.7 against 30.7).
-    if (p.ok && !(tile_ok && M > 16 && N * K > 9000000)) {
+    // From 25 rows the tiled kernel is faster on per-row scales and weights past 9 MB of 1536
+    // rows or more (M = 32: 3840 x 3200 15.8 -> 12.8 us, 6656 x 18560 48.2 -> 34.3, 5888 x 24960
+    // 55.8 -> 43.3). Up to 24 rows neither is throughout (M = 19: 20096 x 640 12.1 -> 9.7; M = 17:
+    // 3712 x 20864 24.9 -> 27.0, 1536 x 21120 16.9 -> 22.0), on narrower weights its 128-row tiles
+    // leave too few pieces (M = 31: 583 x 27520 17.6 -> 26.8), and block scales cost it more (M =
+    // 19: 24448 x 1920 22.7 -> 31.5; M = 32: 1024 x 22656 17.8 -> 29.4; half of 66 shapes lose).
+    if (p.ok && !(tile_ok && M > 24 && N >= 1536 && N * K > 9000000 && block_size_x >= K)) {
       SkinnyArgs a{};
       a.x = g.x; a.ldx = ldx; a.M = M; a.w = g.w; a.ldw = ldw; a.N = N; a.K = K;
       a.scale = scale; a.scale_dtype = scale_dtype; a.srs = scale_row_stride; a.by = block_size_y; a.bx = block_size_x;

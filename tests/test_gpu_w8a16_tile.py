@@ -32,6 +32,26 @@ def _operands(m, n, k, xdt, by, bx, sdt, dev):
     return x.to(dev), w.to(dev), scale.to(dev), full.to(dev)
 
 
+def _check(m, n, k, xdt, by, bx, sdt, dev):
+    """One call within the bound; returns its recorded plan."""
+    from ayaka.kernel.hip import _lib, fp8_weight_only_gemm
+
+    bx = k if bx is None else bx
+    print(f"w8a16 m={m} n={n} k={k} x={xdt} by={by} bx={bx} scale={sdt}", flush=True)
+    x, w, scale, full = _operands(m, n, k, xdt, by, bx, sdt, dev)
+    y = fp8_weight_only_gemm(x, w, scale, scale.shape[1], by, bx, sdt).double()
+    plan = _lib.last_plan()
+    ws = w.double() * full
+    ref, mag = x.double() @ ws.t(), x.double().abs() @ ws.abs().t()
+    u = UNIT[xdt]
+    bound = u * ref.abs() + (u + (k + 2) * 2.0**-24) * mag
+    if xdt == torch.float16:
+        bound = bound + 2.0**-25 * x.double().abs().sum(1, keepdim=True)
+    worst = ((y - ref).abs() / bound.clamp_min(1e-30)).max().item()
+    assert worst <= 1.01, worst  # 1% for second-order terms
+    return plan
+
+
 @pytest.mark.parametrize("m,n,k,xdt,by,bx,sdt,plan", [
     (33, 129, 16, torch.bfloat16, 1, None, "float32", "128x64 split=1"),      # one short stage
     (64, 128, 64, torch.float16, 1, None, "float32", "128x64 split=1"),       # exact tile and stage
@@ -48,22 +68,22 @@ def _operands(m, n, k, xdt, by, bx, sdt, dev):
     (2049, 8200, 576, torch.float16, 1, None, "float32", "split=1"),
 ])
 def test_weight_only_gemm_tile(gpu, m, n, k, xdt, by, bx, sdt, plan):
-    from ayaka.kernel.hip import _lib, fp8_weight_only_gemm
-
-    bx = k if bx is None else bx
-    print(f"w8a16 tile m={m} n={n} k={k} x={xdt} by={by} bx={bx} scale={sdt}", flush=True)
-    x, w, scale, full = _operands(m, n, k, xdt, by, bx, sdt, gpu)
-    y = fp8_weight_only_gemm(x, w, scale, scale.shape[1], by, bx, sdt).double()
-    got = _lib.last_plan()
+    got = _check(m, n, k, xdt, by, bx, sdt, gpu)
     assert got.startswith("w8a16 tile") and plan in got, got
-    ws = w.double() * full
-    ref, mag = x.double() @ ws.t(), x.double().abs() @ ws.abs().t()
-    u = UNIT[xdt]
-    bound = u * ref.abs() + (u + (k + 2) * 2.0**-24) * mag
-    if xdt == torch.float16:
-        bound = bound + 2.0**-25 * x.double().abs().sum(1, keepdim=True)
-    worst = ((y - ref).abs() / bound.clamp_min(1e-30)).max().item()
-    assert worst <= 1.01, worst  # 1% for second-order terms
+
+
+@pytest.mark.parametrize("m,n,k,bx,plan", [
+    (32, 3840, 3200, None, "w8a16 tile 128x64 split=6"),
+    (25, 3840, 3200, None, "w8a16 tile 128x64 split=6"),
+    (24, 3840, 3200, None, "w8a16 skinny split=13"),
+    (31, 640, 14464, None, "w8a16 skinny split=57"),  # few 128-row tiles
+    (32, 3840, 3200, 128, "w8a16 skinny split=13"),   # block scales
+])
+def test_weight_only_gemm_decode_choice(gpu, m, n, k, bx, plan):
+    """Batches of 17 to 32 rows whose K only the skinny kernel or the tiled one takes (an odd
+    multiple of 128), at the edges of the rule between the two."""
+    got = _check(m, n, k, torch.bfloat16, 1 if bx is None else 128, bx, "float32", gpu)
+    assert got == plan, got
 
 
 def test_weight_only_gemm_tile_all_codes_and_special_scales(gpu):
