@@ -414,19 +414,6 @@ __device__ inline void load_bias4(const GemmArgs& g, int64_t n, float* b) {
   }
 }
 
-template <int OUT>
-__device__ inline void store4_typed(const GemmArgs& g, int64_t m, int64_t n, const float* v) {
-  if (OUT == AYK_F32) {
-    *reinterpret_cast<float4*>(reinterpret_cast<float*>(g.out) + m * g.ldo + n) = make_float4(v[0], v[1], v[2], v[3]);
-  } else {
-    uint16_t b[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) b[i] = OUT == AYK_BF16 ? f32_to_bf16_bits(v[i]) : f32_to_f16_bits(v[i]);
-    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.out) + m * g.ldo + n) =
-        make_uint2((uint32_t)b[0] | ((uint32_t)b[1] << 16), (uint32_t)b[2] | ((uint32_t)b[3] << 16));
-  }
-}
-
 // Epilogue of the large-tile kernel, staged through LDS (free once the K loop ends).
 // A lane's accumulators hold 4 consecutive n of one row m per store group, spread over
 // 32 rows per instruction; writing them straight to HBM costs one cache line per lane
@@ -1871,10 +1858,10 @@ int launch_block_big(GemmArgs g, hipStream_t st, const char* op) {
 }
 
 // The general kernel, for operands whose row strides leave the medium tiles' 32-bit
-// offsets and the shapes of general_wanted: tiles of 32, 64 or 128 activation rows and a K split. With 128-row tiles and no
-// split alone, a decode batch leaves most CUs idle (activation rows 8 MiB apart: per-row
-// 4096 x 14464, M = 16, 138 us against 21; block 4096 x 4096, M = 16, 57 against 13; MXFP8
-// 4096 x 4224, M = 128, 51 against 26).
+// offsets and the shapes of general_wanted: tiles of 32, 64 or 128 activation rows and a K
+// split. With 128-row tiles and no split alone, a decode batch leaves most CUs idle
+// (activation rows 8 MiB apart: per-row 4096 x 14464, M = 16, 138 us against 21; block 4096 x
+// 4096, M = 16, 57 against 13; MXFP8 4096 x 4224, M = 128, 51 against 26).
 template <int MODE, int BM, int WN, int WM>
 int launch_cfg(GemmArgs g, hipStream_t st, const char* op) {
   constexpr int kBn = 128;

@@ -9,11 +9,11 @@
 //  * 256 x 256 (eight wavefronts), 128 x 128, 128 x 64 and 64 x 64 (four) tiles on
 //    v_mfma_scale_f32_32x32x64_f8f6f4, weight = operand A: a lane's accumulator column is
 //    one activation row.
-//  * Direct-to-LDS loads (8 rows x 128 bytes an instruction) into a ring of two to four
+//  * Direct-to-LDS loads (8 rows x 128 bytes an instruction) into a ring of two or four
 //    128-K stage buffers. Two buffers leave room for several workgroups a CU, which run
-//    while one waits at its stage barrier (throughput, the larger batches); three or four
-//    hide the latency of a stage inside one workgroup (few tiles a CU, long K), which also
-//    saves most K splits.
+//    while one waits at its stage barrier (throughput, the larger batches); four hide the
+//    latency of a stage inside one workgroup (few tiles a CU, long K), which also saves
+//    most K splits.
 //  * A K tail is zero-filled by the loads' bounds check, so any K % 16 == 0 takes the same
 //    loop; rows past M and N likewise.
 //  * Block scales: a 128-K stage is one scale block; its two MFMAs start from zero and one
@@ -83,11 +83,10 @@ __global__ __launch_bounds__(WN * WM * 64, WGS) void fp8_mid_kernel(MidArgs g, i
   constexpr int kWords = scale_words(MODE), kWordRows = 64 * kWaves;  // each wavefront loads 64 rows' words
   constexpr int kOps = kWDma + kADma + kWords, kBuf = kStage + kWordRows * 4 * kWords;
   static_assert(kRows <= kWordRows, "a lane a row");
-  static_assert(MODE != kMidMx || D != 3, "whole rings in a chunk of four stages");
-  static_assert(D >= 2 && D <= 4 && (D - 2) * kOps <= 63, "stage buffers, vmcnt range");
+  static_assert((D == 2 || D == 4) && (D - 2) * kOps <= 63, "whole rings in a chunk of four stages; vmcnt range");
   // Distinct LDS objects with compile-time names, so that the compiler keeps the loads in
   // flight to one apart from the reads of another.
-  __shared__ __attribute__((aligned(1024))) uint8_t B0[kBuf], B1[kBuf], B2[D > 2 ? kBuf : 16], B3[D > 3 ? kBuf : 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t B0[kBuf], B1[kBuf], B2[D == 4 ? kBuf : 16], B3[D == 4 ? kBuf : 16];
   constexpr bool kChunks = MODE == kMidMx;
   __shared__ __attribute__((aligned(1024))) uint8_t chunk[kChunks ? kWordRows * 16 : 16];
   __shared__ float col_scale[BN], col_bias[BN];
@@ -459,8 +458,7 @@ struct MidModel {
 };
 constexpr MidModel kModels[3] = {
     {{1.25f, 0.44f, 0.32f, 0.50f, 0.27f, 0.19f}, {1.25f, 0.71f, 0.52f, 0.32f, 0.34f, 0.20f}, 9.0f, 2.9f, 3.4f, 1.68e-6f, 8.0e-8f},
-    // (128 x 64 ring: three buffers, two workgroups a CU)
-    {{0.0f, 0.57f, 0.36f, 0.0f, 0.37f, 0.25f}, {0.0f, 0.99f, 0.74f, 0.0f, 0.545f, 0.33f}, 4.6f, 4.2f, 2.8f, 1.95e-6f, 7.0e-8f},
+    {{0.0f, 0.57f, 0.36f, 0.0f, 0.0f, 0.25f}, {0.0f, 0.99f, 0.74f, 0.0f, 0.0f, 0.33f}, 4.6f, 4.2f, 2.8f, 1.95e-6f, 7.0e-8f},
     {{1.71f, 0.55f, 0.37f, 0.33f, 0.37f, 0.22f}, {1.40f, 0.70f, 0.54f, 0.56f, 0.39f, 0.24f}, 3.8f, 2.8f, 3.5f, 1.92e-6f, 9.0e-8f}};
 constexpr int kSplits[8] = {1, 2, 3, 4, 6, 8, 12, 16};
 constexpr int kMinSplitK = 512;
@@ -479,12 +477,11 @@ MidPlan mid_plan(MidMode mode, int64_t M, int64_t N, int64_t K, bool may_split) 
   for (int c = 0; c < kConfigs; ++c) {
     if (m.tau[c] == 0.0f) continue;
     const MidTile& t = kTiles[c];
-    const int resident = mode == kMidBlock && c == 4 ? 2 : t.resident;
     const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
     for (const int s : kSplits) {
       // INT8 never splits: a partial would leave the exact int32 sum.
       if (s > 1 && (!may_split || mode == kMidInt8 || K < (int64_t)kMinSplitK * s)) break;
-      const float u = (float)cdiv(tiles * s, kCus), rounds = (float)cdiv(cdiv(tiles * s, kCus), resident);
+      const float u = (float)cdiv(tiles * s, kCus), rounds = (float)cdiv(cdiv(tiles * s, kCus), t.resident);
       const float stage = rounds * m.lambda[c] > u * m.tau[c] ? rounds * m.lambda[c] : u * m.tau[c];
       float us = m.base + m.cold * (float)N * (float)K + (float)cdiv(cdiv(K, kStageK), s) * stage + m.store * u * (float)(t.bn * t.bm) / 65536.0f;
       if (s > 1) us += m.reduce + m.partial * (float)s * (float)M * (float)N;
@@ -512,7 +509,6 @@ void launch_tile(const MidArgs& g, const MidPlan& p, int64_t kps, hipStream_t st
     switch (p.config) {
       case 1: AYK_MID(128, 128, 2, 2, 2, 2); break;
       case 2: AYK_MID(128, 64, 2, 2, 2, 2); break;
-      case 4: AYK_MID(128, 64, 2, 2, 3, 2); break;
       default: AYK_MID(64, 64, 2, 2, 4, 2); break;
     }
   } else {

@@ -1476,7 +1476,7 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
   g.out = static_cast<uint16_t*>(out);
   g.ldo = ldo;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // Decode batch sizes (all three need 16-byte aligned activation rows): wide
+  // Decode batch sizes (all three need the 16-byte aligned activation rows checked above): wide
   // projections take the stream kernel (K a multiple of 512, scale blocks of whole
   // 16 K), the others the row-stream kernel (whole 256-K stages, scale blocks of whole
   // 16 K), else the skinny streaming kernel (whole 128-K steps, scale blocks of >= 32 K).
@@ -1484,7 +1484,7 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
                       out, ldo, static_cast<float*>(workspace), workspace_bytes};
   const bool tile_ok = w16_tile_supported(t);
   auto tile_beats = [&](float us) { return tile_ok && w16_tile_time(M, N, K) < 0.75f * us; };
-  if (M >= 2 && ldx % 8 == 0) {
+  if (M >= 2) {
     const StPlan sp = stream_plan(M, N, K, block_size_x);
     if (sp.ok && !tile_beats(stream_time(sp, N, K))) {
       RsArgs a{};
@@ -1495,7 +1495,7 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
                                  : launch_stream<false>(sp, a, workspace_bytes, st);
     }
   }
-  if (M >= 2 && ldx % 8 == 0) {
+  if (M >= 2) {
     const RsPlan rp = rows_plan(M, N, K, block_size_x);
     if (rp.ok && !tile_beats(rows_time(rp, N, K))) {
       RsArgs a{};
@@ -1506,7 +1506,7 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
                                  : launch_rows<false>(rp, a, workspace_bytes, st);
     }
   }
-  if (M >= 2 && ldx % 8 == 0) {
+  if (M >= 2) {
     const SkinnyPlan p = skinny_plan(M, N, K, block_size_x);
     // From 25 rows the tiled kernel is faster on per-row scales and weights past 9 MB of 1536
     // rows or more (M = 32: 3840 x 3200 15.8 -> 12.8 us, 6656 x 18560 48.2 -> 34.3, 5888 x 24960

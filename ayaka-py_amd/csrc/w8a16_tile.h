@@ -1,4 +1,4 @@
-// W8A16 GEMM for M > 32 on gfx950: out[M, N] = x[M, K] . dequant(w[N, K])^T with e4m3
+// W8A16 GEMM of any M on gfx950: out[M, N] = x[M, K] . dequant(w[N, K])^T with e4m3
 // weights, 16-bit activations and fp32 accumulation, LDS-tiled on
 // v_mfma_f32_32x32x16_{bf16,f16}. The launcher that w8a16.hip's dispatch calls.
 #pragma once
