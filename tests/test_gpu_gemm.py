@@ -99,10 +99,12 @@ def test_blockwise_gemv(gpu, n, k):
 # ------------------------------------------------------------------ W8A8 GEMMs
 MNK = [(8, 3072, 1024), (17, 300, 256), (64, 256, 384), (200, 1000, 1024), (256, 512, 2048), (129, 130, 528),
        (300, 520, 1024), (513, 772, 2048), (1024, 1024, 3584),
-       # 256x256 kernel with 1, 5 and 19 K stages of 64: steps padded to a multiple of four
-       (256, 256, 64), (400, 300, 320), (260, 1028, 1216),
-       # its 128-byte-row variant (K % 128 == 0) with 1 and 3 pairs of stages: pairs padded to even
-       (256, 260, 128), (512, 512, 384),  # from (300, 520, 1024) on: the 256x256 kernels
+       # up to here and with these (few 256x256 tiles) the decode kernel and the medium tiles
+       (256, 256, 64), (400, 300, 320), (260, 1028, 1216), (256, 260, 128), (512, 512, 384),
+       # 256x256 kernel with 1, 5 and 17 K stages of 64: steps padded to a multiple of four
+       (258, 13264, 64), (2304, 8192, 320), (516, 13264, 1088),
+       # its 128-byte-row variant (K % 128 == 0) with 1 and 5 pairs of stages: pairs padded to even
+       (258, 8016, 128), (2304, 8192, 640),
        # K splits whose N is not a multiple of 4: the one-element-per-thread reduce
        (300, 1002, 8192), (40, 1002, 8192)]
 
@@ -129,11 +131,12 @@ def test_fp8_scaled_mm(gpu, m, n, k, rowwise):
 
 
 @pytest.mark.parametrize("m,n,k,rowwise,out_dtype", [
-    (512, 3584, 18944, True, torch.bfloat16),   # 256x256 pair kernel, 28 tiles: 15 K splits
-    (300, 520, 4096, False, torch.float16),     # pair kernel, ragged M / N, per-tensor scales
-    (128, 1024, 4096, True, torch.float32),     # general kernel (128-row tiles)
-    (40, 768, 8192, True, torch.bfloat16),      # general kernel (64-row tiles)
-    (8, 3584, 18944, False, torch.bfloat16),    # general kernel (32-row tiles), last split shorter
+    (512, 3584, 18944, True, torch.bfloat16),   # 256x256 pair kernel, 28 tiles: 8 K pieces, the last one shorter
+    (300, 3608, 8192, False, torch.float16),    # pair kernel, ragged M / N, per-tensor scales
+    (300, 520, 4096, False, torch.float16),     # medium tiles
+    (128, 1024, 4096, True, torch.float32),
+    (40, 768, 8192, True, torch.bfloat16),      # decode kernel
+    (8, 3584, 18944, False, torch.bfloat16),
 ])
 def test_fp8_scaled_mm_split_k(gpu, m, n, k, rowwise, out_dtype):
     """Launches short of one round of tiles split K: scaled fp32 partials in the workspace
@@ -154,10 +157,12 @@ def test_fp8_scaled_mm_split_k(gpu, m, n, k, rowwise, out_dtype):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (512, 2048, 4096),   # 256x256 pair kernel: 16 tiles, 4 splits of 1024 K (whole code chunks)
-    (300, 520, 8704),    # pair kernel, ragged M / N, 17 chunks of 512 K: the last split shorter
-    (64, 1024, 8192),    # general kernel, 64-row tiles
-    (5, 768, 4096),      # general kernel, 32-row tiles
+    (258, 3608, 7168),   # 256x256 pair kernel: 7 splits of 1024 K (whole code chunks), ragged M / N
+    (258, 1672, 20992),  # pair kernel, 41 chunks of 512 K: the last split shorter
+    (512, 2048, 4096),   # medium tiles
+    (300, 520, 8704),
+    (64, 1024, 8192),    # decode kernel
+    (5, 768, 4096),
 ])
 def test_mxfp8_scaled_mm_split_k(gpu, m, n, k):
     """MXFP8 launches short of one round of tiles split K; each split reads its UE8M0
@@ -280,9 +285,10 @@ def test_decode_batch_scales_not_16_byte_aligned(gpu):
 
 
 @pytest.mark.parametrize("m,n,k,rowwise,with_bias", [(2048, 4096, 1024, True, True), (1300, 11712, 1536, False, False),
-                                                    (4096, 37888, 512, True, False)])
+                                                    (4096, 37888, 512, True, False), (1300, 11712, 3072, True, True)])
 def test_fp8_scaled_mm_half_outputs_are_the_fp32_result_rounded(gpu, m, n, k, rowwise, with_bias):
-    """The 16-bit outputs of the 256 x 256 kernel are its fp32 result rounded once to
+    """The 16-bit outputs of the medium tiles and (the last two shapes) of the 256 x 256 pair
+    kernel, its tail split's reduce included, are the fp32 result rounded once to
     nearest even (torch's cast), bit for bit: no step of the epilogue may fold a multiply
     into the conversion (one rounding of the exact product differs at fp16 ties)."""
     from ayaka.kernel.hip import fp8_scaled_mm
@@ -302,18 +308,20 @@ def test_fp8_scaled_mm_half_outputs_are_the_fp32_result_rounded(gpu, m, n, k, ro
         assert torch.equal(y.view(torch.int16), y32.to(dt).view(torch.int16)), f"{dt} output is not the rounded fp32 result"
 
 
-# 276 tiles of 256 x 256: one whole round, then a last round of 20 tiles that the pair
-# kernel splits over K (three 512-K pieces each) into the workspace, ragged M and N.
-TAIL_MNK = (1300, 11712, 1536)
+# One whole round of 256 x 256 tiles, then a last round of 20 or 4 tiles that the pair kernel
+# splits over K (pieces of 512 K) into the workspace, ragged M and N. The first shape has the
+# split's workspace, but the medium tiles are faster on it.
+TAIL_MNK = [(1300, 11712, 1536, 3 * 20, "mid 128x128 split=1"), (1300, 11712, 3072, 6 * 20, "pair tail=6"),
+            (258, 33136, 1536, 3 * 4, "pair tail=3")]
 
 
+@pytest.mark.parametrize("m,n,k,pieces,plan", TAIL_MNK)
 @pytest.mark.parametrize("rowwise,out_dtype", [(True, torch.bfloat16), (False, torch.float16), (True, torch.float32)])
-def test_fp8_scaled_mm_tail_split(gpu, rowwise, out_dtype):
+def test_fp8_scaled_mm_tail_split(gpu, m, n, k, pieces, plan, rowwise, out_dtype):
     from ayaka.kernel.hip import _lib, fp8_scaled_mm
 
-    m, n, k = TAIL_MNK
     _say(f"fp8_scaled_mm tail split m={m} n={n} k={k} rowwise={rowwise} out={out_dtype}")
-    assert _lib.query("ayk_fp8_scaled_mm_workspace_bytes", m, n, k) == 3 * 20 * 256 * 256 * 4, "tail split expected"
+    assert _lib.query("ayk_fp8_scaled_mm_workspace_bytes", m, n, k) == pieces * 256 * 256 * 4, "tail split expected"
     a = _fp8((m, k), seed=41, scale=40)
     w = _fp8((n, k), seed=42, scale=40)
     sa = (torch.rand(m, generator=_gen(43)) * 0.01 + 1e-3) if rowwise else torch.tensor(0.004)
@@ -322,15 +330,16 @@ def test_fp8_scaled_mm_tail_split(gpu, rowwise, out_dtype):
     ref = ora.fp8_scaled_mm(a, w, sa, sb, bias)
     out = torch.empty(m, n, dtype=out_dtype, device=gpu)
     fp8_scaled_mm(a.to(gpu), w.to(gpu).t(), sa.to(gpu), sb.to(gpu), bias.to(gpu), out=out)
+    assert _plan() == plan, _plan()
     assert_linear_close(out, ref, "fp8_scaled_mm tail split")
 
 
-def test_mxfp8_scaled_mm_tail_split(gpu):
+@pytest.mark.parametrize("m,n,k,pieces,plan", TAIL_MNK)
+def test_mxfp8_scaled_mm_tail_split(gpu, m, n, k, pieces, plan):
     from ayaka.kernel.hip import _lib, mxfp8_scaled_mm
 
-    m, n, k = TAIL_MNK
     _say(f"mxfp8_scaled_mm tail split m={m} n={n} k={k}")
-    assert _lib.query("ayk_mxfp8_scaled_mm_workspace_bytes", m, n, k) == 3 * 20 * 256 * 256 * 4, "tail split expected"
+    assert _lib.query("ayk_mxfp8_scaled_mm_workspace_bytes", m, n, k) == pieces * 256 * 256 * 4, "tail split expected"
     torch.manual_seed(46)
     x = torch.distributions.StudentT(3.0).sample((m, k))
     wf = torch.randn(n, k, generator=_gen(47))
@@ -340,16 +349,19 @@ def test_mxfp8_scaled_mm_tail_split(gpu):
     ref = ora.mxfp8_scaled_mm(qa, ca, qw, cw, bias)
     y = mxfp8_scaled_mm(qa.to(gpu), ca.to(gpu), qw.to(gpu), cw.to(gpu), bias.to(gpu),
                         out=torch.empty(m, n, dtype=torch.bfloat16, device=gpu))
+    assert _plan() == plan, _plan()
     assert_linear_close(y, ref, "mxfp8_scaled_mm tail split")
 
 
 @pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16, torch.float32])
-def test_fp8_scaled_mm_big_tile_strided_out(gpu, out_dtype):
-    """256x256-tile kernel: every output dtype, a padded output row stride, M/N tails."""
+@pytest.mark.parametrize("m,n,k,plan", [(520, 1284, 1280, "mid 64x64 ring split=1"), (520, 16388, 1280, "pair tail=1"),
+                                        (516, 13252, 1088, "big")])
+def test_fp8_scaled_mm_big_tile_strided_out(gpu, out_dtype, m, n, k, plan):
+    """256x256-tile kernels (and a shape that the medium tiles take): every output dtype, a
+    padded output row stride, M/N tails."""
     from ayaka.kernel.hip import fp8_scaled_mm
 
-    m, n, k = 520, 1284, 1280
-    _say(f"fp8_scaled_mm big tile out={out_dtype}")
+    _say(f"fp8_scaled_mm big tile m={m} n={n} k={k} out={out_dtype}")
     a = _fp8((m, k), seed=21, scale=40)
     w = _fp8((n, k), seed=22, scale=40)
     sa = torch.rand(m, generator=_gen(1)) * 0.01 + 1e-3
@@ -359,6 +371,7 @@ def test_fp8_scaled_mm_big_tile_strided_out(gpu, out_dtype):
     buf = torch.full((m, n + 12), 7.0, dtype=out_dtype, device=gpu)  # row stride n + 12
     out = buf[:, :n]
     fp8_scaled_mm(a.to(gpu), w.to(gpu).t(), sa.to(gpu), sb.to(gpu), bias.to(gpu), out=out)
+    assert _plan() == plan, _plan()
     assert_linear_close(out, ref, f"big tile {out_dtype}")
     assert torch.all(buf[:, n:].float() == 7.0), "wrote past the output columns"
 
@@ -380,6 +393,7 @@ def test_fp8_scaled_mm_many_tiles(gpu, k, rowwise, with_bias):
     ref = ora.fp8_scaled_mm(a, w, sa, sb, bias)
     out = torch.empty(m, n, dtype=torch.bfloat16, device=gpu)
     fp8_scaled_mm(a.to(gpu), w.to(gpu).t(), sa.to(gpu), sb.to(gpu), None if bias is None else bias.to(gpu), out=out)
+    assert _plan() == ("pair tail=1" if k % 128 == 0 else "big"), _plan()
     assert_linear_close(out, ref, "many tiles bf16")
     # A second call into the same buffer (every tile is rewritten).
     out.fill_(float("nan"))
@@ -427,6 +441,7 @@ BLOCK256 = [
     (2304, 4352, 384, False, torch.float16, torch.float16, True),
     (2048, 4096, 8192, False, torch.float32, torch.bfloat16, True),   # 128 tiles: K split 2
     (512, 2304, 7040, True, torch.float32, torch.bfloat16, True),     # 18 tiles: 6 K pieces, the last 5 blocks of 10
+    (258, 2184, 7296, False, torch.float32, torch.float32, False),    # 18 tiles, ragged: 7 pieces, the last 3 blocks of 9
     (4096, 2048, 256, True, torch.float32, torch.bfloat16, False),    # two blocks, one pair
 ]
 
@@ -449,16 +464,17 @@ def test_fp8_blockwise_mm_256(gpu, m, n, k, col_major, sdt, out_dtype, with_bias
     out = torch.empty(m, n, dtype=out_dtype, device=gpu)
     fp8_blockwise_mm(a.to(gpu), w.to(gpu), sa_arg.to(gpu), sb.to(gpu), bias.to(gpu) if bias is not None else None,
                      out=out, a_scale_col_major=col_major)
+    assert _plan().startswith("block256"), _plan()
     assert_linear_close(out, ref, "blockwise_mm 256-tile")
 
 
-def test_fp8_blockwise_mm_256_scale_edges(gpu):
+@pytest.mark.parametrize("m,n,k,plan", [(2048, 4096, 1024, "mid 128x128 split=1"), (2304, 4352, 1024, "block256 split=1")])
+def test_fp8_blockwise_mm_256_scale_edges(gpu, m, n, k, plan):
     """Zero weight-block scales add nothing (the MFMA exponent code 0 weighs a block's
     products by 2^-127), and a NaN scale poisons exactly the outputs whose sums include it,
     as in the oracle."""
     from ayaka.kernel.hip import fp8_blockwise_mm
 
-    m, n, k = 2048, 4096, 1024
     _say(f"fp8_blockwise_mm 256-tile scale edges m={m} n={n} k={k}")
     kb, nb = k // 128, n // 128
     a = _fp8((m, k), seed=31, scale=30)
@@ -471,6 +487,7 @@ def test_fp8_blockwise_mm_256_scale_edges(gpu):
     ref = ora.fp8_blockwise_mm(a, w, sa, sb)
     out = torch.empty(m, n, dtype=torch.float32, device=gpu)
     fp8_blockwise_mm(a.to(gpu), w.to(gpu), sa.to(gpu), sb.to(gpu), out=out)
+    assert _plan() == plan, _plan()
     y = out.cpu()
     assert torch.equal(torch.isnan(y), torch.isnan(ref))
     keep = ~torch.isnan(ref)
@@ -479,19 +496,20 @@ def test_fp8_blockwise_mm_256_scale_edges(gpu):
 
 
 @pytest.mark.parametrize("m,n,k,col_major,sdt,with_bias", [
-    (32, 1024, 4096, False, torch.float16, True),     # K split 4
-    (200, 768, 8192, True, torch.bfloat16, True),     # split 8, column-major activation scales
-    (7, 256, 2048, False, torch.float16, False),      # split 2, 7 rows
-    (256, 2048, 7168, False, torch.float32, False),   # DeepSeek-V3 K, split 4
-    (32, 7168, 18432, False, torch.bfloat16, True),   # DeepSeek-V3 (7168, 18432) at M = 32, split 16
-    (16, 64, 4096, False, torch.float16, False),      # N < 128: general kernel split 4
-    (40, 96, 8192, True, torch.bfloat16, True),       # N < 128, 64-row tiles: split 8
+    (32, 1024, 4096, False, torch.float16, True),
+    (200, 768, 8192, True, torch.bfloat16, True),     # column-major activation scales
+    (7, 256, 2048, False, torch.float16, False),      # 7 rows
+    (256, 2048, 7168, False, torch.float32, False),   # DeepSeek-V3 K
+    (32, 7168, 18432, False, torch.bfloat16, True),   # DeepSeek-V3 (7168, 18432) at M = 32
+    (16, 64, 4096, False, torch.float16, False),      # N < 128
+    (40, 96, 8192, True, torch.bfloat16, True),       # N < 128
+    (258, 516, 16384, True, torch.bfloat16, True),    # 128 x 128 kernel, split 16
 ])
 def test_fp8_blockwise_mm_split_k(gpu, m, n, k, col_major, sdt, with_bias):
-    """Launches with too few 128 x 128 tiles split K over fp32 partials (the workspace the
-    wrapper allocates from the size query) and reduce them in a fixed order. (Up to 64
-    rows with fp32 weight scales take the decode-batch kernel instead: 16-bit weight scales
-    here keep these on the general kernel.)"""
+    """Launches with too few tiles split K over fp32 partials (the workspace the wrapper
+    allocates from the size query) and reduce them in a fixed order. (Up to 64 rows with fp32
+    weight scales take the decode-batch kernel instead: 16-bit weight scales here keep these
+    on the medium tiles.)"""
     from ayaka.kernel.hip import _lib, fp8_blockwise_mm
 
     _say(f"fp8_blockwise_mm split-K m={m} n={n} k={k} col_major={col_major} sdt={sdt} bias={with_bias}")
@@ -627,10 +645,11 @@ def test_block128_default_bf16_scales_reach_decode_batch_kernel(gpu, m):
 
 @pytest.mark.parametrize("m,n,k", [(1, 512, 1024), (1, 1000, 8192), (64, 256, 512), (100, 300, 1024), (512, 512, 2048), (33, 96, 96),
                                    (300, 520, 1024), (777, 1028, 2048),
-                                   # 256x256 kernels: codes staged in chunks of four 128-K pairs
-                                   # (K % 512 == 0; three chunks, M / N tails, 288 tiles) and the
-                                   # 128-K-stage kernel for other K % 128 == 0
-                                   (520, 1040, 1536), (2304, 8192, 1024), (512, 512, 640)])
+                                   # medium tiles: codes staged in chunks of four 128-K stages
+                                   # (K % 512 == 0, three chunks, M / N tails) and one by one
+                                   (520, 1040, 1536), (512, 512, 640),
+                                   # the same chunks in the 256x256 kernel (three and two)
+                                   (520, 16392, 1536), (2304, 8192, 1024)])
 def test_mxfp8_scaled_mm(gpu, m, n, k):
     from ayaka.kernel.hip import mxfp8_scaled_mm
 
@@ -647,9 +666,11 @@ def test_mxfp8_scaled_mm(gpu, m, n, k):
     assert_linear_close(out, ref, "mxfp8_scaled_mm")
 
 
-# Kernel routes for the code-edge cases: M = 1 GEMV, general kernel, 256 x 256 pair
-# kernel unsplit and split over K, and the 128-K-stage kernel (K % 512 != 0).
-MX_EDGE = [(1, 512, 2048), (100, 300, 1024), (1024, 1024, 512), (512, 2048, 4096), (512, 512, 640)]
+# Kernel routes for the code-edge cases: M = 1 GEMV, medium tiles (whole code chunks, and
+# K % 512 != 0), 256 x 256 pair kernel unsplit and split over K.
+MX_EDGE = [(1, 512, 2048), (100, 300, 1024), (1024, 1024, 512), (512, 2048, 4096), (512, 512, 640),
+           (258, 21904, 512), (258, 3608, 7168)]
+MX_EDGE_PLAN = {(258, 21904, 512): "pair tail=1", (258, 3608, 7168): "pair split=7"}
 
 
 def _mx_edge_operands(m, n, k):
@@ -684,6 +705,7 @@ def test_mxfp8_code_zero_weight_scales(gpu, m, n, k):
     assert torch.equal(ref[:, 3], bias[3].expand(m)), "oracle: a code-0 row contributes exactly 0"
     out = torch.empty(m, n, dtype=torch.float32, device=gpu)
     mxfp8_scaled_mm(qa.to(gpu), ca.to(gpu), qw.to(gpu), cw.to(gpu), bias.to(gpu), out=out)
+    assert _plan() == MX_EDGE_PLAN.get((m, n, k), _plan()), _plan()
     assert_linear_close(out, ref, "mxfp8 code-0 weight scales")
     assert (out[:, 3].cpu() - bias[3]).abs().max().item() < 1e-20
 
@@ -702,6 +724,7 @@ def test_mxfp8_code_ff_scales_give_nan(gpu, m, n, k):
     ref = ora.mxfp8_scaled_mm(qa, ca, qw, cw)
     out = torch.empty(m, n, dtype=torch.float32, device=gpu)
     mxfp8_scaled_mm(qa.to(gpu), ca.to(gpu), qw.to(gpu), cw.to(gpu), out=out)
+    assert _plan() == MX_EDGE_PLAN.get((m, n, k), _plan()), _plan()
     y = out.cpu()
     nan_ref = torch.isnan(ref)
     assert nan_ref[:, 5].all() and nan_ref[m // 2, :].all()
@@ -988,8 +1011,9 @@ def _i8(shape, seed):
     return torch.randint(-128, 128, shape, generator=_gen(seed), dtype=torch.int8)
 
 
-INT8_MNK = [(8, 3072, 1024), (17, 300, 256), (200, 1000, 1040),  # general kernel (K % 64 != 0 included)
-            (300, 520, 1024), (400, 300, 320), (260, 1028, 1216), (2304, 8192, 640)]  # 256x256 kernels
+INT8_MNK = [(8, 3072, 1024), (17, 300, 256), (200, 1000, 1040),  # medium tiles (K % 64 != 0 included)
+            (300, 520, 1024), (400, 300, 320), (260, 1028, 1216),
+            (2304, 8192, 640), (520, 16392, 1216)]  # 256x256 kernels, K % 128 == 0 and 64
 
 
 @pytest.mark.parametrize("m,n,k", INT8_MNK)

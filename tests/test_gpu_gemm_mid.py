@@ -12,7 +12,7 @@ FP8 = torch.float8_e4m3fn
 
 
 def _fp8(shape, g):
-    return (torch.randn(shape, generator=g) * 50).clamp(-448, 448).to(FP8)
+    return (torch.randn(shape, generator=g, device=g.device) * 50).clamp(-448, 448).to(FP8)
 
 
 def _expand(scale, rows, cols, by, bx):
@@ -30,18 +30,27 @@ def _wide(t, stride, dev):
     return view
 
 
-def _run(recipe, m, n, k, bias, odt, col_major, gpu, lda=None, ldw=None):
-    """(output, fp64 reference, plan) of one call with seeded operands."""
-    from ayaka.kernel.hip import _lib, fp8_blockwise_mm, fp8_scaled_mm, mxfp8_scaled_mm
+def _run(recipe, m, n, k, bias, odt, col_major, gpu, lda=None, ldw=None, on="cpu", pad=0):
+    """(output, fp64 reference, plan) of one call with seeded operands, drawn on device ``on``;
+    ``pad`` columns behind the output's stay as they were."""
+    from ayaka.kernel.hip import _lib, fp8_blockwise_mm, fp8_scaled_mm, int8_scaled_mm, mxfp8_scaled_mm
 
-    g = torch.Generator().manual_seed(m * 131 + n * 7 + k)
-    a, w = _fp8((m, k), g), _fp8((n, k), g)
+    g = torch.Generator(device=on).manual_seed(m * 131 + n * 7 + k)
+    draw = lambda *shape: torch.rand(*shape, generator=g, device=on)  # noqa: E731
+    if recipe == "int8":
+        a, w = (torch.randint(-127, 128, (r, k), generator=g, dtype=torch.int8, device=on) for r in (m, n))
+    else:
+        a, w = _fp8((m, k), g), _fp8((n, k), g)
     ag, wg = _wide(a, lda, gpu), _wide(w, ldw, gpu)
-    b = torch.randn(n, generator=g).to(odt) if bias else None
-    out = torch.empty(m, n, dtype=odt, device=gpu)
+    b = torch.randn(n, generator=g, device=on).to(odt) if bias else None
+    buffer = torch.full((m, n + pad), 7.0, dtype=odt, device=gpu)
+    out = buffer[:, :n]
     bg = None if b is None else b.to(gpu)
-    if recipe == "scaled":
-        sa, sb = torch.rand(m, generator=g) * 1e-2, torch.rand(n, generator=g) * 1e-2
+    if recipe == "int8":
+        int8_scaled_mm(ag, wg.t(), torch.ones(m, device=gpu), torch.ones(n, device=gpu), bias=bg, out=out)
+        sa = sb = 1.0
+    elif recipe == "scaled":
+        sa, sb = draw(m) * 1e-2, draw(n) * 1e-2
         fp8_scaled_mm(ag, wg.t(), sa.to(gpu), sb.to(gpu), bias=bg, out=out)
         sa, sb = sa[:, None].double(), sb[:, None].double()
     elif recipe == "scalar":
@@ -49,7 +58,7 @@ def _run(recipe, m, n, k, bias, odt, col_major, gpu, lda=None, ldw=None):
         fp8_scaled_mm(ag, wg.t(), sa.to(gpu), sb.to(gpu), bias=bg, out=out)
     elif recipe in ("block", "block16"):
         kb = -(-k // 128)
-        ta, tb = torch.rand(m, kb, generator=g) * 1e-2, torch.rand(-(-n // 128), kb, generator=g) * 1e-2
+        ta, tb = draw(m, kb) * 1e-2, draw(-(-n // 128), kb) * 1e-2
         if not col_major:
             tb = tb.to(torch.bfloat16)
         if recipe == "block16":
@@ -58,16 +67,16 @@ def _run(recipe, m, n, k, bias, odt, col_major, gpu, lda=None, ldw=None):
         fp8_blockwise_mm(ag, wg, table.to(gpu), tb.to(gpu), bias=bg, out=out, a_scale_col_major=col_major)
         sa, sb = _expand(ta, m, k, 1, 128), _expand(tb, n, k, 128, 128)
     else:
-        ca = torch.randint(112, 122, (m, k // 32), generator=g, dtype=torch.uint8)
-        cb = torch.randint(112, 122, (n, k // 32), generator=g, dtype=torch.uint8)
+        ca, cb = (torch.randint(112, 122, (r, k // 32), generator=g, dtype=torch.uint8, device=on) for r in (m, n))
         mxfp8_scaled_mm(ag, ca.to(gpu), wg, cb.to(gpu), bg, out=out)
         sa, sb = (_expand(torch.exp2(c.double() - 127), c.shape[0], k, 1, 32) for c in (ca, cb))
     plan = _lib.last_plan()
+    assert (buffer[:, n:] == 7).all(), "wrote past the output columns"
     ref = (a.double() * sa).to(gpu) @ (w.double() * sb).to(gpu).t()
     return out, ref if b is None else ref + bg.double(), plan
 
 
-@pytest.mark.parametrize("recipe,m,n,k,bias,odt,col_major", [
+@pytest.mark.parametrize("recipe,m,n,k,bias,odt,col_major", [  # most on 64 x 64 tiles
     ("scaled", 65, 129, 16, True, torch.float32, False),       # one short stage
     ("scaled", 100, 128, 128, False, torch.bfloat16, False),   # exact stage
     ("scaled", 33, 1001, 4112, True, torch.float16, False),    # K tail, odd N, split
@@ -84,7 +93,7 @@ def _run(recipe, m, n, k, bias, odt, col_major, gpu, lda=None, ldw=None):
     ("mx", 100, 1000, 4096, False, torch.bfloat16, False),     # split in whole chunks
     ("mx", 70, 260, 1184, True, torch.float16, False),         # K % 128 != 0: unaligned codes
     ("mx", 40, 300, 2688, False, torch.bfloat16, False),       # K % 512 != 0
-    ("mx", 200, 2050, 2944, True, torch.float32, False),       # K % 512 != 0, split
+    ("mx", 200, 2050, 2944, True, torch.float32, False),       # K % 512 != 0, several tiles a side
     ("mx", 40, 4096, 11008, False, torch.bfloat16, False),     # a K the decode kernel cannot split
     ("mx", 300, 3072, 1536, True, torch.bfloat16, False),
 ])
@@ -138,7 +147,7 @@ def test_medium_tiles_nan_codes_stay_in_their_row(gpu):
 @pytest.mark.parametrize("stages", [1, 2, 3, 4, 5, 7, 8, 9])
 @pytest.mark.parametrize("recipe", ["scaled", "block", "block16", "mx", "int8"])
 def test_ring_stage_counts(gpu, recipe, stages):
-    """Every remainder of a K loop that runs in rounds of two, three or four 128-K stages, on
+    """Every remainder of the 64 x 64 ring's K loop, which runs in rounds of four 128-K stages, on
     shapes of one and of several tiles a side; 16-bit block scales start off a dword."""
     from ayaka.kernel.hip import _lib, fp8_blockwise_mm, int8_scaled_mm
 
@@ -162,7 +171,68 @@ def test_ring_stage_counts(gpu, recipe, stages):
         else:
             out, ref, _ = _run(recipe, m, n, k, True, torch.bfloat16, stages % 2 == 0, gpu)
             assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
-        assert _lib.last_plan().startswith("mid "), _lib.last_plan()
+        assert _lib.last_plan() == "mid 64x64 ring split=1", _lib.last_plan()
+
+
+# One shape per tile, ragged on both sides, that keeps its tile up to K = 1536. N % 4 == 2 also
+# keeps the 256 x 256 kernels away. Block scales have no 256 x 256 tile and one ring.
+_TILES = {"256x256": (463, 28958), "128x128": (205, 28958), "128x64": (137, 16634), "128x128 ring": (205, 12358),
+          "128x64 ring": (65, 8318), "64x64 ring": (65, 130)}
+_TILE_SHAPES = {"scaled": _TILES, "int8": _TILES, "mx": _TILES | {"256x256": (403, 28390), "128x128": (205, 24718)}}
+for _recipe in ("block", "block16"):
+    _TILE_SHAPES[_recipe] = {"128x128": (205, 24718), "128x64": (65, 24718), "64x64 ring": (65, 130)}
+
+
+@pytest.mark.parametrize("recipe,tile,m,n", [(r, t, *mn) for r, tiles in _TILE_SHAPES.items() for t, mn in tiles.items()])
+def test_every_tile_and_stage_count(gpu, recipe, tile, m, n):
+    """Each tile and ring with every remainder of its K loop (rounds of two or four stages), K
+    tails and, for MXFP8, the three layouts of its codes: whole 512-K chunks (4, 8, 12 stages),
+    whole dwords and unaligned."""
+    less = {"scaled": (0, 48), "int8": (0, 112), "mx": (0, 32), "block": (0,), "block16": (0,)}[recipe]
+    for stages in (*range(1, 10), 12):
+        for k in (128 * stages - d for d in less):
+            print(f"every tile recipe={recipe} tile={tile} m={m} n={n} k={k}", flush=True)
+            out, ref, plan = _run(recipe, m, n, k, stages % 2 == 1, torch.bfloat16 if stages % 3 else torch.float32,
+                                  stages % 2 == 0, gpu, on=gpu)
+            assert plan == f"mid {tile} split=1", plan
+            assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("recipe,m,n,k,expect", [
+    ("scaled", 205, 16634, 7792, "256x256 split=3"),
+    ("scaled", 65, 16634, 7792, "128x128 split=3"),
+    ("scaled", 137, 5486, 9872, "128x64 split=3"),
+    ("scaled", 65, 8318, 5712, "128x128 ring split=3"),
+    ("scaled", 65, 2690, 11952, "128x64 ring split=4"),
+    ("scaled", 65, 130, 3632, "64x64 ring split=6"),
+    ("block", 65, 16634, 3968, "128x128 split=3"),
+    ("block", 65, 4158, 6656, "128x64 split=6"),
+    ("block16", 65, 130, 2432, "64x64 ring split=4"),
+    ("mx", 205, 16634, 6656, "256x256 split=3"),       # codes: whole chunks
+    ("mx", 205, 16634, 7040, "256x256 split=3"),       # whole dwords
+    ("mx", 205, 16634, 6336, "256x256 split=3"),       # unaligned
+    ("mx", 65, 16634, 8192, "128x128 split=3"),
+    ("mx", 65, 16634, 7808, "128x128 split=3"),
+    ("mx", 65, 16634, 7232, "128x128 split=3"),
+    ("mx", 137, 5486, 8192, "128x64 split=3"),
+    ("mx", 137, 5486, 8576, "128x64 split=3"),
+    ("mx", 137, 5486, 7904, "128x64 split=3"),
+    ("mx", 65, 2690, 10240, "128x128 ring split=7"),
+    ("mx", 65, 2690, 8960, "128x128 ring split=6"),
+    ("mx", 65, 2690, 8800, "128x128 ring split=6"),
+    ("mx", 65, 2690, 5632, "128x64 ring split=4"),
+    ("mx", 65, 1346, 10880, "128x64 ring split=8"),
+    ("mx", 65, 1346, 10816, "128x64 ring split=8"),
+    ("mx", 65, 130, 2560, "64x64 ring split=3"),
+    ("mx", 65, 130, 2816, "64x64 ring split=3"),
+    ("mx", 65, 130, 2528, "64x64 ring split=3"),
+])
+def test_every_tile_split(gpu, recipe, m, n, k, expect):
+    """K splits of each tile whose last piece is shorter."""
+    print(f"tile split recipe={recipe} m={m} n={n} k={k}", flush=True)
+    out, ref, plan = _run(recipe, m, n, k, True, torch.bfloat16, recipe == "block16", gpu, on=gpu)
+    assert plan == f"mid {expect}", plan
+    assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
 
 
 _FAR = 1 << 23  # rows 8 MiB apart: 256 of them leave the medium tiles' 32-bit offsets
@@ -240,3 +310,40 @@ def test_large_kernel_choice(gpu, recipe, m, n, k, expect):
     out, ref, plan = _run(recipe, m, n, k, True, torch.bfloat16, recipe == "block", gpu)
     assert plan == expect, plan
     assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("recipe,m,n,k,odt,pad,expect", [
+    ("scaled", 258, 33132, 1536, torch.bfloat16, 4, "pair tail=3"),    # padded output rows
+    ("scaled", 258, 33132, 1536, torch.float32, 0, "pair tail=3"),
+    ("scaled", 1300, 11712, 3072, torch.float16, 0, "pair tail=6"),    # a last round of 20 tiles
+    ("scaled", 258, 8016, 128, torch.bfloat16, 0, "pair tail=1"),      # one pair of stages
+    ("scaled", 520, 16388, 1280, torch.float16, 12, "pair tail=1"),
+    ("scaled", 258, 3608, 10368, torch.bfloat16, 8, "pair split=8"),   # last piece shorter
+    ("scaled", 258, 13252, 64, torch.float16, 4, "big"),               # one stage
+    ("scaled", 516, 13260, 1088, torch.bfloat16, 4, "big"),
+    ("int8", 258, 8016, 128, torch.float32, 4, "pair split=1"),
+    ("int8", 520, 16388, 1280, torch.float32, 0, "pair split=1"),
+    ("int8", 520, 16388, 1216, torch.float32, 4, "big"),
+    ("mx", 258, 33132, 1536, torch.float16, 4, "pair tail=3"),
+    ("mx", 1300, 11712, 3072, torch.bfloat16, 0, "pair tail=6"),
+    ("mx", 258, 21904, 512, torch.float32, 4, "pair tail=1"),          # one chunk of codes
+    ("mx", 520, 16388, 1024, torch.bfloat16, 12, "pair tail=1"),
+    ("mx", 258, 3608, 7168, torch.bfloat16, 0, "pair split=7"),
+    ("mx", 258, 1672, 20992, torch.float32, 0, "pair split=14"),       # last piece shorter
+    ("block", 258, 1828, 128, torch.float32, 0, "block256 split=1"),   # one block
+    ("block", 258, 1828, 8192, torch.float16, 4, "block256 split=8"),
+    ("block", 258, 2184, 7296, torch.bfloat16, 0, "block256 split=7"),  # last piece shorter
+    ("block", 258, 516, 16384, torch.bfloat16, 4, "block128 split=16"),
+    ("block", 128, 26532, 3072, torch.float16, 4, "block128 split=1"),
+])
+@pytest.mark.parametrize("bias", [False, True])
+def test_large_kernel_edges(gpu, recipe, m, n, k, odt, pad, expect, bias):
+    """The 256 x 256 kernels' (and the block-scaled 128 x 128 one's) tails of M and N, first and
+    last K steps, K splits, tail splits and strided outputs, on shapes that the dispatch gives
+    them."""
+    print(f"large edges recipe={recipe} m={m} n={n} k={k} out={odt} pad={pad} bias={bias}", flush=True)
+    out, ref, plan = _run(recipe, m, n, k, bias, odt, recipe == "block" and bias, gpu, on=gpu, pad=pad)
+    assert plan == expect, plan
+    assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
+    if recipe == "int8" and not bias:
+        assert torch.equal(out, ref.float())

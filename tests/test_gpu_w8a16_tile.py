@@ -55,21 +55,35 @@ def _check(m, n, k, xdt, by, bx, sdt, dev):
 @pytest.mark.parametrize("m,n,k,xdt,by,bx,sdt,plan", [
     (33, 129, 16, torch.bfloat16, 1, None, "float32", "128x64 split=1"),      # one short stage
     (64, 128, 64, torch.float16, 1, None, "float32", "128x64 split=1"),       # exact tile and stage
-    (65, 257, 1040, torch.bfloat16, 1, None, "bfloat16", "128x64 split="),    # every remainder, split
-    (20, 1000, 1936, torch.float16, 1, None, "float32", "128x64 split="),     # K no decode kernel takes
-    (40, 2051, 3072, torch.bfloat16, 1, None, "float32", "128x64 split="),    # N not a multiple of 4, split
+    (65, 257, 1040, torch.bfloat16, 1, None, "bfloat16", "128x64 split=1"),   # every remainder
+    (20, 1000, 1936, torch.float16, 1, None, "float32", "128x64 split=3"),    # K no decode kernel takes, last piece shorter
+    (40, 2051, 3072, torch.bfloat16, 1, None, "float32", "128x64 split=6"),   # N not a multiple of 4, split
     (1, 300, 144, torch.bfloat16, 1, None, "e8m0", "128x64 split=1"),
-    (200, 4099, 14336, torch.float16, 1, None, "float32", "split="),
-    (129, 9000, 7168, torch.bfloat16, 128, 128, "float32", "split="),
-    (500, 5000, 4096, torch.bfloat16, 1, None, "float32", "split="),
-    (257, 513, 336, torch.bfloat16, 64, 128, "float32", "split=1"),
-    (300, 640, 4160, torch.float16, 128, 64, "bfloat16", "split="),
-    (1000, 28672, 1040, torch.bfloat16, 1, None, "float32", "split=1"),
-    (2049, 8200, 576, torch.float16, 1, None, "float32", "split=1"),
+    (200, 4099, 14336, torch.float16, 1, None, "float32", "256x256 split=12"),
+    (129, 9000, 7168, torch.bfloat16, 128, 128, "float32", "256x256 split=6"),
+    (500, 5000, 4096, torch.bfloat16, 1, None, "float32", "128x128 split=3"),
+    (257, 513, 336, torch.bfloat16, 64, 128, "float32", "128x64 split=1"),
+    (300, 640, 4160, torch.float16, 128, 64, "bfloat16", "128x64 split=8"),
+    (1000, 28672, 1040, torch.bfloat16, 1, None, "float32", "256x256 split=1"),
+    (2049, 8200, 576, torch.float16, 1, None, "float32", "128x128 split=1"),
+    (65, 16634, 8320, torch.bfloat16, 1, None, "float32", "256x128 split=6"),
+    (65, 16634, 8320, torch.float16, 128, 128, "float32", "256x128 split=6"),
+    (65, 4158, 8320, torch.float16, 128, 192, "float32", "128x128 split=12"),  # scale blocks of three stages
 ])
 def test_weight_only_gemm_tile(gpu, m, n, k, xdt, by, bx, sdt, plan):
     got = _check(m, n, k, xdt, by, bx, sdt, gpu)
-    assert got.startswith("w8a16 tile") and plan in got, got
+    assert got == f"w8a16 tile {plan}", got
+
+
+@pytest.mark.parametrize("tile,m,n", [("256x256", 403, 24718), ("256x128", 529, 21946), ("128x128", 205, 24718),
+                                      ("128x64", 65, 130)])
+@pytest.mark.parametrize("by,bx", [(1, None), (128, 64), (96, 128)])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
+def test_weight_only_gemm_every_tile(gpu, tile, m, n, by, bx, xdt):
+    """One to five K stages and tails on each tile, ragged on both sides."""
+    for k in (16, 64, 112, 128, 192, 208, 320):
+        got = _check(m, n, k, xdt, by, bx, "float32", gpu)
+        assert got == f"w8a16 tile {tile} split=1", got
 
 
 @pytest.mark.parametrize("m,n,k,bx,plan", [
