@@ -72,8 +72,9 @@ __device__ inline v16f mid_mma(const v8i& w, const v8i& a, const v16f& c, int cw
 
 // WN x WM wavefronts of (BN / WN) weight rows x (BM / WM) activation rows. kps > 0: the
 // launch splits K (whole 128-K stages), blockIdx.y takes [y kps, (y + 1) kps) and writes
-// an fp32 partial without the bias. D stage buffers: D - 1 stages are in flight.
-template <int MODE, int BN, int BM, int WN, int WM, int D, int WGS>
+// an fp32 partial without the bias. D stage buffers: D - 1 stages are in flight. F32:
+// large fp32 outputs, whose rows pass through LDS (no K split).
+template <int MODE, bool F32, int BN, int BM, int WN, int WM, int D, int WGS>
 __global__ __launch_bounds__(WN * WM * 64, WGS) void fp8_mid_kernel(MidArgs g, int tiles_m, int64_t kps) {
   constexpr int kThreads = WN * WM * 64, kWaves = WN * WM;
   constexpr int TN = BN / WN, TM = BM / WM, FN = TN / 32, FM = TM / 32;
@@ -382,6 +383,25 @@ __global__ __launch_bounds__(WN * WM * 64, WGS) void fp8_mid_kernel(MidArgs g, i
       asm volatile("" : "+v"(v[q]));
     }
   };
+  // Every wavefront stages 32 (m) x TN (n) slabs in a private region of the stage buffers.
+  constexpr int kRegion = 32 * TN * (F32 ? 4 : 2), kPerBuf = kStage / kRegion;
+  static_assert(2 * kPerBuf >= kWaves, "the staging regions fit the stage buffers");
+  uint8_t* region = wave < kPerBuf ? B0 + wave * kRegion : B1 + (wave - kPerBuf) * kRegion;
+  if constexpr (F32) {
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int grp = 0; grp < 4; ++grp) {
+          float v[4];
+          value(i, j, grp, v);
+          stage_slab32<TN>(region, frow, 32 * i + 8 * grp + 4 * h, v);
+        }
+      store_slab32<TN>(region, static_cast<float*>(g.out), g.ldo, g.M, g.N, m_w + 32 * j, n_w, lane);
+    }
+    return;
+  }
   if (kps > 0 || g.out_dtype == AYK_F32) {
     float* base = kps > 0 ? g.ws + (int64_t)blockIdx.y * g.M * g.N : static_cast<float*>(g.out);
     const int64_t ldo = kps > 0 ? g.N : g.ldo;
@@ -401,9 +421,6 @@ __global__ __launch_bounds__(WN * WM * 64, WGS) void fp8_mid_kernel(MidArgs g, i
     }
     return;
   }
-  constexpr int kRegion = 32 * TN * 2, kPerBuf = kStage / kRegion;
-  static_assert(2 * kPerBuf >= kWaves, "the staging regions fit the stage buffers");
-  uint8_t* region = wave < kPerBuf ? B0 + wave * kRegion : B1 + (wave - kPerBuf) * kRegion;
   const bool bf16 = g.out_dtype == AYK_BF16;
 #pragma unroll
   for (int j = 0; j < FM; ++j) {
@@ -498,12 +515,12 @@ size_t split_bytes(const MidPlan& p, int64_t M, int64_t N) {
   return p.split > 1 ? (size_t)p.split * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
-template <int MODE>
+template <int MODE, bool F32>
 void launch_tile(const MidArgs& g, const MidPlan& p, int64_t kps, hipStream_t st) {
   const MidTile& t = kTiles[p.config];
   const int tiles_m = (int)cdiv(g.M, t.bm);
   const dim3 grid((unsigned)(tiles_m * cdiv(g.N, t.bn)), (unsigned)p.split);
-#define AYK_MID(...) hipLaunchKernelGGL((fp8_mid_kernel<MODE, __VA_ARGS__>), grid, dim3(threads), 0, st, g, tiles_m, kps)
+#define AYK_MID(...) hipLaunchKernelGGL((fp8_mid_kernel<MODE, F32, __VA_ARGS__>), grid, dim3(threads), 0, st, g, tiles_m, kps)
   const unsigned threads = p.config == 0 ? 512 : 256;
   if constexpr (MODE == kMidBlock) {
     switch (p.config) {
@@ -522,6 +539,15 @@ void launch_tile(const MidArgs& g, const MidPlan& p, int64_t kps, hipStream_t st
     }
   }
 #undef AYK_MID
+}
+
+// fp32 outputs of 4 MB and more pass through LDS up to K = 4096: below, the staging is a wait
+// without a return (72 x 868 x 128: 4.8 -> 5.6 us), and past it the output is a small part of
+// the launch.
+template <int MODE>
+void launch_mode(const MidArgs& g, const MidPlan& p, int64_t kps, hipStream_t st) {
+  if (g.out_dtype == AYK_F32 && p.split == 1 && g.M * g.N >= (1 << 20) && g.K <= 4096) launch_tile<MODE, true>(g, p, kps, st);
+  else launch_tile<MODE, false>(g, p, kps, st);
 }
 
 }  // namespace
@@ -552,16 +578,16 @@ int mid_launch(MidMode mode, const MidArgs& g, hipStream_t st, const char* op) {
   note_plan("mid %dx%d%s split=%d", kTiles[p.config].bn, kTiles[p.config].bm, p.config >= 3 ? " ring" : "", p.split);
   const uintptr_t code_align = reinterpret_cast<uintptr_t>(g.sa) | reinterpret_cast<uintptr_t>(g.sb) | (uintptr_t)(g.ld_sa | g.ld_sb);
   switch (mode) {
-    case kMidScaled: launch_tile<kMidScaled>(g, p, kps, st); break;
-    case kMidBlock: launch_tile<kMidBlock>(g, p, kps, st); break;
-    case kMidInt8: launch_tile<kMidInt8>(g, p, kps, st); break;
+    case kMidScaled: launch_mode<kMidScaled>(g, p, kps, st); break;
+    case kMidBlock: launch_mode<kMidBlock>(g, p, kps, st); break;
+    case kMidInt8: launch_mode<kMidInt8>(g, p, kps, st); break;
     default:
       if (g.K % (4 * kStageK) == 0 && (code_align & 15) == 0) {
-        launch_tile<kMidMx>(g, p, kps, st);
+        launch_mode<kMidMx>(g, p, kps, st);
       } else if (g.K % kStageK == 0 && (code_align & 3) == 0) {
-        launch_tile<kMidMx4>(g, p, kps, st);
+        launch_mode<kMidMx4>(g, p, kps, st);
       } else {
-        launch_tile<kMidMxAny>(g, p, kps, st);
+        launch_mode<kMidMxAny>(g, p, kps, st);
       }
   }
   if (int rc = check_launch(op)) return rc;

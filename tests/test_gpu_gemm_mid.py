@@ -116,6 +116,20 @@ def test_medium_tiles_half_outputs(gpu, recipe, k, n):
         assert plan == plan2 and torch.equal(half, full.to(odt))
 
 
+@pytest.mark.parametrize("recipe", ["scaled", "block", "block16", "mx", "int8"])
+@pytest.mark.parametrize("m,k,n,pad", [(70, 256, 16633, 0), (70, 256, 16634, 1), (70, 256, 16635, 5), (70, 384, 16636, 0),
+                                       (1030, 256, 1031, 2), (137, 4096, 16634, 0), (137, 4224, 16634, 0)])
+def test_medium_tiles_large_f32_outputs(gpu, recipe, m, k, n, pad):
+    """fp32 outputs of 2^20 elements and more, which pass through LDS up to K = 4096: rows of every
+    alignment, and the 16-bit outputs are their rounding."""
+    print(f"large fp32 output recipe={recipe} m={m} n={n} k={k} pad={pad}", flush=True)
+    full, ref, plan = _run(recipe, m, n, k, False, torch.float32, False, gpu, on=gpu, pad=pad)
+    assert plan.startswith("mid ") and plan.endswith("split=1"), plan
+    assert_linear_close(full, ref, f"{recipe} {m}x{n}x{k}")
+    half, _, plan2 = _run(recipe, m, n, k, False, torch.bfloat16, False, gpu, on=gpu)
+    assert plan == plan2 and torch.equal(half, full.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("m,n,k", [(8, 130, 16), (100, 1000, 1040), (65, 257, 4096), (300, 2052, 2064)])
 def test_medium_tiles_int8_exact(gpu, m, n, k):
     """The int32 sums are exact (4096 x 127^2 < 2^31): scales of one return them rounded to fp32."""
