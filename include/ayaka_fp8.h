@@ -122,9 +122,11 @@ int ayk_fp8_scaled_mm(const void* a, int64_t lda, const void* b, int64_t ldb,
 /* Bytes of split-K partials ayk_fp8_scaled_mm may need for this shape (0: none). A
  * launch short of one full round of tiles splits K; a launch whose last round of
  * 256 x 256 tiles is at most a third full splits that round's tiles over K; a decode
- * batch (M <= 64) on a narrow projection splits K across workgroups. Each piece writes
- * its fp32 partial and a fixed-order sum adds the bias and rounds once. The size is
- * the largest any of these needs for the shape. */
+ * batch (M <= 64) on a narrow projection splits K across workgroups, as the medium tiles
+ * do at any M. Each piece writes its fp32 partial and a fixed-order sum adds the bias and
+ * rounds once. The size is the largest any of these needs for the shape. With a smaller
+ * workspace or none, the medium tiles run without a split; every other kernel that would
+ * split returns AYK_EWORKSPACE. */
 size_t ayk_fp8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /* fp8_rowwise_linear (gemm/fp8_linear.py:168) for 2 to 8 activation rows in one launch:
@@ -150,8 +152,7 @@ int ayk_int8_scaled_mm(const void* a, int64_t lda, const void* b, int64_t ldb,
                        const void* bias, int bias_dtype,
                        void* out, int out_dtype, int64_t ldo,
                        void* workspace, size_t workspace_bytes, ayk_stream_t stream);
-/* Bytes of split-K partials ayk_int8_scaled_mm may need for this shape (0: none); the
- * same rule as ayk_fp8_scaled_mm_workspace_bytes. */
+/* Always 0: the INT8 GEMM never splits K (its int32 sums stay exact). */
 size_t ayk_int8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /* Replaces ayaka::fp8_blockwise_mm (gemm/fp8_gemm.py:370; oracle reference/gemm.py:40-70).
@@ -167,7 +168,8 @@ int ayk_fp8_blockwise_mm(const void* a, int64_t lda, const void* b, int64_t ldb,
                          void* workspace, size_t workspace_bytes, ayk_stream_t stream);
 /* Bytes of split-K partials ayk_fp8_blockwise_mm may need for this shape (0: none). A
  * launch with fewer tiles than fill the machine (or, for M <= 64, fewer row groups)
- * splits K and sums fp32 partials in a fixed order before the single rounding. */
+ * splits K and sums fp32 partials in a fixed order before the single rounding. A smaller
+ * workspace is treated as by ayk_fp8_scaled_mm. */
 size_t ayk_fp8_blockwise_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /* Replaces fp8_blockwise_scaled_grouped_mm (kernel/triton/moe/moe_grouped_gemm.py:599,
@@ -238,11 +240,11 @@ size_t ayk_fp8_weight_only_gemv_static_max_bytes(void);
 /* Replaces ayaka::fp8_weight_only_gemm (gemm/fp8_w8a16_gemm.py:144; oracle
  * reference/gemm.py:95-126). The [M, K] form of ayk_fp8_weight_only_gemv; out dtype ==
  * x dtype. Each dequantized weight w * scale is rounded to the activation dtype before
- * the product, as the reference does (with a per-row scale, block_size_x >= K, the
- * exact fp8 weight enters the product and the scale multiplies the fp32 sum).
- * Decode batches (M <= 32) may use a K split whose partials live in the workspace;
- * ayk_fp8_weight_only_gemm_workspace_bytes(M, N, K, block_size_x) gives its size
- * (0: none needed). */
+ * the product, as the reference does. Launches of any M may use a K split whose partials
+ * live in the workspace; ayk_fp8_weight_only_gemm_workspace_bytes(M, N, K, block_size_x)
+ * gives its size (0: none needed). With a smaller workspace or none, the tiled kernel
+ * (every batch past 32 rows) runs without a split; the decode kernels that would split
+ * return AYK_EWORKSPACE. */
 int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
                              const void* w, int64_t ldw, int64_t N, int64_t K,
                              const void* scale, int scale_dtype, int64_t scale_row_stride,
