@@ -2008,8 +2008,9 @@ template <int MODE>
 int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
   const MidArgs mid = mid_args(g);
   const bool mid_ok = mid_supported(mid_mode(MODE), mid);
+  const MidPlan plan = mid_ok ? mid_plan(mid_mode(MODE), g.M, g.N, g.K) : MidPlan{};
   // Whether the medium tiles beat a kernel that is modelled at `us`.
-  auto mid_beats = [&](float us) { return mid_ok && mid_time(mid_mode(MODE), g.M, g.N, g.K) < us; };
+  auto mid_beats = [&](float us) { return mid_ok && mid_time(plan, g.N, g.K) < us; };
   // The large-tile kernels need K % 64 == 0, fp32 scales (MXFP8: K % 512 == 0 and 16-byte
   // aligned code rows), N % 4 == 0 and 16-byte aligned output rows (its epilogue stores
   // 16-byte chunks).
@@ -2064,7 +2065,7 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
       }
     }
   }
-  if (mid_ok && !general_wanted<MODE>(g.M, g.N, g.K)) return mid_launch(mid_mode(MODE), mid, st, op);
+  if (mid_ok && !general_wanted<MODE>(g.M, g.N, g.K)) return mid_launch(mid_mode(MODE), mid, plan, st, op);
   return launch_general<MODE>(g, st, op);
 }
 

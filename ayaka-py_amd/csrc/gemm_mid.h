@@ -32,12 +32,18 @@ struct MidArgs {
   size_t ws_bytes;
 };
 
-// Workspace bytes of the launch (0: no K split) and its modelled time in microseconds;
-// functions of the mode and shape only.
+// Tile and K split of a shape with their modelled time in microseconds, and the workspace
+// bytes of the launch (0: no K split); functions of the mode and shape only.
+struct MidPlan {
+  int config, split;
+  float us;
+};
+MidPlan mid_plan(MidMode mode, int64_t M, int64_t N, int64_t K, bool may_split = true);
+float mid_time(const MidPlan& p, int64_t N, int64_t K);
 size_t mid_workspace(MidMode mode, int64_t M, int64_t N, int64_t K);
-float mid_time(MidMode mode, int64_t M, int64_t N, int64_t K);
 // 32-bit offsets within a tile's rows.
 bool mid_supported(MidMode mode, const MidArgs& g);
-int mid_launch(MidMode mode, const MidArgs& g, hipStream_t st, const char* op);
+// `p`: mid_plan of the shape.
+int mid_launch(MidMode mode, const MidArgs& g, MidPlan p, hipStream_t st, const char* op);
 
 }  // namespace ayk

@@ -459,11 +459,9 @@ __global__ __launch_bounds__(256) void mid_reduce(const float* __restrict__ part
 // latency) and `store` per 256 x 256 outputs; `cold` is the weights' share that no stage
 // hides; a split adds a reduce launch and the fp32 partials' traffic. Its choice is 1-2%
 // slower than the fastest triple on average (tau of the two-buffer tiles: from the launches of
-// two rounds and more, above the fit, whose weight lies on the small ones).
-struct MidPlan {
-  int config, split;
-  float us;
-};
+// two rounds and more, above the fit, whose weight lies on the small ones). It runs for every
+// workspace query and launch, so no division in its loops has a variable divisor (0.40 us a plan
+// with them, 0.15 without).
 struct MidTile {
   int bn, bm, resident;
 };
@@ -487,20 +485,35 @@ int64_t mid_kps(MidMode mode, int64_t K, int split) {
   return cdiv(cdiv(K, unit), split) * unit;
 }
 
+// Tiles of `side` rows (64, 128 or 256).
+int64_t tile_count(int64_t rows, int side) { return side == 256 ? cdiv(rows, 256) : (side == 128 ? cdiv(rows, 128) : cdiv(rows, 64)); }
+int64_t by_resident(int64_t n, int resident) { return resident == 1 ? n : (resident == 2 ? cdiv(n, 2) : cdiv(n, 3)); }
+
+size_t split_bytes(const MidPlan& p, int64_t M, int64_t N) {
+  return p.split > 1 ? (size_t)p.split * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+
+}  // namespace
+
 MidPlan mid_plan(MidMode mode, int64_t M, int64_t N, int64_t K, bool may_split) {
   const MidModel& m = kModels[mode == kMidInt8 ? kMidScaled : mode];
   MidPlan best{5, 1, 0.0f};
   bool first = true;
+  // INT8 never splits: a partial would leave the exact int32 sum.
+  int splits = 1;
+  while (may_split && mode != kMidInt8 && splits < 8 && K >= (int64_t)kMinSplitK * kSplits[splits]) ++splits;
+  int64_t stages[8];
+  for (int i = 0; i < splits; ++i) stages[i] = cdiv(cdiv(K, kStageK), kSplits[i]);
   for (int c = 0; c < kConfigs; ++c) {
     if (m.tau[c] == 0.0f) continue;
     const MidTile& t = kTiles[c];
-    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
-    for (const int s : kSplits) {
-      // INT8 never splits: a partial would leave the exact int32 sum.
-      if (s > 1 && (!may_split || mode == kMidInt8 || K < (int64_t)kMinSplitK * s)) break;
-      const float u = (float)cdiv(tiles * s, kCus), rounds = (float)cdiv(cdiv(tiles * s, kCus), t.resident);
+    const int64_t tiles = tile_count(M, t.bm) * tile_count(N, t.bn);
+    for (int i = 0; i < splits; ++i) {
+      const int s = kSplits[i];
+      const int64_t wgs = cdiv(tiles * s, kCus);  // a CU
+      const float u = (float)wgs, rounds = (float)by_resident(wgs, t.resident);
       const float stage = rounds * m.lambda[c] > u * m.tau[c] ? rounds * m.lambda[c] : u * m.tau[c];
-      float us = m.base + m.cold * (float)N * (float)K + (float)cdiv(cdiv(K, kStageK), s) * stage + m.store * u * (float)(t.bn * t.bm) / 65536.0f;
+      float us = m.base + m.cold * (float)N * (float)K + (float)stages[i] * stage + m.store * u * (float)(t.bn * t.bm) / 65536.0f;
       if (s > 1) us += m.reduce + m.partial * (float)s * (float)M * (float)N;
       if (first || us < best.us) {
         first = false;
@@ -511,9 +524,8 @@ MidPlan mid_plan(MidMode mode, int64_t M, int64_t N, int64_t K, bool may_split) 
   best.split = (int)cdiv(K, mid_kps(mode, K, best.split));  // rounded-up pieces may need fewer of them
   return best;
 }
-size_t split_bytes(const MidPlan& p, int64_t M, int64_t N) {
-  return p.split > 1 ? (size_t)p.split * (size_t)M * (size_t)N * sizeof(float) : 0;
-}
+
+namespace {
 
 template <int MODE, bool F32>
 void launch_tile(const MidArgs& g, const MidPlan& p, int64_t kps, hipStream_t st) {
@@ -552,14 +564,12 @@ void launch_mode(const MidArgs& g, const MidPlan& p, int64_t kps, hipStream_t st
 
 }  // namespace
 
-size_t mid_workspace(MidMode mode, int64_t M, int64_t N, int64_t K) {
-  return split_bytes(mid_plan(mode, M, N, K, true), M, N);
-}
+size_t mid_workspace(MidMode mode, int64_t M, int64_t N, int64_t K) { return split_bytes(mid_plan(mode, M, N, K), M, N); }
 // The weights stream at no more than 4.4 TB/s beside a launch and its prologue (only the
 // smallest batches are near that; the plan itself does not depend on it).
-float mid_time(MidMode mode, int64_t M, int64_t N, int64_t K) {
-  const float us = mid_plan(mode, M, N, K, true).us, stream = 6.0f + (float)N * (float)K / 4.4e6f;
-  return us > stream ? us : stream;
+float mid_time(const MidPlan& p, int64_t N, int64_t K) {
+  const float stream = 6.0f + (float)N * (float)K / 4.4e6f;
+  return p.us > stream ? p.us : stream;
 }
 
 bool mid_supported(MidMode mode, const MidArgs& g) {
@@ -570,8 +580,7 @@ bool mid_supported(MidMode mode, const MidArgs& g) {
          !(mode == kMidBlock && g.sa_vec && 4 * g.M * cdiv(g.K, 128) >= lim) && cdiv(g.M, 64) * cdiv(g.N, 64) < lim;
 }
 
-int mid_launch(MidMode mode, const MidArgs& g, hipStream_t st, const char* op) {
-  MidPlan p = mid_plan(mode, g.M, g.N, g.K, true);
+int mid_launch(MidMode mode, const MidArgs& g, MidPlan p, hipStream_t st, const char* op) {
   // A caller that brings no workspace gets the best plan without a split.
   if (p.split > 1 && (g.ws == nullptr || g.ws_bytes < split_bytes(p, g.M, g.N))) p = mid_plan(mode, g.M, g.N, g.K, false);
   const int64_t kps = p.split > 1 ? mid_kps(mode, g.K, p.split) : 0;

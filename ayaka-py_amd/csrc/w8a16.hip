@@ -1483,7 +1483,8 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
   const W16TileArgs t{g.x, ldx, g.w, ldw, M, N, K, scale, scale_dtype, scale_row_stride, block_size_y, block_size_x,
                       out, ldo, static_cast<float*>(workspace), workspace_bytes};
   const bool tile_ok = w16_tile_supported(t);
-  auto tile_beats = [&](float us) { return tile_ok && w16_tile_time(M, N, K) < 0.75f * us; };
+  const W16TilePlan tp = tile_ok ? w16_tile_plan(M, N, K) : W16TilePlan{};
+  auto tile_beats = [&](float us) { return tile_ok && w16_tile_time(tp, N, K) < 0.75f * us; };
   if (M >= 2) {
     const StPlan sp = stream_plan(M, N, K, block_size_x);
     if (sp.ok && !tile_beats(stream_time(sp, N, K))) {
@@ -1524,7 +1525,7 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
     }
   }
   // Everything else: the tiled kernel, but for scale blocks that split its 64-K stages.
-  if (tile_ok) return w16_tile_launch(t, x_dtype == AYK_BF16, st, op);
+  if (tile_ok) return w16_tile_launch(t, tp, x_dtype == AYK_BF16, st, op);
   return x_dtype == AYK_BF16 ? dispatch_w16<true>(g, st) : dispatch_w16<false>(g, st);
 }
 

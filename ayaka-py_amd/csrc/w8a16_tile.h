@@ -25,12 +25,18 @@ struct W16TileArgs {
   size_t part_bytes;
 };
 
-// Workspace bytes of the launch below (0: no K split); a function of the shape only.
+// Tile and K split of a shape with their modelled time in microseconds, and the workspace
+// bytes of the launch below (0: no K split); functions of the shape only.
+struct W16TilePlan {
+  int config, split;
+  float us;
+};
+W16TilePlan w16_tile_plan(int64_t M, int64_t N, int64_t K, bool may_split = true);
+float w16_tile_time(const W16TilePlan& p, int64_t N, int64_t K);
 size_t w16_tile_workspace(int64_t M, int64_t N, int64_t K);
-// Its modelled time in microseconds.
-float w16_tile_time(int64_t M, int64_t N, int64_t K);
 // Whether the tiled kernel takes this problem.
 bool w16_tile_supported(const W16TileArgs& a);
-int w16_tile_launch(const W16TileArgs& a, bool bf16, hipStream_t st, const char* op);
+// `p`: w16_tile_plan of the shape.
+int w16_tile_launch(const W16TileArgs& a, W16TilePlan p, bool bf16, hipStream_t st, const char* op);
 
 }  // namespace ayk

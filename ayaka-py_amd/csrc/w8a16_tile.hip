@@ -12,7 +12,7 @@
 //    256 as 64 x 128 wavefront tiles: 382 us on 4096 x 4096 x 14336, as 128 x 64: 429;
 //    128 x 128 as 32 x 128 against 64 x 64: 462 and 491).
 //  * 256 x 256, 256 x 128, 128 x 128 and 128 x 64 (n x m) tiles, two to four workgroups a
-//    CU for the smaller ones, and a K split, chosen by tile_plan.
+//    CU for the smaller ones, and a K split, chosen by w16_tile_plan.
 // Measured against the register-staged 128 x 128 kernel this replaces (Llama-3-8B, bf16,
 // 218 MB of weights, M = 1024): 274 -> 960 TFLOP/s over the four projections; 4096 x
 // 14336 at M = 4096 reaches 1260 TFLOP/s, 88% of a bf16 library product on the same card.
@@ -262,11 +262,8 @@ __global__ __launch_bounds__(256) void w8a16_tile_reduce(const float* __restrict
 // max(u tau, ceil(u / resident) lambda) per 64-K stage (throughput, or one round's
 // latency) and an epilogue in proportion to its output; a split adds a reduce launch and
 // the fp32 partials' traffic. Over those shapes its choice is 1.4% slower than the
-// fastest tile and split on average, 15% at worst.
-struct TilePlan {
-  int config, split;
-  float us;
-};
+// fastest tile and split on average, 15% at worst. It runs for every workspace query and
+// launch: no division in its loops has a variable divisor (0.27 us a plan with them, 0.10 without).
 struct TileConfig {
   int bn, bm, resident;
   float tau, lambda;
@@ -280,17 +277,34 @@ constexpr int kCus = 256;
 int64_t stages(int64_t K) { return cdiv(K, kStepK); }
 int64_t split_kps(int64_t K, int split) { return cdiv(stages(K), split) * kStepK; }
 
-TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
-  TilePlan best{0, 1, 0.0f};
+// Tiles of `side` rows (64, 128 or 256).
+int64_t tile_count(int64_t rows, int side) { return side == 256 ? cdiv(rows, 256) : (side == 128 ? cdiv(rows, 128) : cdiv(rows, 64)); }
+int64_t by_resident(int64_t n, int resident) {
+  return resident == 1 ? n : (resident == 2 ? cdiv(n, 2) : (resident == 3 ? cdiv(n, 3) : cdiv(n, 4)));
+}
+
+size_t split_bytes(const W16TilePlan& p, int64_t M, int64_t N) {
+  return p.split > 1 ? (size_t)p.split * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+
+}  // namespace
+
+W16TilePlan w16_tile_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
+  W16TilePlan best{0, 1, 0.0f};
   bool first = true;
+  int splits = 1;
+  while (may_split && splits < 8 && K >= (int64_t)kMinSplitK * kSplits[splits]) ++splits;
+  int64_t pieces[8];  // stages of one
+  for (int i = 0; i < splits; ++i) pieces[i] = cdiv(stages(K), kSplits[i]);
   for (int c = 0; c < 4; ++c) {
     const TileConfig& t = kConfigs[c];
-    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
-    for (const int s : kSplits) {
-      if (s > 1 && (!may_split || K < (int64_t)kMinSplitK * s)) break;
-      const float u = (float)cdiv(tiles * s, kCus), rounds = (float)cdiv(cdiv(tiles * s, kCus), t.resident);
+    const int64_t tiles = tile_count(M, t.bm) * tile_count(N, t.bn);
+    for (int i = 0; i < splits; ++i) {
+      const int s = kSplits[i];
+      const int64_t wgs = cdiv(tiles * s, kCus);  // a CU
+      const float u = (float)wgs, rounds = (float)by_resident(wgs, t.resident);
       const float stage = rounds * t.lambda > u * t.tau ? rounds * t.lambda : u * t.tau;
-      float us = (float)cdiv(stages(K), s) * stage + 1.5f * u * (float)(t.bn * t.bm) / 65536.0f;
+      float us = (float)pieces[i] * stage + 1.5f * u * (float)(t.bn * t.bm) / 65536.0f;
       if (s > 1) us += 5.0f + 1.6e-6f * (float)s * (float)M * (float)N;
       if (first || us < best.us) {
         first = false;
@@ -301,12 +315,11 @@ TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
   best.split = (int)cdiv(K, split_kps(K, best.split));  // whole stages a piece may need fewer pieces
   return best;
 }
-size_t split_bytes(const TilePlan& p, int64_t M, int64_t N) {
-  return p.split > 1 ? (size_t)p.split * (size_t)M * (size_t)N * sizeof(float) : 0;
-}
+
+namespace {
 
 template <bool BF16, bool ROW>
-void launch_config(const W16TileArgs& a, const TilePlan& p, hipStream_t st) {
+void launch_config(const W16TileArgs& a, const W16TilePlan& p, hipStream_t st) {
   const TileConfig& t = kConfigs[p.config];
   const int tiles_m = (int)cdiv(a.M, t.bm);
   const dim3 grid((unsigned)(tiles_m * cdiv(a.N, t.bn)), (unsigned)p.split);
@@ -321,12 +334,12 @@ void launch_config(const W16TileArgs& a, const TilePlan& p, hipStream_t st) {
 
 }  // namespace
 
-size_t w16_tile_workspace(int64_t M, int64_t N, int64_t K) { return split_bytes(tile_plan(M, N, K, true), M, N); }
+size_t w16_tile_workspace(int64_t M, int64_t N, int64_t K) { return split_bytes(w16_tile_plan(M, N, K), M, N); }
 
 // The weights stream at no more than 4.4 TB/s beside a launch and its prologue.
-float w16_tile_time(int64_t M, int64_t N, int64_t K) {
-  const float us = tile_plan(M, N, K, true).us, stream = 6.0f + (float)N * (float)K / 4.4e6f;
-  return us > stream ? us : stream;
+float w16_tile_time(const W16TilePlan& p, int64_t N, int64_t K) {
+  const float stream = 6.0f + (float)N * (float)K / 4.4e6f;
+  return p.us > stream ? p.us : stream;
 }
 
 bool w16_tile_supported(const W16TileArgs& a) {
@@ -335,10 +348,9 @@ bool w16_tile_supported(const W16TileArgs& a) {
          512 * a.ldx < ((int64_t)1 << 31) && cdiv(a.M, 64) * cdiv(a.N, 128) < ((int64_t)1 << 31);
 }
 
-int w16_tile_launch(const W16TileArgs& a, bool bf16, hipStream_t st, const char* op) {
-  TilePlan p = tile_plan(a.M, a.N, a.K, true);
+int w16_tile_launch(const W16TileArgs& a, W16TilePlan p, bool bf16, hipStream_t st, const char* op) {
   // A caller that brings no workspace gets the best plan without a split.
-  if (p.split > 1 && (a.part == nullptr || a.part_bytes < split_bytes(p, a.M, a.N))) p = tile_plan(a.M, a.N, a.K, false);
+  if (p.split > 1 && (a.part == nullptr || a.part_bytes < split_bytes(p, a.M, a.N))) p = w16_tile_plan(a.M, a.N, a.K, false);
   const bool row = a.bx >= a.K;
   note_plan("w8a16 tile %dx%d split=%d", kConfigs[p.config].bn, kConfigs[p.config].bm, p.split);
   if (bf16) row ? launch_config<true, true>(a, p, st) : launch_config<true, false>(a, p, st);
