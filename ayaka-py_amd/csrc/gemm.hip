@@ -1989,16 +1989,18 @@ float block128_time(int64_t M, int64_t N, int64_t K) {
 // a stage ring for them that a short K does not fill, on two rounds of workgroups past 32768
 // columns (general against medium, M = 17 to 25: block 38144 x 128 5.6 us and 8.9, 27648 x 128
 // 5.1 and 5.9, MXFP8 36828 x 128 5.5 and 9.0, 25140 x 320 7.0 and 8.2, per-row 34064 x 96 7.0
-// and 8.1; M = 64, MXFP8 37324 x 128 7.6 and 10.2). Below 16384 columns both take 4 to 5 us,
-// and past these K the medium tiles are faster. MXFP8 batches of up to 8 rows on large weights
-// whose K the decode kernel refuses stream faster in the general kernel's K split (6400 x
-// 21376, M = 5: 38.4 and 44.2, 18584 x 4736, M = 2: 26.9 and 30.9); in two pieces, from 9 rows
-// on and below 66 MB they mostly do not (29184 x 6784, M = 8: 54.5 and 47.2; 13552 x 4736, M = 2:
-// 23.8 and 16.7).
+// and 8.1; M = 64, MXFP8 37324 x 128 7.6 and 10.2). With per-stage scales that holds up to K =
+// 896: over random batches of 1 to 40 rows the general kernel takes 0.86 of their time (block,
+// K from 513), 0.88 (641) and 0.91 (769), 0.94 to 0.98 (MXFP8), and 1.01 past it. Below 16384
+// columns both take 4 to 5 us, and past these K the medium tiles are faster. MXFP8 batches of
+// up to 8 rows on large weights whose K the decode kernel refuses stream faster in the general
+// kernel's K split (6400 x 21376, M = 5: 38.4 and 44.2, 18584 x 4736, M = 2: 26.9 and 30.9); in
+// two pieces, from 9 rows on and below 66 MB they mostly do not (29184 x 6784, M = 8: 54.5 and
+// 47.2; 13552 x 4736, M = 2: 23.8 and 16.7).
 template <int MODE>
 bool general_wanted(int64_t M, int64_t N, int64_t K) {
   constexpr bool mx = MODE == MODE_MX, scales = mx || MODE == MODE_BLOCK;  // per-stage scale loads
-  if (N > 32768 && (M <= 32 ? K <= 512 : M <= 64 && scales && K <= (mx ? 128 : 384))) return true;
+  if (N > 32768 && (M <= 32 ? K <= (scales ? 896 : 512) : M <= 64 && scales && K <= (mx ? 128 : 384))) return true;
   // (MXFP8 rows of codes that no dword bounds cost the medium tiles two loads a row and stage)
   if (scales && M <= 32 && N > 16384 && K <= (mx && K % 128 ? 448 : 256)) return true;
   return mx && M <= 8 && N * K > 66000000 && K % 256 == 128 && scaled_split(M, N, K, 32, 128) >= 3;

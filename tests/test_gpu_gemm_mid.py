@@ -287,7 +287,12 @@ def test_general_kernel_int8_rows_far_apart(gpu):
 @pytest.mark.parametrize("recipe,m,n,k,expect", [
     ("scaled", 32, 32900, 208, "general 128x32 split=1"),
     ("scaled", 33, 32900, 208, "mid 64x64 ring split=1"),
+    ("scaled", 20, 32900, 640, "mid 64x64 ring split=1"),
     ("block", 17, 32900, 512, "general 128x32 split=1"),     # bf16 weight scales
+    ("block", 1, 32900, 640, "general 128x32 split=1"),
+    ("block16", 32, 32900, 896, "general 128x32 split=1"),
+    ("block16", 32, 32900, 1024, "mid 64x64 ring split=1"),
+    ("mx", 20, 32900, 640, "general 128x32 split=1"),
     ("block", 64, 32900, 384, "general 128x64 split=1"),
     ("block", 20, 16500, 128, "general 128x32 split=1"),
     ("block", 20, 16300, 128, "mid 64x64 ring split=1"),
