@@ -1785,7 +1785,7 @@ int launch_pair_tail(GemmArgs g, int64_t tiles, hipStream_t st, const char* op) 
 
 template <int MODE>
 int launch_big(GemmArgs g, hipStream_t st, const char* op) {
-  static_assert(MODE != MODE_BLOCK, "block scales use the general kernel");
+  static_assert(MODE != MODE_BLOCK, "block scales have kernels of their own");
   g.tiles_m = (int)cdiv(g.M, kBigTile);
   const int64_t tiles = (int64_t)g.tiles_m * cdiv(g.N, kBigTile);
   if (tiles > 0x7FFFFFFF) return fail(AYK_EINVAL, "%s: problem too large", op);
@@ -1868,15 +1868,10 @@ int launch_cfg(GemmArgs g, hipStream_t st, const char* op) {
   g.tiles_m = (int)cdiv(g.M, BM);
   const int64_t tiles = (int64_t)g.tiles_m * cdiv(g.N, kBn);
   if (tiles > 0x7FFFFFFF) return fail(AYK_EINVAL, "%s: problem too large", op);
-  const int64_t split = MODE == MODE_BLOCK ? general_block_split(g.M, g.N, g.K)
-                        : (MODE == MODE_INT8 ? 1 : scaled_split(g.M, g.N, g.K, BM, kBn));
-  g.kps = 0;
-  if (split > 1) {
-    const size_t need = (size_t)split * (size_t)g.M * (size_t)g.N * sizeof(float);
-    if (g.ws == nullptr || g.ws_bytes < need)
-      return fail(AYK_EWORKSPACE, "%s: workspace of %zu bytes required, %zu given", op, need, g.ws_bytes);
-    g.kps = MODE == MODE_BLOCK ? g.K / split : scaled_kps(g.K, split);
-  }
+  int64_t split = MODE == MODE_BLOCK ? general_block_split(g.M, g.N, g.K)
+                  : (MODE == MODE_INT8 ? 1 : scaled_split(g.M, g.N, g.K, BM, kBn));
+  if (g.ws == nullptr || g.ws_bytes < (size_t)split * (size_t)g.M * (size_t)g.N * sizeof(float)) split = 1;
+  g.kps = split == 1 ? 0 : (MODE == MODE_BLOCK ? g.K / split : scaled_kps(g.K, split));
   note_plan("general %dx%d split=%d", kBn, BM, (int)split);
   hipLaunchKernelGGL((fp8_gemm_kernel<MODE, kBn, BM, WN, WM>), dim3((unsigned)tiles, (unsigned)split), dim3(kThreads), 0, st, g);
   if (int rc = check_launch(op)) return rc;
@@ -2013,6 +2008,9 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
   const MidPlan plan = mid_ok ? mid_plan(mid_mode(MODE), g.M, g.N, g.K) : MidPlan{};
   // Whether the medium tiles beat a kernel that is modelled at `us`.
   auto mid_beats = [&](float us) { return mid_ok && mid_time(plan, g.N, g.K) < us; };
+  // A launch that did not bring the workspace its kernel splits K in goes on, in the end to the
+  // medium tiles, which run it without a split.
+  auto settled = [&](int rc) { return rc != AYK_EWORKSPACE || !mid_ok; };
   // The large-tile kernels need K % 64 == 0, fp32 scales (MXFP8: K % 512 == 0 and 16-byte
   // aligned code rows), N % 4 == 0 and 16-byte aligned output rows (its epilogue stores
   // 16-byte chunks).
@@ -2026,12 +2024,16 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
                       (MODE == MODE_MX || (g.sa_dtype == AYK_F32 && g.sb_dtype == AYK_F32 &&
                                            (!g.sb_vec || aligned16(g.sb)))) &&
                       (g.bias == nullptr || (reinterpret_cast<uintptr_t>(g.bias) & 15) == 0);
-  if (big_ok && !mid_beats(medium_limit(pair_time(MODE, g.M, g.N, g.K)))) return launch_big<MODE>(g, st, op);
+  if (big_ok && !mid_beats(medium_limit(pair_time(MODE, g.M, g.N, g.K)))) {
+    if (const int rc = launch_big<MODE>(g, st, op); settled(rc)) return rc;
+  }
   } else {
     // The 256 x 256 block-scaled kernel from half a round of its tiles on.
     if (g.sa_dtype == AYK_F32 && block256_wanted(g.M, g.N, g.K)) {
       const Block256Args b = block256_args(g);
-      if (block256_supported(b) && !mid_beats(medium_limit(block256_time(g.M, g.N, g.K)))) return block256_launch(b, st, op);
+      if (block256_supported(b) && !mid_beats(medium_limit(block256_time(g.M, g.N, g.K)))) {
+        if (const int rc = block256_launch(b, st, op); settled(rc)) return rc;
+      }
     }
     // The block-scaled 128 x 128 kernel: K % 128 == 0, fp32 activation scales, any float
     // weight-scale dtype, and the same output / bias alignment as above.
@@ -2041,7 +2043,9 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
                         g.N % 4 == 0 && g.sa_dtype == AYK_F32 &&
                         (g.ldo * out_bytes) % 16 == 0 && aligned16(g.out) &&
                         (g.bias == nullptr || (reinterpret_cast<uintptr_t>(g.bias) & 15) == 0);
-    if (big_ok && !mid_beats(0.9f * block128_time(g.M, g.N, g.K))) return launch_block_big(g, st, op);
+    if (big_ok && !mid_beats(0.9f * block128_time(g.M, g.N, g.K))) {
+      if (const int rc = launch_block_big(g, st, op); settled(rc)) return rc;
+    }
   }
   // Decode batches (M <= 64) with fp32 or UE8M0 scales: the weight-streaming kernel
   // (gemm_skinny.hip) where its shape and alignment rules hold. Its plans leave some shapes
@@ -2063,7 +2067,9 @@ int launch_gemm(const GemmArgs& g, hipStream_t st, const char* op) {
       const float save = one ? 4.0f : 6.0f;
       if (skinny_fp8_supported(sk)) {
         const float us = skinny_fp8_time(sk);
-        if (!mid_beats(std::min(share * us, us - save))) return skinny_fp8_launch(sk, st, op);
+        if (!mid_beats(std::min(share * us, us - save))) {
+          if (const int rc = skinny_fp8_launch(sk, st, op); settled(rc)) return rc;
+        }
       }
     }
   }

@@ -1484,6 +1484,9 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
                       out, ldo, static_cast<float*>(workspace), workspace_bytes};
   const bool tile_ok = w16_tile_supported(t);
   const W16TilePlan tp = tile_ok ? w16_tile_plan(M, N, K) : W16TilePlan{};
+  // A launch that did not bring the workspace its kernel splits K in goes on, in the end to the
+  // tiled kernel, which runs it without a split.
+  auto settled = [&](int rc) { return rc != AYK_EWORKSPACE || !tile_ok; };
   auto tile_beats = [&](float us) { return tile_ok && w16_tile_time(tp, N, K) < 0.75f * us; };
   if (M >= 2) {
     const StPlan sp = stream_plan(M, N, K, block_size_x);
@@ -1492,8 +1495,9 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
       a.x = g.x; a.ldx = ldx; a.M = M; a.w = g.w; a.ldw = ldw; a.N = N; a.K = K;
       a.scale = scale; a.scale_dtype = scale_dtype; a.srs = scale_row_stride; a.by = block_size_y; a.bx = block_size_x;
       a.out = g.out; a.ldo = ldo; a.part = static_cast<float*>(workspace);
-      return x_dtype == AYK_BF16 ? launch_stream<true>(sp, a, workspace_bytes, st)
-                                 : launch_stream<false>(sp, a, workspace_bytes, st);
+      const int rc = x_dtype == AYK_BF16 ? launch_stream<true>(sp, a, workspace_bytes, st)
+                                         : launch_stream<false>(sp, a, workspace_bytes, st);
+      if (settled(rc)) return rc;
     }
   }
   if (M >= 2) {
@@ -1503,8 +1507,9 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
       a.x = g.x; a.ldx = ldx; a.M = M; a.w = g.w; a.ldw = ldw; a.N = N; a.K = K;
       a.scale = scale; a.scale_dtype = scale_dtype; a.srs = scale_row_stride; a.by = block_size_y; a.bx = block_size_x;
       a.out = g.out; a.ldo = ldo; a.part = static_cast<float*>(workspace);
-      return x_dtype == AYK_BF16 ? launch_rows<true>(rp, a, workspace_bytes, st)
-                                 : launch_rows<false>(rp, a, workspace_bytes, st);
+      const int rc = x_dtype == AYK_BF16 ? launch_rows<true>(rp, a, workspace_bytes, st)
+                                         : launch_rows<false>(rp, a, workspace_bytes, st);
+      if (settled(rc)) return rc;
     }
   }
   if (M >= 2) {
@@ -1520,8 +1525,9 @@ int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
       a.x = g.x; a.ldx = ldx; a.M = M; a.w = g.w; a.ldw = ldw; a.N = N; a.K = K;
       a.scale = scale; a.scale_dtype = scale_dtype; a.srs = scale_row_stride; a.by = block_size_y; a.bx = block_size_x;
       a.out = g.out; a.ldo = ldo; a.part = static_cast<float*>(workspace);
-      return x_dtype == AYK_BF16 ? launch_skinny<true>(p, a, workspace_bytes, st)
-                                 : launch_skinny<false>(p, a, workspace_bytes, st);
+      const int rc = x_dtype == AYK_BF16 ? launch_skinny<true>(p, a, workspace_bytes, st)
+                                         : launch_skinny<false>(p, a, workspace_bytes, st);
+      if (settled(rc)) return rc;
     }
   }
   // Everything else: the tiled kernel, but for scale blocks that split its 64-K stages.

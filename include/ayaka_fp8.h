@@ -125,8 +125,7 @@ int ayk_fp8_scaled_mm(const void* a, int64_t lda, const void* b, int64_t ldb,
  * batch (M <= 64) on a narrow projection splits K across workgroups, as the medium tiles
  * do at any M. Each piece writes its fp32 partial and a fixed-order sum adds the bias and
  * rounds once. The size is the largest any of these needs for the shape. With a smaller
- * workspace or none, the medium tiles run without a split; every other kernel that would
- * split returns AYK_EWORKSPACE. */
+ * workspace or none, the launch takes a slower kernel that needs none. */
 size_t ayk_fp8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /* fp8_rowwise_linear (gemm/fp8_linear.py:168) for 2 to 8 activation rows in one launch:
@@ -242,9 +241,9 @@ size_t ayk_fp8_weight_only_gemv_static_max_bytes(void);
  * x dtype. Each dequantized weight w * scale is rounded to the activation dtype before
  * the product, as the reference does. Launches of any M may use a K split whose partials
  * live in the workspace; ayk_fp8_weight_only_gemm_workspace_bytes(M, N, K, block_size_x)
- * gives its size (0: none needed). With a smaller workspace or none, the tiled kernel
- * (every batch past 32 rows) runs without a split; the decode kernels that would split
- * return AYK_EWORKSPACE. */
+ * gives its size (0: none needed). With a smaller workspace or none, the launch takes a
+ * slower kernel that needs none (AYK_EWORKSPACE where block_size_x is no multiple of 64,
+ * which leaves no such kernel for a decode batch that would split). */
 int ayk_fp8_weight_only_gemm(const void* x, int x_dtype, int64_t ldx, int64_t M,
                              const void* w, int64_t ldw, int64_t N, int64_t K,
                              const void* scale, int scale_dtype, int64_t scale_row_stride,

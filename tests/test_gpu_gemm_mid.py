@@ -316,6 +316,32 @@ def test_decode_kernel_choice(gpu, recipe, m, n, k, expect):
     assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
 
 
+@pytest.mark.parametrize("recipe,m,n,k,lda,expect", [
+    ("scaled", 258, 3608, 10368, None, "pair split=8"),
+    ("scaled", 258, 33136, 1536, None, "pair tail=3"),
+    ("scaled", 64, 1302, 8192, None, "skinny"),
+    ("scaled", 20, 300, 4224, _FAR, "general 128x32 split=4"),
+    ("mx", 258, 3608, 7168, None, "pair split=7"),
+    ("mx", 3, 1807, 12288, None, "skinny"),
+    ("mx", 8, 4100, 16512, None, "general 128x32 split=15"),
+    ("block", 258, 2184, 7296, None, "block256 split=7"),
+    ("block", 258, 520, 16384, None, "block128 split=16"),
+    ("block", 65, 1000, 4096, None, "mid 64x64 ring split=8"),
+    ("block16", 40, 200, 4096, _FAR, "general 128x64 split=4"),
+])
+def test_launch_without_its_workspace(gpu, monkeypatch, recipe, m, n, k, lda, expect):
+    """A launch that would split K and brings no workspace runs without the split."""
+    from ayaka.kernel.hip import _lib
+
+    print(f"no workspace recipe={recipe} m={m} n={n} k={k}", flush=True)
+    _, _, plan = _run(recipe, m, n, k, False, torch.bfloat16, False, gpu, lda=lda)
+    assert plan.startswith(expect) and "split=1" != plan.split()[-1], plan
+    monkeypatch.setattr(_lib, "query", lambda name, *args: 0)
+    out, ref, plan = _run(recipe, m, n, k, True, torch.bfloat16, False, gpu, lda=lda)
+    assert plan.endswith("split=1"), plan
+    assert_linear_close(out, ref, f"{recipe} {m}x{n}x{k}")
+
+
 @pytest.mark.parametrize("recipe,m,n,k,expect", [
     ("scaled", 1794, 5888, 10752, "pair tail=1"),   # 115 us, its model just above the medium tiles'
     ("scaled", 1025, 3072, 1024, "mid 128x128 ring split=1"),

@@ -100,6 +100,17 @@ def test_weight_only_gemm_decode_choice(gpu, m, n, k, bx, plan):
     assert got == plan, got
 
 
+@pytest.mark.parametrize("m,n,k", [(24, 3840, 3200), (16, 512, 8192), (30, 1280, 17664), (40, 2051, 3072), (200, 4099, 14336)])
+def test_weight_only_gemm_without_its_workspace(gpu, monkeypatch, m, n, k):
+    """A launch that would split K and brings no workspace runs without the split."""
+    from ayaka.kernel.hip import _lib
+
+    assert not _check(m, n, k, torch.bfloat16, 1, None, "float32", gpu).endswith("split=1")
+    monkeypatch.setattr(_lib, "query", lambda name, *args: 0)
+    plan = _check(m, n, k, torch.bfloat16, 1, None, "float32", gpu)
+    assert plan.startswith("w8a16 tile") and plan.endswith("split=1"), plan
+
+
 def test_weight_only_gemm_tile_all_codes_and_special_scales(gpu):
     """Every weight code against a one-hot activation: the weight times its row's scale,
     rounded to bf16, NaN codes included; tiny and huge scales."""
